@@ -878,8 +878,12 @@ static hipError_t launch_adj_stage_t(const DevTables& T, const AdjStageArgs& a, 
   int nkch = 1536 / tiles;
   const int maxk = T.nr / 24 > 0 ? T.nr / 24 : 1;
   if (nkch > maxk) nkch = maxk;
-  if (a.chunks > 0) nkch = std::min(a.chunks, T.nr);
   if (nkch < 1) nkch = 1;
+  // below two rounds the split with the shortest chain (adjoint step, us,
+  // before -> after: 6x16^2x24 448 -> 114, 6x32^2x64 699 -> 283, 6x48^2x100
+  // 674 -> 600; 6x64^2x128 keeps its 5 chunks in one round, 1018)
+  if (tiles * nkch < 1024) nkch = small_grid_chunks(tiles, T.nr, 1.5, 2, 1.25);
+  if (a.chunks > 0) nkch = std::min(a.chunks, T.nr);
   const int kchunk = (T.nr + nkch - 1) / nkch;
   hipLaunchKernelGGL((k_adj_stage<TI, TJ, D32>), dim3(tiles * nkch), dim3(TI, TJ), 0, st, T, a.W, a.Yin, a.Yout,
                      a.Wout, a.divs, a.gc2, a.c2f, a.gxa_p, a.gya_p, a.gxa_v, a.gya_v, a.dt, a.alpha, a.beta, a.wscale,
@@ -948,6 +952,7 @@ static hipError_t launch_adj_filter_t(const DevTables& T, const double* in, doub
   int nkch = (2048 + tiles - 1) / tiles;
   const int maxk = T.nr / 48 > 0 ? T.nr / 48 : 1;
   if (nkch > maxk) nkch = maxk;
+  if (tiles * nkch < 1536) nkch = small_grid_chunks(tiles, T.nr, 2.0 * kNstr, 1, 1.5);  // as the forward filter
   if (chunks > 0) nkch = std::min(chunks, T.nr);
   const int kchunk = (T.nr + nkch - 1) / nkch;
   hipLaunchKernelGGL((k_adj_filter<TI, TJ>), dim3(tiles * nkch), dim3(TI, TJ), 0, st, T, in, out, kchunk, nkch);

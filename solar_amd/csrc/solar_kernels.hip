@@ -1230,6 +1230,35 @@ int chunks_for(int tiles, int nr, int target_blocks, int min_chunk) {
   return nk;
 }
 
+// Radial chunks of a march of `tiles` column tiles that does not fill the
+// chip: of every split of the nr planes, the one with the least estimated
+// time, (rounds of blocks) x (planes per block + warm).  The first rule,
+// chunks_for, keeps chunks long, for the bytes that a chunk's window re-reads;
+// a small grid lies in the caches and is bound by the serial chain of its
+// planes instead (about 2 us a plane in the stage kernels, 0.5 in the filter).
+//   warm: planes' worth of work before a block's first output;
+//   resident: blocks a CU holds; one block alone runs `alone` times as long
+//   per plane as its share of a full CU.
+int small_grid_chunks(int tiles, int nr, double warm, int resident, double alone) {
+  constexpr int kCus = 256;
+  int best = 1;
+  double least = 0.0;
+  for (int nk = 1; nk <= nr; ++nk) {
+    const int planes = (nr + nk - 1) / nk;
+    if (nk > 1 && planes == (nr + nk - 2) / (nk - 1)) continue;  // the same chunk length in more blocks
+    const int blocks = tiles * ((nr + planes - 1) / planes);
+    const int slots = kCus * resident, rest = blocks % slots;
+    const double rounds =
+        blocks / slots * resident + (rest == 0 ? 0.0 : rest <= kCus ? alone : (rest + kCus - 1) / kCus);
+    const double t = rounds * (planes + warm);
+    if (nk == 1 || t < least) {
+      least = t;
+      best = nk;
+    }
+  }
+  return best;
+}
+
 // Dynamic LDS of one gather launch; above 64 KiB the kernel is allowed it once.
 template <typename K>
 static hipError_t gather_lds(K kernel, size_t lds) {
@@ -1287,7 +1316,14 @@ static hipError_t launch_stage_t(const DevTables& T, const S* qin, S* qout, S* q
   const int tiles = ((T.n + TI - 1) / TI) * ((T.n + TJ - 1) / TJ) * 6;
   // radial chunks of >= 24 planes, ~12k blocks, at most 8 chunks: 8 chunks measured best at
   // 6x96^2x192 (0.342 ms per stage against 0.375 with 6), 6x128^2x256 and 6x256^2x384
-  const int nkch = ls.stage_chunks > 0 ? ls.stage_chunks : std::min(8, chunks_for(tiles, T.nr, 12288, 24));
+  int nkch = std::min(8, chunks_for(tiles, T.nr, 12288, 24));
+  // below four rounds of 512 blocks the split with the shortest chain
+  // (us per stage, before -> after: 6x16^2x24 56 -> 10, 6x32^2x64 79 -> 23,
+  // 6x64^2x64 85 -> 61, 6x128^2x64 209 -> 202, FP32 state 6x64^2x128 83 -> 67;
+  // at 1728 blocks, 6x96^2x192, the long chunks are still the best: 332 against
+  // 343 at half their length).  The FP32 state runs three blocks a CU, FP64 two.
+  if (tiles * nkch < 1536) nkch = small_grid_chunks(tiles, T.nr, 1.0, sizeof(S) == 4 ? 3 : 2, 1.25);
+  if (ls.stage_chunks > 0) nkch = ls.stage_chunks;
   const int kchunk = (T.nr + nkch - 1) / nkch;
   dim3 grid(tiles * nkch), block(TI, TJ);
   const double al = kAlphaRk4[stage < 0 ? 0 : stage], be = kBetaRk4[stage < 0 ? 0 : stage];
@@ -1400,7 +1436,13 @@ static hipError_t launch_filter_t(const DevTables& T, const S* qin, S* qout, con
   const int tiles = ((T.n + TI - 1) / TI) * ((T.n + TJ - 1) / TJ) * 30;
   // radial chunks of >= 64 planes (each re-reads 10 halo planes), ~4k blocks: a single chunk per
   // column at 6x256^2x384 leaves a long tail (3.45 ms against 2.96 ms with two)
-  const int nkch = ls.filter_chunks > 0 ? ls.filter_chunks : chunks_for(tiles, T.nr, 4096, 64);
+  int nkch = chunks_for(tiles, T.nr, 4096, 64);
+  // a chunk re-reads ten planes, so a small grid is split less far than the
+  // stages (us, before -> after: 6x16^2x96 55 -> 16, 6x32^2x64 48 -> 25,
+  // 6x48^2x100 66 -> 44; from 1620 blocks on, 6x96^2x192, all splits into
+  // 32 to 96 planes measured within 2%)
+  if (tiles * nkch < 1536) nkch = small_grid_chunks(tiles, T.nr, 2.0 * kNstr, 1, 1.5);
+  if (ls.filter_chunks > 0) nkch = ls.filter_chunks;
   const int kchunk = (T.nr + nkch - 1) / nkch;
   dim3 grid(tiles * nkch), block(TI, TJ);
   hipLaunchKernelGGL((k_filter<TI, TJ, S, PART, PAIR>), grid, block, 0, st, T, qin, qout, fgx, fgy, kchunk, nkch);

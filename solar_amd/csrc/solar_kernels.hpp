@@ -52,6 +52,9 @@ struct LaunchShape {
   int adj_stage_chunks = 0, adj_filter_chunks = 0;  // sensitivity kernels
 };
 
+// Radial chunks of a march whose tiles do not fill the chip (solar_kernels.hip).
+int small_grid_chunks(int tiles, int nr, double warm, int resident, double alone);
+
 // State pointers are float* when f32 is set (FP32-state variant), double* otherwise.
 // ecols (optional): the edge_cols copies of q's W/E edge columns; the
 // column strips are then read from there.
