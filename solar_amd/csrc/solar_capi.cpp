@@ -296,6 +296,8 @@ int solar::upload_tables(const Tables& t, DevTables* d, std::vector<void*>* allo
   for (int q = 0; q < 7; ++q)
     if (d->fcx[q] != d->fcy[q]) return fail(SOLAR_ERR_ARG, "xi and eta stencil coefficients differ");
   if (d->fcx[3] != 0.0) return fail(SOLAR_ERR_ARG, "the angular stencil's centre tap is not zero");
+  for (int q = 0; q < 3; ++q)  // and holds three of its taps
+    if (d->fcx[q] != -d->fcx[6 - q]) return fail(SOLAR_ERR_ARG, "the angular stencil is not antisymmetric");
   // the filter kernel computes each radial product once for taps q and 10 - q
   for (int q = 0; q < 11; ++q)
     if (d->filtr[q] != d->filtr[10 - q]) return fail(SOLAR_ERR_ARG, "radial filter taps are not symmetric");

@@ -279,370 +279,329 @@ void k_gather(DevTables T, const S* __restrict__ q,
                           gxv, gyv, field_stride_out, sline, qwr, betar);
 }
 
-// Values one thread loads for one radial plane of the stage kernel: its own
-// point, the halo cells it fills, and the plane entering the radial window.
-// State values stay in the storage type S until used (FP32 storage halves
-// the registers of the prefetched plane); halo cells may come from the FP64
-// ghost strips and are held as double.
+// Accesses that name global memory with a wave-uniform base and a 32-bit lane
+// offset: the address costs no vector instruction.  lane_offset hides that an
+// offset does not change in a loop: widened to 64 bits outside the loop, it
+// would cost an add at every access.
+__device__ __forceinline__ unsigned lane_offset(unsigned v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+using GlobalBytes = const __attribute__((address_space(1))) char*;
+template <typename V>
+__device__ __forceinline__ V load_at(GlobalBytes base, unsigned off) {
+  return *(const __attribute__((address_space(1))) V*)(base + off);
+}
+template <typename V>
+__device__ __forceinline__ V load_at_nt(GlobalBytes base, unsigned off) {
+  return __builtin_nontemporal_load((const __attribute__((address_space(1))) V*)(base + off));
+}
+template <typename V>
+__device__ __forceinline__ void store_at_nt(GlobalBytes base, unsigned off, V v) {
+  __builtin_nontemporal_store(v, (__attribute__((address_space(1))) V*)const_cast<__attribute__((address_space(1))) char*>(base + off));
+}
+template <typename V>
+__device__ __forceinline__ void store_at(GlobalBytes base, unsigned off, V v) {
+  *(__attribute__((address_space(1))) V*)const_cast<__attribute__((address_space(1))) char*>(base + off) = v;
+}
+
+// Arguments of one stage launch (single grid; an ensemble launch takes the
+// tables, buffers and dt from the members M).
 template <typename S>
-struct StagePlane {
-  S vx, ve, q1;                // v_xi, v_eta, rho' at (i,j,k)
-  S w[5];                      // qw at (i,j,k)
-  double hpx, hvx;             // i-halo cell (p', v_xi)
-  double hpy0, hve0, hpy1, hve1;  // low / high j-halo cells (p', v_eta)
-  // FP32 state: halo cells inside the panel, kept as loaded and widened when
-  // they go to LDS (a conversion at the load would wait on every load in
-  // flight); the double members then hold the ghost-strip cells only
-  S fpx, fvx, fpy0, fve0, fpy1, fve1;
-  S pn, rn;                    // p', v_r of the plane entering the window
-  double ogp, ogv;             // PART: ghosts of an outside thread's own cell (p' and v_xi or v_eta)
-  double c2;                   // optional 3-D c^2 at (i,j,k)
-  double tdc2, tdiv;           // tangent-linear inputs at (i,j,k)
-  // RECON: qw at the halo cells and at the plane entering the window
-  S rpx, rvx, rpy0, rve0, rpy1, rve1, wpn, wrn;
+struct StageArgs {
+  DevTables T;
+  const S* qin;
+  S *qout, *qw, *qwo;  // qwo: kStageRecon's qw output
+  const double *gxp, *gyp, *gxv, *gyv;
+  double alpha, beta, beta_r, dt;
+  int kchunk, nkch, rhs_mode;
+  int tile_w, whole;  // PART only; whole: rows and tiles are of whole 64-byte segments
+  const double* c2f;
+  double* divout;
+  int div32;
+  const double *tl_dc2, *tl_div;
+  S* ecols;
+  const EnsMember* M;
+  const int4* items;
+  int nitems, cur;
 };
 
-// One RK stage (or one RHS evaluation when rhs_mode is set), one pass over
-// HBM.  A block owns a TI x TJ column tile of one panel and marches through a
-// chunk of radial planes; p' and v_r sit in 7-plane register windows for the
-// radial stencils, the i/j neighbours of plane k come from a double-buffered
-// LDS tile, and plane k+1 is loaded into registers while plane k is computed.
+// Flags of a stage instantiation beyond kStoreNoQ and kStageRecon.
+constexpr int kStageRhs = 4;  // evaluates the RHS alone (rhs_mode holds its flags), KIND 0
+constexpr int kStageAux = 8;  // c2f or divout is given
+
+// Reciprocal-based quotients (div_group) in the FP32-state stages only.
+template <typename S>
+constexpr bool kStageRcp = sizeof(S) == 4;
+
+// Occupancy floor of the stage kernel in waves per SIMD.  Every variant takes
+// 111 to 145 registers and none spills at three; floors of two and four
+// measured within 1% of three in every case but one (four, where the divergences
+// are kept, makes the rebuilding stage spill: gradient 218 -> 229 ms).
+constexpr int kStageWaves = 3;
+
+// One RK stage (or one RHS evaluation, kStageRhs), one pass over HBM.  A
+// block owns a TI x TJ column tile of one panel and marches through a chunk
+// of radial planes; p' and v_r sit in 7-plane register windows for the radial
+// stencils, and the i/j neighbours of plane k come from a double-buffered LDS
+// tile, one barrier per plane.
 //   KIND 0: first stage (qw taken as 0, written), 1: middle stage (qw read and
 //   written), 2: last stage (qw read, not written back).
-//   XF (FP64 storage, single grid): the stage schedule that stores q after
-//   stages 2, 4 and 5 only.  kStoreNoQ: the stage stores qw (in place) and
-//   the edge columns of q, but not q itself.  kStageRecon (KIND 1): the stage
-//   input is qin + beta_r * qw_a, rebuilt wherever it is read (own point,
-//   halo cells, radial window) with the expression the previous stage
-//   rounded when it computed it, so the same bits; q goes to qout and qw to
-//   qwo_a, a buffer other than qw_a (other blocks still read qw_a's halo
-//   cells).
-// Occupancy floor of the stage kernel (waves per SIMD); 0 leaves it to the
-// compiler.  2 keeps every variant within 256 registers: left alone, the
-// ensemble and tangent-linear middle stages take 254-255 VGPRs plus 2 AGPRs
-// and drop to one wave per SIMD (measured: ensemble step 44.3 -> 42.4 ms,
-// the single-grid stages unchanged).  The single-grid FP32-state variants
-// get 3 (168 registers): the middle stage then spills 20 bytes per lane, and
-// still runs faster with the third wave (measured at 6x128^2x256: 0.537 ->
-// 0.501 ms per stage, step 7.57e9 -> 7.92e9 grid-point steps/s).
-#ifndef SOLAR_STAGE_WAVES
-#define SOLAR_STAGE_WAVES 2
-#endif
-#ifndef SOLAR_STAGE_WAVES_F32
-#define SOLAR_STAGE_WAVES_F32 3
-#endif
-#if SOLAR_STAGE_WAVES > 0
-#define SOLAR_STAGE_ATTR \
-  __attribute__((amdgpu_waves_per_eu(sizeof(S) == 4 && MODE == 0 ? SOLAR_STAGE_WAVES_F32 : SOLAR_STAGE_WAVES)))
-#else
-#define SOLAR_STAGE_ATTR
-#endif
-
-//   ENS: ensemble launch.  The block walks a list of work items (member,
-//   tile, panel, plane range) with a grid-sized stride; tables, buffers and
-//   dt come from the member (the state ping-pongs between M.q[cur] and
-//   M.q[1-cur]); the single-grid arguments are unused.
-//   MODE 2: tangent-linear stage (tl_dc2, tl_div used).
-//   ecols_a (single grid, not null; in an ensemble the member's ecols): the
-//   stage also stores its output at the edge columns i = 1..3 and n-4..n-2
-//   in the edge_cols layout, for the next gather -- p', v_xi, v_eta after
-//   stages 1-4 (the vector gather), all five fields after the last stage
-//   (the filter gather).
-//   PART: the tiles need not divide n.  The last tile of a row or column
-//   then has threads past the panel edge ("outside" threads): they store
-//   nothing, and those within three points of the edge bring the ghost values
-//   of their own cell (E ghosts of p' and v_xi, N ghosts of p' and v_eta)
-//   into the LDS tile, where the in-panel threads' stencils read them.  Every
-//   other cell an outside thread would load reads a fixed in-bounds address.
-template <int TI, int TJ, int KIND, typename S, int MODE = 0, bool PART = false, int XF = 0>
-__global__ __launch_bounds__(TI* TJ) SOLAR_STAGE_ATTR void k_stage(DevTables Targ, const S* __restrict__ qin_a,
-                                                   S* __restrict__ qout_a, S* __restrict__ qw_a,
-                                                   const double* __restrict__ gxp_a, const double* __restrict__ gyp_a,
-                                                   const double* __restrict__ gxv_a, const double* __restrict__ gyv_a,
-                                                   double alpha, double beta, double dt_a, int kchunk, int nkch,
-                                                   int rhs_mode, const double* __restrict__ c2f,
-                                                   double* __restrict__ divout, int div32,
-                                                   const double* __restrict__ tl_dc2, const double* __restrict__ tl_div,
-                                                   S* __restrict__ ecols_a, const EnsMember* __restrict__ M,
-                                                   const int4* __restrict__ items, int nitems, int cur,
-                                                   S* __restrict__ qwo_a, double beta_r) {
-  constexpr bool NOQ = (XF & kStoreNoQ) != 0, RECON = (XF & kStageRecon) != 0;
-  static_assert(XF == 0 || (MODE == 0 && sizeof(S) == 8), "the stage schedule variants are FP64, single grid");
+//   FL: kStoreNoQ (FP64, single grid): the stage stores qw (in place) and the
+//   edge columns of q, but not q itself.  kStageRecon (KIND 1): the stage
+//   input is qin + beta_r * qw, rebuilt wherever it is read (own point, halo
+//   cells, radial window) with the expression the previous stage rounded when
+//   it computed it, so the same bits; q goes to qout and qw to qwo, a buffer
+//   other than qw (other blocks still read qw's halo cells).  kStageRhs,
+//   kStageAux: above.
+//   MODE 1: ensemble launch.  The block walks a list of work items (member,
+//   tile, panel, plane range) with a grid-sized stride; the state ping-pongs
+//   between M.q[cur] and M.q[1-cur].  MODE 2: tangent-linear stage (tl_dc2,
+//   tl_div used).
+//   ecols (optional; in an ensemble the member's): the stage also stores its
+//   output at the edge columns i = 1..3 and n-4..n-2 in the edge_cols layout,
+//   for the next gather -- p', v_xi, v_eta after stages 1-4 (the vector
+//   gather), all five fields after the last stage (the filter gather).
+//   PART: the tiles are tile_w <= TI wide, any width, and need not divide n;
+//   the block is one-dimensional.  In the last tile of a row or column the E
+//   (N) halo cells begin at the panel edge, inside the tile; threads without a
+//   point of their own load through an in-panel point and write nothing.
+//
+// What bounds it.  At 6x256^2x384 a march of as many streams, with no
+// arithmetic, in the same tiles reaches 4.8 to 5.0 TB/s on this card (one shot
+// over the same streams: 5.5); the five FP64 stages move their 640 bytes a
+// point at 4.8.  On small grids it is the instructions issued per point and
+// plane.  So
+//   - every access is a wave-uniform base plus a 32-bit lane offset;
+//   - a halo cell is loaded by one thread (y halos by the first waves, x
+//     halos by the next, so which of v_xi and v_eta a wave needs is uniform);
+//     ghost-strip values load under a wave-uniform branch that only waves at
+//     a panel edge take;
+//   - a plane's loads come in two groups.  What the plane's start needs (halo
+//     cells, v_xi, v_eta, the plane entering the radial windows) is consumed
+//     there, and the next plane's values load into the freed registers before
+//     the barrier.  What the update at its end needs (rho', qw) loads at the
+//     end of the plane before.  Either group is in flight for a whole plane,
+//     no register holds a value twice, and none is copied between planes.
+// Against six halo loads a thread, a second copy of the plane's registers and
+// results held over to the next plane: vector instructions per plane 390 ->
+// 298 (first stage), 475 -> 348 (rebuilding), 425 -> 339 (FP32 state);
+// registers 234 -> 131 (rebuilding), so three waves per SIMD where there were
+// two; us per launch in 32x8 tiles, 6x128^2x256: first 558 -> 462, rebuilding
+// 978 -> 902; 6x256^2x384 FP32 state, middle 2866 -> 2661, last 2494 -> 2002.
+template <int TI, int TJ, int KIND, typename S, int MODE = 0, bool PART = false, int FL = 0>
+__global__ __launch_bounds__(TI* TJ) __attribute__((amdgpu_waves_per_eu(kStageWaves)))
+void k_stage(StageArgs<S> A) {
+  constexpr bool NOQ = (FL & kStoreNoQ) != 0, RECON = (FL & kStageRecon) != 0;
+  constexpr bool RHS = (FL & kStageRhs) != 0, AUX = (FL & (kStageRhs | kStageAux)) != 0;
+  constexpr bool ENS = MODE == 1, TL = MODE == 2, WIDE = sizeof(S) == 8;
+  static_assert(!(NOQ || RECON) || (MODE == 0 && WIDE), "the stored-q schedule variants are FP64, single grid");
   static_assert(!RECON || (KIND == 1 && !NOQ), "a rebuilt input is a middle stage's");
   static_assert(!NOQ || KIND != 2, "the last stage stores q");
+  static_assert(!RHS || (KIND == 0 && MODE == 0 && !NOQ), "an RHS evaluation is of kind 0");
+  // halo cells: 6 rows of TI (y), then TJ rows of 6 (x) from a wave boundary on
+  constexpr int NT = TI * TJ, NHC = PART ? 1 : ((6 * TI + 63) / 64 * 64 + 6 * TJ + NT - 1) / NT;
   __shared__ double sp[2][TJ + 6][TI + 6];
   __shared__ double svx[2][TJ][TI + 6];
-  __shared__ double sve[2][TJ + 6][TI];
+  __shared__ double sve[2][TJ + 6][TI + 6];
 
-  constexpr bool ENS = MODE == 1, TL = MODE == 2;
-  const int n_items = ENS ? nitems : 1;
+  const int W = PART ? A.tile_w : TI, HY = (6 * W + 63) / 64 * 64;
+  const int tid = PART ? threadIdx.x : threadIdx.y * TI + threadIdx.x;
+  const int tx = PART ? tid % W : threadIdx.x, ty = PART ? tid / W : threadIdx.y;
+  const int wave0 = __builtin_amdgcn_readfirstlane(tid & ~63);  // this wave's first thread
+
+  const int n_items = ENS ? A.nitems : 1;
   for (int item = ENS ? (int)blockIdx.x : 0; item < n_items; item += ENS ? (int)gridDim.x : 1) {
   int bi, bj, P, k0, k1, mem = 0;
   if constexpr (ENS) {
-    const int4 w = items[item];
-    mem = w.x;
-    bi = w.y & 0xffff;
-    bj = w.y >> 16;
-    P = w.z & 0xff;
-    k0 = w.z >> 8;
-    k1 = w.w;
+    const auto w = (const __attribute__((address_space(4))) int*)(A.items + item);
+    mem = w[0];
+    bi = w[1] & 0xffff;
+    bj = w[1] >> 16;
+    P = w[2] & 0xff;
+    k0 = w[2] >> 8;
+    k1 = w[3];
   } else {
-    const int nti = (Targ.n + TI - 1) / TI, ntj = (Targ.n + TJ - 1) / TJ;
-    const int nb = nti * ntj * 6 * nkch;
-    int b = xcd_remap(blockIdx.x, nb);
+    const int nti = (A.T.n + W - 1) / W, ntj = (A.T.n + TJ - 1) / TJ;
+    int b = xcd_remap(blockIdx.x, nti * ntj * 6 * A.nkch);
     bi = b % nti;
     b /= nti;
     bj = b % ntj;
     b /= ntj;
     P = b % 6;
-    const int ch = b / 6;
-    k0 = ch * kchunk;
-    k1 = min(k0 + kchunk, Targ.nr);
-    if (k0 >= Targ.nr) return;
+    k0 = b / 6 * A.kchunk;
+    k1 = min(k0 + A.kchunk, A.T.nr);
+    if (k0 >= A.T.nr) return;
   }
-  const DevTables& T = ENS ? M[mem].T : Targ;
-  const auto qin = to_global(ENS ? reinterpret_cast<const S*>(M[mem].q[cur]) : qin_a);
-  const auto qout = to_global(ENS ? reinterpret_cast<S*>(M[mem].q[1 - cur]) : qout_a);
-  const auto qw = to_global(ENS ? reinterpret_cast<S*>(M[mem].qw) : qw_a);
-  const auto gxp = to_global(ENS ? M[mem].gxp : gxp_a);
-  const auto gyp = to_global(ENS ? M[mem].gyp : gyp_a);
-  const auto gxv = to_global(ENS ? M[mem].gxv : gxv_a);
-  const auto gyv = to_global(ENS ? M[mem].gyv : gyv_a);
-  const double dt = ENS ? M[mem].dt : dt_a;
-  const int n = T.n, nr = T.nr;
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  const int i0 = bi * TI, j0 = bj * TJ;
-  const int i = i0 + tx, j = j0 + ty;
-  // own point inside the panel (always, unless PART); outside threads load
-  // through the nearest in-panel point and store nothing
-  const bool own_in = !PART || (i < n && j < n);
+  // the member's record through the constant address space: scalar loads
+  const auto& E = ((const __attribute__((address_space(4))) EnsMember*)A.M)[mem];
+  const int n = ENS ? E.T.n : A.T.n, nr = ENS ? E.T.nr : A.T.nr;
+  const double dt = ENS ? E.dt : A.dt;
+  const CRadialRows rows = const_rows(ENS ? E.T.rad : A.T.rad);
+  // antisymmetric taps (checked when the tables are uploaded)
+  const double c4 = ENS ? E.T.fcx[4] : A.T.fcx[4], c5 = ENS ? E.T.fcx[5] : A.T.fcx[5],
+               c6 = ENS ? E.T.fcx[6] : A.T.fcx[6];
+  const int i0 = bi * W, j0 = bj * TJ, i = i0 + tx, j = j0 + ty;
+  const int wi = PART ? min(W, n - i0) : TI, wj = PART ? min(TJ, n - j0) : TJ;  // the tile inside the panel
+  const bool own_in = !PART || (tx < wi && ty < wj);
   const int ic = PART ? min(i, n - 1) : i, jc = PART ? min(j, n - 1) : j;
-
   const size_t plane = (size_t)n * n, nf = plane * nr;
-  const size_t ij = (size_t)jc * n + ic;
-  const auto f0 = qin + (size_t)(P * 5) * nf;  // rho'
-  const auto f1 = f0 + nf;                     // v_xi
-  const auto f2 = f1 + nf;                     // v_eta
-  const auto f3 = f2 + nf;                     // v_r
-  const auto f4 = f3 + nf;                     // p'
-  const auto o0 = qout + (size_t)(P * 5) * nf;
-  const auto w0 = qw + (size_t)(P * 5) * nf;
-  // where qw is stored: in place, or (RECON) in the other accumulator
-  const auto wo0 = RECON ? to_global(qwo_a) + (size_t)(P * 5) * nf : w0;
+  const unsigned cell = (unsigned)(jc * n + ic), off = cell * (unsigned)sizeof(S);
+  // byte bases of this panel's field 0 and byte strides of fields and planes
+  const size_t ps = plane * sizeof(S), fs = nf * sizeof(S), pbase = (size_t)P * 5 * nf;
+  const auto bytes = [](const void* p) { return (GlobalBytes)p; };
+  const GlobalBytes qb = bytes((ENS ? reinterpret_cast<const S*>(E.q[A.cur]) : A.qin) + pbase);
+  const GlobalBytes wb = bytes((ENS ? reinterpret_cast<const S*>(E.qw) : A.qw) + pbase);
+  const GlobalBytes ob = bytes((ENS ? reinterpret_cast<const S*>(E.q[1 - A.cur]) : A.qout) + pbase);
+  const GlobalBytes wob = RECON ? bytes(A.qwo + pbase) : wb;
   // edge-column copy: layer l = i (W) or n-1-i (E); the others store none
   const int ecl = i <= 3 ? i : n - 1 - i;
-  S* const ecols = ENS ? reinterpret_cast<S*>(M[mem].ecols) : ecols_a;
-  const bool ec_on = !rhs_mode && ecols != nullptr && ecl >= 1 && ecl <= 3 && own_in;
-  const auto ecw = to_global(ecols);  // stored through only when ec_on
-  const size_t ec_base = ec_on ? (size_t)(P * 2 + (i > 3)) * nr * edge_cols_plane(n) + (size_t)j * 3 + (ecl - 1) : 0;
+  const S* const ecols = RHS ? nullptr : ENS ? reinterpret_cast<const S*>(E.ecols) : A.ecols;
+  const bool ec_on = !RHS && ecols != nullptr && ecl >= 1 && ecl <= 3 && own_in;
+  const GlobalBytes ecb = bytes(ecols + (size_t)(P * 2) * nr * edge_cols_plane(n));
+  const unsigned ec_off =
+      (unsigned)(((i > 3 ? (size_t)nr * edge_cols_plane(n) : 0) + (size_t)j * 3 + (ecl - 1)) * sizeof(S));
 
-  // Halo cells this thread fills: source pointer and plane stride, from the
-  // field inside the panel or from the gathered ghost strips beyond its edge.
-  const size_t gx_side = (size_t)nr * n * 3, gy_side = (size_t)nr * 3 * n;
-  const auto gxpW = gxp + (size_t)(P * 2) * gx_side;
-  const auto gxvW = gxv + (size_t)(P * 2) * gx_side;
-  const auto gypS = gyp + (size_t)(P * 2) * gy_side;
-  const auto gyvS = gyv + (size_t)(P * 2) * gy_side;
-  const bool hx = tx < 3 || tx >= TI - 3, hy0 = ty < 3, hy1 = ty >= TJ - 3;
-  // Each halo slot: a 32-bit offset inside one plane of its source and
-  // whether the source is a ghost strip (plane stride 3n) or the field
-  // (plane stride n*n); the p' and velocity halos share the offset.
-  int hx_off = 0, hy0_off = 0, hy1_off = 0;
-  bool hx_g = false, hy0_g = false, hy1_g = false;
-  int hx_col = 0;
-  // PART: a slot whose cell lies beyond the panel and beyond its three ghost
-  // layers, or in a row or column outside the panel, keeps the fixed address
-  // (no stencil of an in-panel point reads it).
-  if (hx) {
-    const bool lo = tx < 3;
-    const int ii = lo ? i0 - 3 + tx : i + 3;
-    hx_col = lo ? tx : tx + 6;
-    if (PART && (j >= n || ii >= n + 3)) {
-    } else if (ii >= 0 && ii < n) {
-      hx_off = j * n + ii;
+  // This thread's halo cells: the offset in a field plane (0, any valid cell,
+  // for a ghost or an unused slot), the offset in a plane of the ghost strips,
+  // and the LDS cells.
+  const size_t gx_side = (size_t)nr * n * 3, gs = (size_t)3 * n * sizeof(double);
+  const GlobalBytes gxp = bytes((ENS ? E.gxp : A.gxp) + (size_t)(P * 2) * gx_side);
+  const GlobalBytes gyp = bytes((ENS ? E.gyp : A.gyp) + (size_t)(P * 2) * gx_side);
+  const GlobalBytes gxv = bytes((ENS ? E.gxv : A.gxv) + (size_t)(P * 2) * gx_side);
+  const GlobalBytes gyv = bytes((ENS ? E.gyv : A.gyv) + (size_t)(P * 2) * gx_side);
+  unsigned hoff[NHC], goff[NHC];
+  int hrow[NHC], hcol[NHC];
+  bool hin[NHC], hg[NHC], wave_g[NHC], xh[NHC];
+#pragma unroll
+  for (int c = 0; c < NHC; ++c) {
+    const int h = tid + c * NT;
+    xh[c] = wave0 + c * NT >= HY;  // wave-uniform
+    int hi, hj;
+    if (xh[c]) {
+      const int h6 = (h - HY) % 6;
+      hrow[c] = (h - HY) / 6 + 3;
+      hcol[c] = h6 < 3 ? h6 : wi + h6;
+      hin[c] = hrow[c] < wj + 3;
     } else {
-      hx_g = true;
-      hx_off = lo ? j * 3 + (-ii - 1) : (int)gx_side + j * 3 + (ii - n);
+      const int r = h / W;
+      hrow[c] = r < 3 ? r : wj + r;
+      hcol[c] = h % W + 3;
+      hin[c] = r < 6 && hcol[c] < wi + 3;
     }
-  }
-  if (hy0) {
-    const int jj = j0 - 3 + ty;
-    if (PART && i >= n) {
-    } else if (jj >= 0) {
-      hy0_off = jj * n + i;
+    hi = i0 - 3 + hcol[c];
+    hj = j0 - 3 + hrow[c];
+    hoff[c] = goff[c] = 0;
+    hg[c] = false;
+    if (!hin[c]) {
+      hrow[c] = hcol[c] = 0;
+    } else if (hi < 0 || hi >= n) {
+      hg[c] = true;
+      goff[c] = (unsigned)((hi < 0 ? hj * 3 - hi - 1 : gx_side + hj * 3 + hi - n) * sizeof(double));
+    } else if (hj < 0 || hj >= n) {
+      hg[c] = true;
+      goff[c] = (unsigned)((hj < 0 ? (-hj - 1) * n + hi : gx_side + (hj - n) * n + hi) * sizeof(double));
     } else {
-      hy0_g = true;
-      hy0_off = (-jj - 1) * n + i;
+      hoff[c] = (unsigned)((hj * n + hi) * sizeof(S));
     }
-  }
-  if (hy1) {
-    const int jj = j + 3;
-    if (PART && (i >= n || jj >= n + 3)) {
-    } else if (jj < n) {
-      hy1_off = jj * n + i;
-    } else {
-      hy1_g = true;
-      hy1_off = (int)gy_side + (jj - n) * n + i;
-    }
-  }
-  // PART: an outside thread within three points of the E edge (in a panel
-  // row) or of the N edge (in a panel column) owns an LDS cell that holds
-  // ghosts: E ghosts of p' and v_xi, or N ghosts of p' and v_eta.
-  int og = 0, og_off = 0;
-  auto ogp_src = gxpW, ogv_src = gxvW;  // without ghosts: a fixed in-bounds address
-  if (PART) {
-    if (j < n && i >= n && i < n + 3) {
-      og = 1;
-      ogp_src = gxpW + gx_side;
-      ogv_src = gxvW + gx_side;
-      og_off = j * 3 + (i - n);
-    } else if (i < n && j >= n && j < n + 3) {
-      og = 2;
-      ogp_src = gypS + gy_side;
-      ogv_src = gyvS + gy_side;
-      og_off = (j - n) * n + i;
-    }
+    wave_g[c] = __ballot(hg[c]) != 0;
   }
 
-  constexpr bool kWide = sizeof(S) == sizeof(double);
-  // The loads of a plane carry no branches (every halo slot reads a valid
-  // address: offset 0 of the plane when the thread has no such halo cell), so
-  // the waits before their use count exactly the stores issued after them.
-  // FP32 state: field halo cells load as FP32, ghost-strip cells as FP64 in
-  // waves that hold one (a wave-uniform branch).
-  const bool wg_x = kWide || __ballot(hx_g) != 0, wg_y0 = kWide || __ballot(hy0_g) != 0,
-             wg_y1 = kWide || __ballot(hy1_g) != 0;
-  const auto c2base = to_global(c2f ? c2f : T.ci);  // without c2f: a fixed in-bounds address
-  auto load_plane = [&](int k, StagePlane<S>& L) {
-    const size_t kp = (size_t)k * plane + ij;
-    L.vx = f1[kp];
-    L.ve = f2[kp];
-    L.q1 = __builtin_nontemporal_load(f0 + kp);
+  // what plane k's start needs, loaded a plane ahead; in the storage type
+  // (a conversion at the load would wait for it there)
+  S vx_n, ve_n, pn, rn, hp[NHC], hv[NHC];
+  double gp[NHC] = {}, gv[NHC] = {};
+  S w1_n = 0, w2_n = 0, wpn = 0, wrn = 0, rp[NHC] = {}, rv[NHC] = {};  // RECON: qw at the same points
+  auto load_start = [&](int k) {
+    const GlobalBytes q = qb + (size_t)k * ps, w = wb + (size_t)k * ps;
+    const size_t kn = (size_t)min(k + 3, nr - 1) * ps;  // the plane entering the windows before plane k
+#pragma unroll
+    for (int c = 0; c < NHC; ++c)
+      if (wave_g[c]) {
+        const size_t kg = (size_t)k * gs;
+        const unsigned g = lane_offset(goff[c]);
+        gp[c] = load_at<double>((xh[c] ? gxp : gyp) + kg, g);
+        gv[c] = load_at<double>((xh[c] ? gxv : gyv) + kg, g);
+      }
+    const unsigned o = lane_offset(off);
+    pn = load_at<S>(qb + kn + 4 * fs, o);
+    rn = load_at<S>(qb + kn + 3 * fs, o);
+    if constexpr (RECON) {
+      wpn = load_at<S>(wb + kn + 4 * fs, o);
+      wrn = load_at<S>(wb + kn + 3 * fs, o);
+    }
+    vx_n = load_at<S>(q + fs, o);
+    ve_n = load_at<S>(q + 2 * fs, o);
+    if constexpr (RECON) {
+      w1_n = load_at<S>(w + fs, o);
+      w2_n = load_at<S>(w + 2 * fs, o);
+    }
+#pragma unroll
+    for (int c = 0; c < NHC; ++c) {
+      const size_t fv = xh[c] ? fs : 2 * fs;
+      const unsigned h = lane_offset(hoff[c]);
+      hp[c] = load_at<S>(q + 4 * fs, h);
+      hv[c] = load_at<S>(q + fv, h);
+      if constexpr (RECON) {
+        rp[c] = load_at<S>(w + 4 * fs, h);
+        rv[c] = load_at<S>(w + fv, h);
+      }
+    }
+  };
+  // what its update needs
+  S q1_n, w_n[5] = {};
+  double c2_n = 0.0, tdc2 = 0.0, tdiv = 0.0;
+  auto load_update = [&](int k) {
+    const unsigned o = lane_offset(off);
+    q1_n = load_at_nt<S>(qb + (size_t)k * ps, o);
 #pragma unroll
     for (int f = 0; f < 5; ++f)
-      L.w[f] = (KIND == 0) ? S(0) : __builtin_nontemporal_load(w0 + f * nf + kp);
-    const size_t kf = (size_t)k * plane, kg = (size_t)k * 3 * n;
-    if constexpr (kWide) {
-      L.hpx = hx_g ? gxpW[kg + hx_off] : f4[kf + hx_off];
-      L.hvx = hx_g ? gxvW[kg + hx_off] : f1[kf + hx_off];
-      L.hpy0 = hy0_g ? gypS[kg + hy0_off] : f4[kf + hy0_off];
-      L.hve0 = hy0_g ? gyvS[kg + hy0_off] : f2[kf + hy0_off];
-      L.hpy1 = hy1_g ? gypS[kg + hy1_off] : f4[kf + hy1_off];
-      L.hve1 = hy1_g ? gyvS[kg + hy1_off] : f2[kf + hy1_off];
-      if constexpr (RECON) {  // qw of the field cells (a ghost cell reads offset 0 and does not use it)
-        const int fx = hx_g ? 0 : hx_off, fy0 = hy0_g ? 0 : hy0_off, fy1 = hy1_g ? 0 : hy1_off;
-        L.rpx = w0[4 * nf + kf + fx];
-        L.rvx = w0[nf + kf + fx];
-        L.rpy0 = w0[4 * nf + kf + fy0];
-        L.rve0 = w0[2 * nf + kf + fy0];
-        L.rpy1 = w0[4 * nf + kf + fy1];
-        L.rve1 = w0[2 * nf + kf + fy1];
-      }
-    } else {
-      const int fx = hx_g ? 0 : hx_off, fy0 = hy0_g ? 0 : hy0_off, fy1 = hy1_g ? 0 : hy1_off;
-      L.fpx = f4[kf + fx];
-      L.fvx = f1[kf + fx];
-      L.fpy0 = f4[kf + fy0];
-      L.fve0 = f2[kf + fy0];
-      L.fpy1 = f4[kf + fy1];
-      L.fve1 = f2[kf + fy1];
-      if (wg_x) {
-        const int gx = hx_g ? hx_off : 0;
-        L.hpx = gxpW[kg + gx];
-        L.hvx = gxvW[kg + gx];
-      }
-      if (wg_y0) {
-        const int gy = hy0_g ? hy0_off : 0;
-        L.hpy0 = gypS[kg + gy];
-        L.hve0 = gyvS[kg + gy];
-      }
-      if (wg_y1) {
-        const int gy = hy1_g ? hy1_off : 0;
-        L.hpy1 = gypS[kg + gy];
-        L.hve1 = gyvS[kg + gy];
-      }
+      if (KIND != 0 && !(RECON && (f == 1 || f == 2))) w_n[f] = load_at_nt<S>(wb + (size_t)k * ps + f * fs, o);
+    const size_t dk = ((size_t)P * nf + (size_t)k * plane) * sizeof(double);
+    const unsigned o8 = lane_offset(cell * 8u);
+    if (AUX || TL) {
+      if (A.c2f) c2_n = load_at<double>(bytes(A.c2f) + dk, o8);
     }
-    if constexpr (PART) {
-      L.ogp = ogp_src[kg + og_off];
-      L.ogv = ogv_src[kg + og_off];
-    }
-    // plane entering the radial window when the window slides before k
-    const int kn = min(k + 3, nr - 1);
-    L.pn = f4[(size_t)kn * plane + ij];
-    L.rn = f3[(size_t)kn * plane + ij];
-    if constexpr (RECON) {
-      L.wpn = w0[4 * nf + (size_t)kn * plane + ij];
-      L.wrn = w0[3 * nf + (size_t)kn * plane + ij];
-    }
-    // per-point inputs of the RHS, prefetched with the plane: a load issued
-    // in the body would be waited on together with the whole prefetch
-    const size_t dx = (size_t)P * nf + kp;
-    L.c2 = c2base[c2f ? dx : 0];
     if constexpr (TL) {
-      L.tdc2 = tl_dc2[dx];
-      L.tdiv = tl_div[dx];
+      tdc2 = load_at<double>(bytes(A.tl_dc2) + dk, o8);
+      tdiv = load_at<double>(bytes(A.tl_div) + dk, o8);
     }
   };
 
-  const double Ci = to_global(T.ci)[ic], Dj = to_global(T.dj)[jc];
-  const double yCi = 1.0 / Ci, yDj = 1.0 / Dj;  // the divisors fixed for this thread's column
-  // Reciprocal-based quotients in the FP32-state stages only (c3 stage 2.87 ->
-  // 2.74 ms with a guard per quotient, and a further 1% with one guard per
-  // group); the FP64 stages divide in hardware (div_group).
-  const bool fdiv = T.fast_div != 0;
-  const double dc = to_global(T.dc)[ij], tdx = to_global(T.tdx)[ij], tde = to_global(T.tde)[ij],
-               xy = to_global(T.xy)[ij];
-
-  // Radial windows of p' and v_r over planes kb..kb+6 (storage type).
-  S pw[7], rw[7];
+  load_start(k0);
+  double Ci = to_global(ENS ? E.T.ci : A.T.ci)[ic], Dj = to_global(ENS ? E.T.dj : A.T.dj)[jc];
+  double dc = to_global(ENS ? E.T.dc : A.T.dc)[cell], tdx = to_global(ENS ? E.T.tdx : A.T.tdx)[cell],
+         tde = to_global(ENS ? E.T.tde : A.T.tde)[cell], xy = to_global(ENS ? E.T.xy : A.T.xy)[cell];
+  // Radial windows of p' and v_r over planes kb..kb+6.
+  double pw[7], rw[7];
   int kb = clampi(k0 - 3, 0, nr - 7);
 #pragma unroll
   for (int q = 0; q < 7; ++q) {  // (nr == 1, the 2-D case: every slot holds plane 0, with DDR weights 0)
-    const int kq = min(kb + q, nr - 1);
-    pw[q] = f4[(size_t)kq * plane + ij];
-    rw[q] = f3[(size_t)kq * plane + ij];
+    const size_t kq = (size_t)min(kb + q, nr - 1) * ps;
+    pw[q] = load_at<S>(qb + kq + 4 * fs, off);
+    rw[q] = load_at<S>(qb + kq + 3 * fs, off);
     if constexpr (RECON) {
-      pw[q] = pw[q] + beta_r * w0[4 * nf + (size_t)kq * plane + ij];
-      rw[q] = rw[q] + beta_r * w0[3 * nf + (size_t)kq * plane + ij];
+      pw[q] = pw[q] + A.beta_r * load_at<S>(wb + kq + 4 * fs, off);
+      rw[q] = rw[q] + A.beta_r * load_at<S>(wb + kq + 3 * fs, off);
     }
   }
-  // The next plane is loaded while this one is computed (a second plane in
-  // flight was measured: no gain for FP64 or FP32 storage).  Each iteration
-  // ends by moving the prefetched registers into place, which waits for
-  // every vector-memory operation issued before it (the counter retires in
-  // issue order).  So a plane's results are held in registers and stored at
-  // the top of the next iteration, before its prefetch: by the end of that
-  // iteration the stores have had a whole plane's computation to retire.
-  StagePlane<S> nxt;
-  load_plane(k0, nxt);
-  S pq0, pq1, pq2, pq3, pq4, pw0, pw1, pw2, pw3, pw4;  // the previous plane's q, qw (or RHS)
-  size_t px = 0;
-  int pk = 0;  // the plane of px
-  auto flush = [&]() {
-    const S pq[5] = {pq0, pq1, pq2, pq3, pq4}, pwv[5] = {pw0, pw1, pw2, pw3, pw4};
-    if (!own_in) {
-    } else if (rhs_mode) {
+  const double yCi = 1.0 / Ci, yDj = 1.0 / Dj;  // the divisors fixed for this thread's column
+  const bool fdiv = (ENS ? E.T.fast_div : A.T.fast_div) != 0;
+  // Everything loaded so far arrives before the loop, so that the waits inside
+  // it are those of its own loads.
+  asm volatile("" : "+v"(dc), "+v"(tdx), "+v"(tde), "+v"(xy), "+v"(Ci), "+v"(Dj));
 #pragma unroll
-      for (int f = 0; f < 5; ++f) o0[f * nf + px] = pq[f];
-    } else {
+  for (int q = 0; q < 7; ++q) asm volatile("" : "+v"(pw[q]), "+v"(rw[q]));
+  asm volatile("" : "+v"(pn), "+v"(rn), "+v"(vx_n), "+v"(ve_n));
+  if constexpr (RECON) asm volatile("" : "+v"(wpn), "+v"(wrn), "+v"(w1_n), "+v"(w2_n));
 #pragma unroll
-      for (int f = 0; f < 5; ++f) {
-        if (!NOQ) __builtin_nontemporal_store(pq[f], o0 + f * nf + px);
-        if (KIND != 2) __builtin_nontemporal_store(pwv[f], wo0 + f * nf + px);
-      }
-      if (ec_on) {
-        const size_t x = ec_base + (size_t)pk * edge_cols_plane(n);
-#pragma unroll
-        for (int f = 0; f < 5; ++f)
-          if (KIND == 2 || f == 1 || f == 2 || f == 4) ecw[x + (size_t)f * 3 * n] = pq[f];
-      }
-    }
-  };
+  for (int c = 0; c < NHC; ++c) {
+    asm volatile("" : "+v"(hp[c]), "+v"(hv[c]), "+v"(gp[c]), "+v"(gv[c]));
+    if constexpr (RECON) asm volatile("" : "+v"(rp[c]), "+v"(rv[c]));
+  }
+  load_update(k0);
 
   for (int k = k0; k < k1; ++k) {
-    const StagePlane<S> cur = nxt;
-    if (k > k0) flush();
-    load_plane(min(k + 1, k1 - 1), nxt);  // the last plane's prefetch is loaded and not used
     const int want = clampi(k - 3, 0, nr - 7);
     if (want != kb) {  // slides by exactly one plane: plane k+3 enters
 #pragma unroll
@@ -650,84 +609,68 @@ __global__ __launch_bounds__(TI* TJ) SOLAR_STAGE_ATTR void k_stage(DevTables Tar
         pw[q] = pw[q + 1];
         rw[q] = rw[q + 1];
       }
-      pw[6] = RECON ? cur.pn + beta_r * cur.wpn : cur.pn;
-      rw[6] = RECON ? cur.rn + beta_r * cur.wrn : cur.rn;
+      pw[6] = RECON ? pn + A.beta_r * wpn : pn;
+      rw[6] = RECON ? rn + A.beta_r * wrn : rn;
       kb = want;
     }
-    // p', v_r at plane k: window slot k - kb (3 on interior planes)
+    // p', v_r at plane k: window slot k - kb, 3 on interior planes
     const int wk = k - kb;
-    S pcs = pw[0], rcs = rw[0];
+    double pc = pw[3], rc = rw[3];
+    if (wk != 3) {
+      asm volatile("");  // stays a branch
 #pragma unroll
-    for (int q = 1; q < 7; ++q) {
-      pcs = wk == q ? pw[q] : pcs;
-      rcs = wk == q ? rw[q] : rcs;
+      for (int q = 0; q < 7; ++q) {
+        pc = wk == q ? pw[q] : pc;
+        rc = wk == q ? rw[q] : rc;
+      }
     }
-    const double pc = pcs, rc = rcs;
     const int bf = k & 1;
-    // the stage input at the own point (RECON: rebuilt from q and qw)
-    const double vx = RECON ? cur.vx + beta_r * cur.w[1] : cur.vx;
-    const double ve = RECON ? cur.ve + beta_r * cur.w[2] : cur.ve;
-    const double q1 = RECON ? cur.q1 + beta_r * cur.w[0] : cur.q1;
-    double own_p = pc, own_vx = vx, own_ve = ve;
-    if constexpr (PART) {
-      if (og == 1) {
-        own_p = cur.ogp;
-        own_vx = cur.ogv;
-      } else if (og == 2) {
-        own_p = cur.ogp;
-        own_ve = cur.ogv;
+    const double vx = RECON ? vx_n + A.beta_r * w1_n : vx_n;
+    const double ve = RECON ? ve_n + A.beta_r * w2_n : ve_n;
+    const S w1 = w1_n, w2 = w2_n;  // RECON: used by the update as well
+    if (own_in) {
+      sp[bf][ty + 3][tx + 3] = pc;
+      svx[bf][ty][tx + 3] = vx;
+      sve[bf][ty + 3][tx + 3] = ve;
+    }
+#pragma unroll
+    for (int c = 0; c < NHC; ++c) {
+      // field halo cells (rebuilt); ghost cells are the gathered stage input
+      double p = RECON ? hp[c] + A.beta_r * rp[c] : hp[c];
+      double v = RECON ? hv[c] + A.beta_r * rv[c] : hv[c];
+      if (wave_g[c]) {
+        p = hg[c] ? gp[c] : p;
+        v = hg[c] ? gv[c] : v;
+      }
+      if (hin[c]) {
+        sp[bf][hrow[c]][hcol[c]] = p;
+        if (xh[c])
+          svx[bf][hrow[c] - 3][hcol[c]] = v;
+        else
+          sve[bf][hrow[c]][hcol[c]] = v;
       }
     }
-    sp[bf][ty + 3][tx + 3] = own_p;
-    svx[bf][ty][tx + 3] = own_vx;
-    sve[bf][ty + 3][tx] = own_ve;
-    if constexpr (RECON) {  // field halo cells rebuilt; ghost cells are the gathered stage input
-      if (hx) {
-        sp[bf][ty + 3][hx_col] = hx_g ? cur.hpx : cur.hpx + beta_r * cur.rpx;
-        svx[bf][ty][hx_col] = hx_g ? cur.hvx : cur.hvx + beta_r * cur.rvx;
-      }
-      if (hy0) {
-        sp[bf][ty][tx + 3] = hy0_g ? cur.hpy0 : cur.hpy0 + beta_r * cur.rpy0;
-        sve[bf][ty][tx] = hy0_g ? cur.hve0 : cur.hve0 + beta_r * cur.rve0;
-      }
-      if (hy1) {
-        sp[bf][ty + 6][tx + 3] = hy1_g ? cur.hpy1 : cur.hpy1 + beta_r * cur.rpy1;
-        sve[bf][ty + 6][tx] = hy1_g ? cur.hve1 : cur.hve1 + beta_r * cur.rve1;
-      }
-    } else {
-      if (hx) {
-        sp[bf][ty + 3][hx_col] = kWide || hx_g ? cur.hpx : static_cast<double>(cur.fpx);
-        svx[bf][ty][hx_col] = kWide || hx_g ? cur.hvx : static_cast<double>(cur.fvx);
-      }
-      if (hy0) {
-        sp[bf][ty][tx + 3] = kWide || hy0_g ? cur.hpy0 : static_cast<double>(cur.fpy0);
-        sve[bf][ty][tx] = kWide || hy0_g ? cur.hve0 : static_cast<double>(cur.fve0);
-      }
-      if (hy1) {
-        sp[bf][ty + 6][tx + 3] = kWide || hy1_g ? cur.hpy1 : static_cast<double>(cur.fpy1);
-        sve[bf][ty + 6][tx] = kWide || hy1_g ? cur.hve1 : static_cast<double>(cur.fve1);
-      }
-    }
+    load_start(min(k + 1, k1 - 1));  // the last plane's is loaded and not used
     __syncthreads();
 
     // 7-point DRP stencils, ascending taps from 0 (derivative.f90:137-148,
     // 456-467, 656-668, 704-754).  In xi and eta the coefficients are the
-    // same (d_eta = d_xi) and the centre tap is 0 (both checked when the
-    // tables are uploaded): its product, +-0 for a finite value, leaves the
-    // sum unchanged, so it is not formed.  Fewer uniform operands also keep
-    // the kernel's scalar registers from spilling.
+    // same (d_eta = d_xi), antisymmetric, and the centre tap is 0 (checked
+    // when the tables are uploaded): its product, +-0 for a finite value,
+    // leaves the sum unchanged, so it is not formed.
+    const double tap[7] = {-c6, -c5, -c4, 0.0, c4, c5, c6};
     double dvx = 0.0, dve = 0.0, dpx = 0.0, dpe = 0.0, dvr = 0.0, dpr = 0.0;
     // the radial row is block-uniform and read-only: through the constant
     // address space it comes in with scalar loads, which the vector-load
     // waits do not count
-    const auto& row = const_rows(T.rad)[k];
+    const auto& row = rows[k];
 #pragma unroll
     for (int q = 0; q < 7; ++q) {
       if (q != 3) {
-        dvx = dvx + T.fcx[q] * svx[bf][ty][tx + q];
-        dve = dve + T.fcx[q] * sve[bf][ty + q][tx];
-        dpx = dpx + T.fcx[q] * sp[bf][ty + 3][tx + q];
-        dpe = dpe + T.fcx[q] * sp[bf][ty + q][tx + 3];
+        dvx = dvx + tap[q] * svx[bf][ty][tx + q];
+        dve = dve + tap[q] * sve[bf][ty + q][tx + 3];
+        dpx = dpx + tap[q] * sp[bf][ty + 3][tx + q];
+        dpe = dpe + tap[q] * sp[bf][ty + q][tx + 3];
       }
       dvr = dvr + row.w[q] * rw[q];
       dpr = dpr + row.w[q] * pw[q];
@@ -737,12 +680,13 @@ __global__ __launch_bounds__(TI* TJ) SOLAR_STAGE_ATTR void k_stage(DevTables Tar
     // quotients by C, D, r and rho0 (grad.f90:52-53, 128-130;
     // compute_rhs_acoustic.f90:88-146), in two groups: the second divides
     // the first's results
+    const double q1 = RECON ? q1_n + A.beta_r * w_n[0] : q1_n;
     double qa[7];
     {
       const double na[7] = {dvx, dve, 2.0 * rc, xy * dpe, xy * dpx, dpr, q1 * row.g0};
       const double ba[7] = {Ci, Dj, row.r, Dj, Ci, row.rho0, row.rho0};
       const double ya[7] = {yCi, yDj, row.inv_r, yDj, yCi, row.inv_rho0, row.inv_rho0};
-      div_group<kWide ? false : true>(na, ba, ya, fdiv, qa);
+      div_group<kStageRcp<S>>(na, ba, ya, fdiv, qa);
     }
     const double div = (row.inv_r * ((dc * (qa[0] + qa[1]) - tdx * vx) - tde * ve) + dvr) + qa[2];
     const double gxi = row.inv_r * (Dj * dpx + qa[3]);
@@ -751,70 +695,101 @@ __global__ __launch_bounds__(TI* TJ) SOLAR_STAGE_ATTR void k_stage(DevTables Tar
     // compute_rhs_acoustic.f90:38-149 (forcing omitted).
     double r1 = -(row.rho0 * div);
     r1 = r1 - rc * row.drho0dr;
-    double qb[2];
+    double qc[2];
     {
       const double nb[2] = {gxi, get};
       const double bb[2] = {row.rho0, row.rho0};
       const double yb[2] = {row.inv_rho0, row.inv_rho0};
-      div_group<kWide ? false : true>(nb, bb, yb, fdiv, qb);
+      div_group<kStageRcp<S>>(nb, bb, yb, fdiv, qc);
     }
-    double r2 = -qb[0];
-    double r3 = -qb[1];
+    double r2 = -qc[0];
+    double r3 = -qc[1];
     double r4 = -qa[5];
     r4 = r4 - qa[6];
     // c2f: optional 3-D c^2 (n,n,nr,6); the radial profile otherwise
-    const double c2rho0 = c2f ? cur.c2 * row.rho0 : row.c2rho0;
-    const size_t dx = (size_t)P * nf + (size_t)k * plane + ij;
-    if (divout && own_in) {  // div(v) of the stage input, kept for the adjoint (FP64, or FP32 when div32)
-      if (div32)
-        reinterpret_cast<float*>(divout)[dx] = static_cast<float>(div);
-      else
-        divout[dx] = div;
+    double c2rho0 = row.c2rho0;
+    if (AUX || TL) {
+      if (A.c2f) c2rho0 = c2_n * row.rho0;
+    }
+    if constexpr (AUX) {
+      if (A.divout && own_in) {  // div(v) of the stage input, kept for the adjoint (FP64, or FP32 when div32)
+        const size_t dk = (size_t)P * nf + (size_t)k * plane;
+        if (A.div32)
+          store_at(bytes(A.divout) + dk * 4, cell * 4u, static_cast<float>(div));
+        else
+          store_at(bytes(A.divout) + dk * 8, cell * 8u, div);
+      }
     }
     double r5 = -(c2rho0 * div);
     // tangent-linear run: d r5 / d c^2 = -rho0 div of the primal stage input
-    if constexpr (TL) r5 = r5 - (cur.tdc2 * row.rho0) * cur.tdiv;
+    if constexpr (TL) r5 = r5 - (tdc2 * row.rho0) * tdiv;
     r5 = r5 + row.rho0g0 * rc;
 
     // no BC_RHS and no SPONGE in 2-D (bc_acoustic_wave.f90:11, sponge.f90:18)
-    const bool do_bc = (rhs_mode ? (rhs_mode & 1) : true) && nr > 1;
-    const bool do_sp = (rhs_mode ? (rhs_mode & 2) : true) && nr > 1;
+    const bool do_bc = (RHS ? (A.rhs_mode & 1) : true) && nr > 1;
+    const bool do_sp = (RHS ? (A.rhs_mode & 2) : true) && nr > 1;
     if (do_bc && (k == 0 || k == nr - 1)) {  // bc_acoustic_wave.f90:14-34
+      asm volatile("");  // stays a branch
       r1 = 0.0; r2 = 0.0; r3 = 0.0; r4 = 0.0; r5 = 0.0;
     }
     if (do_sp) {  // sponge.f90:48-50, after BC_RHS (timestep.f90:65-66)
+      asm volatile("");
       const double sg = row.sigma;
       r1 = r1 - sg * (q1 - 0.0);
       r4 = r4 - sg * (rc - 0.0);
       r5 = r5 - sg * (pc - 0.0);
     }
 
-    px = (size_t)k * plane + ij;
-    pk = k;
-    if (rhs_mode) {
-      pq0 = static_cast<S>(r1);
-      pq1 = static_cast<S>(r2);
-      pq2 = static_cast<S>(r3);
-      pq3 = static_cast<S>(r4);
-      pq4 = static_cast<S>(r5);
+    const size_t kp = (size_t)k * ps;
+    const unsigned o = lane_offset(off);
+    if constexpr (RHS) {
+      const double r[5] = {r1, r2, r3, r4, r5};
+      load_update(min(k + 1, k1 - 1));
+      if (own_in) {
+#pragma unroll
+        for (int f = 0; f < 5; ++f) store_at(ob + kp + f * fs, o, static_cast<S>(r[f]));
+      }
     } else {
       // timestep.f90:68-69: qw = alpha*qw + dt*rhs ; q = q + beta*qw
-      const double w0n = alpha * cur.w[0] + dt * r1, w1n = alpha * cur.w[1] + dt * r2,
-                   w2n = alpha * cur.w[2] + dt * r3, w3n = alpha * cur.w[3] + dt * r4,
-                   w4n = alpha * cur.w[4] + dt * r5;
-      pq0 = static_cast<S>(q1 + beta * w0n);
-      pq1 = static_cast<S>(vx + beta * w1n);
-      pq2 = static_cast<S>(ve + beta * w2n);
-      pq3 = static_cast<S>(rc + beta * w3n);
-      pq4 = static_cast<S>(pc + beta * w4n);
-      pw0 = static_cast<S>(w0n);
-      pw1 = static_cast<S>(w1n);
-      pw2 = static_cast<S>(w2n);
-      pw3 = static_cast<S>(w3n);
-      pw4 = static_cast<S>(w4n);
+      const double r[5] = {r1, r2, r3, r4, r5}, x[5] = {q1, vx, ve, rc, pc};
+      S wn[5], qn[5];
+#pragma unroll
+      for (int f = 0; f < 5; ++f) {
+        const S w = RECON && f == 1 ? w1 : RECON && f == 2 ? w2 : w_n[f];
+        const double wd = (KIND == 0 ? 0.0 : A.alpha * w) + dt * r[f];
+        qn[f] = static_cast<S>(x[f] + A.beta * wd);
+        wn[f] = static_cast<S>(wd);
+      }
+      load_update(min(k + 1, k1 - 1));
+      if (own_in) {
+        // Non-temporal stores, except where rows or tiles begin inside a
+        // 64-byte segment: a neighbouring tile completes that segment in L2
+        // (stage, 6x204^2x100: 1.03 -> 0.95 ms; with whole segments,
+        // 6x200^2x150, plain stores are slower: 1.17 -> 1.24 ms).
+        if (PART && !A.whole) {
+          asm volatile("");  // stays a branch
+#pragma unroll
+          for (int f = 0; f < 5; ++f) {
+            if (!NOQ) store_at(ob + kp + f * fs, o, qn[f]);
+            if (KIND != 2) store_at(wob + kp + f * fs, o, wn[f]);
+          }
+        } else {
+#pragma unroll
+          for (int f = 0; f < 5; ++f) {
+            if (!NOQ) store_at_nt(ob + kp + f * fs, o, qn[f]);
+            if (KIND != 2) store_at_nt(wob + kp + f * fs, o, wn[f]);
+          }
+        }
+      }
+      if (ec_on) {
+        const GlobalBytes e = ecb + (size_t)k * edge_cols_plane(n) * sizeof(S);
+        const unsigned eo = lane_offset(ec_off);
+#pragma unroll
+        for (int f = 0; f < 5; ++f)
+          if (KIND == 2 || f == 1 || f == 2 || f == 4) store_at(e + (size_t)f * 3 * n * sizeof(S), eo, qn[f]);
+      }
     }
   }
-  flush();
   if constexpr (ENS) __syncthreads();  // the next item rewrites the LDS tiles
   }
 }
@@ -1220,7 +1195,6 @@ __global__ void k_place(const double* __restrict__ src, S* __restrict__ dst, siz
 
 // ---------------------------------------------------------------- launchers
 
-static int pick_ti(int n) { return (n % 32 == 0) ? 32 : 16; }
 
 int chunks_for(int tiles, int nr, int target_blocks, int min_chunk) {
   int nk = (target_blocks + tiles - 1) / tiles;
@@ -1235,7 +1209,7 @@ int chunks_for(int tiles, int nr, int target_blocks, int min_chunk) {
 // time, (rounds of blocks) x (planes per block + warm).  The first rule,
 // chunks_for, keeps chunks long, for the bytes that a chunk's window re-reads;
 // a small grid lies in the caches and is bound by the serial chain of its
-// planes instead (about 2 us a plane in the stage kernels, 0.5 in the filter).
+// planes instead (about 1.8 us a plane in the stage kernels, 0.5 in the filter).
 //   warm: planes' worth of work before a block's first output;
 //   resident: blocks a CU holds; one block alone runs `alone` times as long
 //   per plane as its share of a full CU.
@@ -1307,67 +1281,94 @@ hipError_t launch_gather(const DevTables& T, const void* q, bool f32, bool vec, 
                          gxs, gys, gxv, gyv, st, static_cast<const double*>(qwr), betar);
 }
 
+// Threads of a stage block with tiles of width w: its points, and its halo
+// cells (6 w above and below, filled up to a wave, and 6 tj beside).
+constexpr int part_threads(int w, int tj) {
+  const int points = (w * tj + 63) / 64 * 64, halo = ((6 * w + 63) / 64 * 64 + 6 * tj + 63) / 64 * 64;
+  return points > halo ? points : halo;
+}
+// PART: a.tile_w is the tile width (at most TI).
 template <int TI, int TJ, typename S, bool PART = false>
-static hipError_t launch_stage_t(const DevTables& T, const S* qin, S* qout, S* qw, const double* gxp,
-                                 const double* gyp, const double* gxv, const double* gyv, int stage, double dt,
-                                 int rhs_mode, hipStream_t st, const LaunchShape& ls, const double* c2f,
-                                 double* divout, int div32, const double* tl_dc2, const double* tl_div, S* ecols,
-                                 int xf, S* qwo, double beta_r) {
-  const int tiles = ((T.n + TI - 1) / TI) * ((T.n + TJ - 1) / TJ) * 6;
+static hipError_t launch_stage_t(StageArgs<S> a, int stage, int xf, hipStream_t st, const LaunchShape& ls) {
+  const DevTables& T = a.T;
+  const int W = PART ? a.tile_w : TI;
+  const int tiles = ((T.n + W - 1) / W) * ((T.n + TJ - 1) / TJ) * 6;
   // radial chunks of >= 24 planes, ~12k blocks, at most 8 chunks: 8 chunks measured best at
   // 6x96^2x192 (0.342 ms per stage against 0.375 with 6), 6x128^2x256 and 6x256^2x384
   int nkch = std::min(8, chunks_for(tiles, T.nr, 12288, 24));
-  // below four rounds of 512 blocks the split with the shortest chain
-  // (us per stage, before -> after: 6x16^2x24 56 -> 10, 6x32^2x64 79 -> 23,
-  // 6x64^2x64 85 -> 61, 6x128^2x64 209 -> 202, FP32 state 6x64^2x128 83 -> 67;
-  // at 1728 blocks, 6x96^2x192, the long chunks are still the best: 332 against
-  // 343 at half their length).  The FP32 state runs three blocks a CU, FP64 two.
-  if (tiles * nkch < 1536) nkch = small_grid_chunks(tiles, T.nr, 1.0, sizeof(S) == 4 ? 3 : 2, 1.25);
+  // below two rounds of three blocks a CU the split with the shortest chain
+  // (us per stage, before -> after: 6x16^2x24 49 -> 9, 6x32^2x64 71 -> 21,
+  // 6x64^2x64 78 -> 51, FP32 state 6x64^2x128 75 -> 58, 6x128^2x128 345 -> 336;
+  // at 1728 blocks, 6x96^2x192, 24-plane chunks are still the best: 294
+  // against 318 at 20 planes, 308 at 16)
+  if (tiles * nkch < 1536) nkch = small_grid_chunks(tiles, T.nr, 1.0, 3, 1.25);
   if (ls.stage_chunks > 0) nkch = ls.stage_chunks;
-  const int kchunk = (T.nr + nkch - 1) / nkch;
-  dim3 grid(tiles * nkch), block(TI, TJ);
-  const double al = kAlphaRk4[stage < 0 ? 0 : stage], be = kBetaRk4[stage < 0 ? 0 : stage];
-  const int kind = (rhs_mode || stage == 0) ? 0 : (stage < 4 ? 1 : 2);
-#define SOLAR_STAGE_LAUNCH(K, M, X)                                                                                  \
-  hipLaunchKernelGGL((k_stage<TI, TJ, K, S, M, PART, X>), grid, block, 0, st, T, qin, qout, qw, gxp, gyp, gxv, gyv,  \
-                     al, be, dt, kchunk, nkch, rhs_mode, c2f, divout, div32, tl_dc2, tl_div, ecols, nullptr, nullptr, \
-                     0, 0, qwo, beta_r)
-  if (xf) {
-    // stored-q schedule variants: FP64, 32x8 and 16x16 tiles, no RHS or tangent-linear mode
-    constexpr bool kHave = sizeof(S) == 8 && ((TI == 32 && TJ == 8) || (TI == 16 && TJ == 16));
-    if constexpr (kHave) {
-      if (rhs_mode || tl_dc2) return hipErrorInvalidValue;
-      if (xf == kStoreNoQ && kind == 0)
-        SOLAR_STAGE_LAUNCH(0, 0, kStoreNoQ);
-      else if (xf == kStoreNoQ && kind == 1)
-        SOLAR_STAGE_LAUNCH(1, 0, kStoreNoQ);
-      else if (xf == kStageRecon && kind == 1 && qwo)
-        SOLAR_STAGE_LAUNCH(1, 0, kStageRecon);
-      else
-        return hipErrorInvalidValue;
+  a.whole = T.n * sizeof(S) % 64 == 0 && W * sizeof(S) % 64 == 0;
+  a.nkch = nkch;
+  a.kchunk = (T.nr + nkch - 1) / nkch;
+  const dim3 grid(tiles * nkch), block = PART ? dim3(part_threads(W, TJ)) : dim3(TI, TJ);
+  a.alpha = kAlphaRk4[stage < 0 ? 0 : stage];
+  a.beta = kBetaRk4[stage < 0 ? 0 : stage];
+  const int kind = stage <= 0 ? 0 : (stage < 4 ? 1 : 2);
+#define SOLAR_STAGE_LAUNCH(K, M, FL) hipLaunchKernelGGL((k_stage<TI, TJ, K, S, M, PART, FL>), grid, block, 0, st, a)
+  if (a.rhs_mode) {
+    if (xf || a.tl_dc2 || a.divout) return hipErrorInvalidValue;
+    SOLAR_STAGE_LAUNCH(0, 0, kStageRhs);
+    return hipGetLastError();
+  }
+  // the variants beyond the plain stages: 64x8, 32x8 and 16x16 tiles
+  constexpr bool kMain = (TI == 64 && TJ == 8) || (TI == 32 && TJ == 8) || (TI == 16 && TJ == 16);
+  const bool aux = a.c2f || a.divout;
+  if constexpr (kMain && sizeof(S) == 8) {
+    if (xf) {
+      if (a.tl_dc2) return hipErrorInvalidValue;
+#define SOLAR_STAGE_XF(AUX)                                     \
+  if (xf == kStoreNoQ && kind == 0)                             \
+    SOLAR_STAGE_LAUNCH(0, 0, kStoreNoQ | (AUX));                \
+  else if (xf == kStoreNoQ && kind == 1)                        \
+    SOLAR_STAGE_LAUNCH(1, 0, kStoreNoQ | (AUX));                \
+  else if (xf == kStageRecon && kind == 1 && a.qwo)             \
+    SOLAR_STAGE_LAUNCH(1, 0, kStageRecon | (AUX));              \
+  else                                                          \
+    return hipErrorInvalidValue;
+      if (aux) {
+        SOLAR_STAGE_XF(kStageAux)
+      } else {
+        SOLAR_STAGE_XF(0)
+      }
+#undef SOLAR_STAGE_XF
       return hipGetLastError();
+    }
+    if constexpr (!PART) {  // the tangent-linear stage: FP64, tiles that divide n
+      if (a.tl_dc2) {
+        if (kind == 0)
+          SOLAR_STAGE_LAUNCH(0, 2, 0);
+        else if (kind == 1)
+          SOLAR_STAGE_LAUNCH(1, 2, 0);
+        else
+          SOLAR_STAGE_LAUNCH(2, 2, 0);
+        return hipGetLastError();
+      }
+    }
+  }
+  if (xf || a.tl_dc2) return hipErrorInvalidValue;
+#define SOLAR_STAGE_KIND(FL)      \
+  if (kind == 0)                  \
+    SOLAR_STAGE_LAUNCH(0, 0, FL); \
+  else if (kind == 1)             \
+    SOLAR_STAGE_LAUNCH(1, 0, FL); \
+  else                            \
+    SOLAR_STAGE_LAUNCH(2, 0, FL);
+  if (aux) {
+    if constexpr (kMain) {
+      SOLAR_STAGE_KIND(kStageAux)
     } else {
       return hipErrorInvalidValue;
     }
-  }
-  if (tl_dc2) {
-    if constexpr (sizeof(S) == 8 && !PART) {
-      if (kind == 0)
-        SOLAR_STAGE_LAUNCH(0, 2, 0);
-      else if (kind == 1)
-        SOLAR_STAGE_LAUNCH(1, 2, 0);
-      else
-        SOLAR_STAGE_LAUNCH(2, 2, 0);
-    } else {
-      return hipErrorInvalidValue;  // the tangent-linear stage is FP64 only, on tiles that divide n
-    }
-  } else if (kind == 0) {
-    SOLAR_STAGE_LAUNCH(0, 0, 0);
-  } else if (kind == 1) {
-    SOLAR_STAGE_LAUNCH(1, 0, 0);
   } else {
-    SOLAR_STAGE_LAUNCH(2, 0, 0);
+    SOLAR_STAGE_KIND(0)
   }
+#undef SOLAR_STAGE_KIND
 #undef SOLAR_STAGE_LAUNCH
   return hipGetLastError();
 }
@@ -1378,56 +1379,92 @@ static hipError_t launch_stage_t(const DevTables& T, const S* qin, S* qout, S* q
 // shape divides n (n not a multiple of 16), the partial-tile kernels run with
 // 32-wide or 16-wide tiles, whichever pads n less (ties to 32).
 static bool fits(int n, int ti, int tj) { return ti > 0 && tj > 0 && n % ti == 0 && n % tj == 0; }
+// Width of a partial-tile panel's stage tiles: from 64 down to 33, the one
+// that leaves the fewest lanes without a point, the widest of near equals (us
+// per stage, 6x200^2x150: 40 wide 1177, 50 1432, 34 1608, 16x16 tiles 1240;
+// 6x250^2x60: 63 wide 771, 50 856, 42 895).  Multiples of 8 where the rows
+// are.  One shell makes too few blocks to fill the chip: there the narrowest
+// of near equals, down to 26 (6x204^2: 30 wide 19.9, 51 22.8; 6x250^2: 32 wide
+// 24.2, 63 26.2).
+static int part_width(int n, int nr) {
+  const int narrow = nr == 1 ? 26 : 33;
+  int best = 0;
+  double least = 0.0;
+  for (int t = (n + 63) / 64; t <= (n + narrow - 1) / narrow || t == (n + 63) / 64; ++t) {
+    int w = (n + t - 1) / t;
+    if (n % 8 == 0) w = (w + 7) / 8 * 8;
+    const double lanes = (double)part_threads(w, 8) * t;
+    if (least == 0.0 || lanes < (nr == 1 ? 1.03 : 0.97) * least) {
+      least = lanes;
+      best = w;
+    }
+  }
+  return best;
+}
 static int pad_pick_ti(int n) { return ((n + 31) / 32) * 32 <= ((n + 15) / 16) * 16 ? 32 : 16; }
 
 template <typename S>
-static hipError_t launch_stage_s(const DevTables& T, const S* qin, S* qout, S* qw, const double* gxp, const double* gyp,
-                                 const double* gxv, const double* gyv, int stage, double dt, int rhs_mode,
-                                 hipStream_t st, const LaunchShape& ls, const double* c2f, double* divout,
-                                 int div32, const double* tl_dc2, const double* tl_div, S* ecols, int xf, S* qwo,
-                                 double beta_r) {
-#define SOLAR_STAGE_ARGS \
-  T, qin, qout, qw, gxp, gyp, gxv, gyv, stage, dt, rhs_mode, st, ls, c2f, divout, div32, tl_dc2, tl_div, ecols, xf, qwo, beta_r
-  if (T.n % 16 != 0) {  // partial tiles: 32x8 or 16x16
-    if (pad_pick_ti(T.n) == 32) return launch_stage_t<32, 8, S, true>(SOLAR_STAGE_ARGS);
-    return launch_stage_t<16, 16, S, true>(SOLAR_STAGE_ARGS);
+static hipError_t launch_stage_s(StageArgs<S> a, int stage, int xf, hipStream_t st, const LaunchShape& ls) {
+  const int n = a.T.n;
+  if (n % 16 != 0) {
+    a.tile_w = part_width(n, a.T.nr);
+    return launch_stage_t<64, 8, S, true>(a, stage, xf, st, ls);
   }
   int ti = ls.stage_ti, tj = ls.stage_tj;
-  // measured best: 32x8 (64x8 within 2%), then 16x16; the stored-q schedule
-  // variants exist for these two only
-  if (!fits(T.n, ti, tj) || (xf && !((ti == 32 && tj == 8) || (ti == 16 && tj == 16)))) {
-    ti = pick_ti(T.n);
-    tj = ti == 64 ? 8 : 256 / ti;
+  // Measured best (us per stage): 64x8 on panels from 128 (32x8 there:
+  // 6x128^2x256 660 -> 705, and the 6x256^2x384 step 24.9 -> 23.7 ms: fewer
+  // halo cells), 32x8 on smaller ones that 32 divides (6x64^2x64 52 against 58
+  // for 64x8), else 16x16.  The variants of the stored-q schedule, of a c^2
+  // field, kept divergences or a tangent-linear run exist for these three.
+  const bool plain = !xf && !a.c2f && !a.divout && !a.tl_dc2;
+  if (!fits(n, ti, tj) || (!plain && !((ti == 64 && tj == 8) || (ti == 32 && tj == 8) || (ti == 16 && tj == 16)))) {
+    ti = n % 64 == 0 && n >= 128 ? 64 : n % 32 == 0 ? 32 : 16;
+    tj = ti == 16 ? 16 : 8;
   }
-#define SOLAR_STAGE_CASE(A, B) \
-  if (ti == A && tj == B) return launch_stage_t<A, B, S>(SOLAR_STAGE_ARGS);
+#define SOLAR_STAGE_CASE(X, Y) \
+  if (ti == X && tj == Y) return launch_stage_t<X, Y, S>(a, stage, xf, st, ls);
   SOLAR_STAGE_CASE(64, 8)
   SOLAR_STAGE_CASE(64, 4)
-  SOLAR_STAGE_CASE(32, 8)
-  SOLAR_STAGE_CASE(16, 16)
   SOLAR_STAGE_CASE(32, 16)
   SOLAR_STAGE_CASE(32, 4)
+  SOLAR_STAGE_CASE(32, 8)
 #undef SOLAR_STAGE_CASE
-  ti = pick_ti(T.n);
-  if (ti == 64) return launch_stage_t<64, 8, S>(SOLAR_STAGE_ARGS);
-  if (ti == 32) return launch_stage_t<32, 8, S>(SOLAR_STAGE_ARGS);
-  return launch_stage_t<16, 16, S>(SOLAR_STAGE_ARGS);
-#undef SOLAR_STAGE_ARGS
+  return launch_stage_t<16, 16, S>(a, stage, xf, st, ls);
+}
+
+template <typename S>
+static StageArgs<S> stage_args(const DevTables& T, const void* qin, void* qout, void* qw, void* qwo, void* ecols) {
+  StageArgs<S> a{};
+  a.T = T;
+  a.qin = static_cast<const S*>(qin);
+  a.qout = static_cast<S*>(qout);
+  a.qw = static_cast<S*>(qw);
+  a.qwo = static_cast<S*>(qwo);
+  a.ecols = static_cast<S*>(ecols);
+  return a;
 }
 
 hipError_t launch_stage(const DevTables& T, const void* qin, void* qout, void* qw, bool f32, const double* gxp,
                         const double* gyp, const double* gxv, const double* gyv, int stage, double dt, int rhs_mode,
                         hipStream_t st, const LaunchShape& ls, const double* c2f, double* divout, int div32,
                         const double* tl_dc2, const double* tl_div, void* ecols, int xf, void* qwo, double beta_r) {
-  if (f32) {
-    if (xf) return hipErrorInvalidValue;  // the stored-q schedule variants are FP64
-    return launch_stage_s(T, static_cast<const float*>(qin), static_cast<float*>(qout), static_cast<float*>(qw), gxp,
-                          gyp, gxv, gyv, stage, dt, rhs_mode, st, ls, c2f, divout, div32, tl_dc2, tl_div,
-                          static_cast<float*>(ecols), 0, static_cast<float*>(nullptr), 0.0);
-  }
-  return launch_stage_s(T, static_cast<const double*>(qin), static_cast<double*>(qout), static_cast<double*>(qw), gxp,
-                        gyp, gxv, gyv, stage, dt, rhs_mode, st, ls, c2f, divout, div32, tl_dc2, tl_div,
-                        static_cast<double*>(ecols), xf, static_cast<double*>(qwo), beta_r);
+  auto go = [&](auto a) {
+    a.gxp = gxp;
+    a.gyp = gyp;
+    a.gxv = gxv;
+    a.gyv = gyv;
+    a.beta_r = beta_r;
+    a.dt = dt;
+    a.rhs_mode = rhs_mode;
+    a.c2f = c2f;
+    a.divout = divout;
+    a.div32 = div32;
+    a.tl_dc2 = tl_dc2;
+    a.tl_div = tl_div;
+    return launch_stage_s(a, stage, xf, st, ls);
+  };
+  // (the stored-q schedule variants and the tangent-linear stage are FP64: launch_stage_t refuses others)
+  return f32 ? go(stage_args<float>(T, qin, qout, qw, qwo, ecols)) : go(stage_args<double>(T, qin, qout, qw, qwo, ecols));
 }
 
 template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4)>
@@ -1517,21 +1554,20 @@ hipError_t launch_place(const double* src, void* dst, bool f32, size_t nf, int d
 template <int TI, int TJ>
 static hipError_t launch_stage_ens_t(const EnsMember* M, const int4* items, int nitems, int grid, int stage, int cur,
                                      hipStream_t st) {
-  const double al = kAlphaRk4[stage], be = kBetaRk4[stage];
-  DevTables none{};
-  dim3 g(grid), block(TI, TJ);
+  StageArgs<double> a{};
+  a.alpha = kAlphaRk4[stage];
+  a.beta = kBetaRk4[stage];
+  a.M = M;
+  a.items = items;
+  a.nitems = nitems;
+  a.cur = cur;
+  const dim3 g(grid), block(TI, TJ);
   if (stage == 0)
-    hipLaunchKernelGGL((k_stage<TI, TJ, 0, double, 1>), g, block, 0, st, none, nullptr, nullptr, nullptr, nullptr,
-                       nullptr, nullptr, nullptr, al, be, 0.0, 0, 0, 0, nullptr, nullptr, 0, nullptr, nullptr, nullptr, M, items,
-                       nitems, cur, nullptr, 0.0);
+    hipLaunchKernelGGL((k_stage<TI, TJ, 0, double, 1>), g, block, 0, st, a);
   else if (stage < 4)
-    hipLaunchKernelGGL((k_stage<TI, TJ, 1, double, 1>), g, block, 0, st, none, nullptr, nullptr, nullptr, nullptr,
-                       nullptr, nullptr, nullptr, al, be, 0.0, 0, 0, 0, nullptr, nullptr, 0, nullptr, nullptr, nullptr, M, items,
-                       nitems, cur, nullptr, 0.0);
+    hipLaunchKernelGGL((k_stage<TI, TJ, 1, double, 1>), g, block, 0, st, a);
   else
-    hipLaunchKernelGGL((k_stage<TI, TJ, 2, double, 1>), g, block, 0, st, none, nullptr, nullptr, nullptr, nullptr,
-                       nullptr, nullptr, nullptr, al, be, 0.0, 0, 0, 0, nullptr, nullptr, 0, nullptr, nullptr, nullptr, M, items,
-                       nitems, cur, nullptr, 0.0);
+    hipLaunchKernelGGL((k_stage<TI, TJ, 2, double, 1>), g, block, 0, st, a);
   return hipGetLastError();
 }
 

@@ -74,8 +74,9 @@ hipError_t launch_gather(const DevTables& T, const void* q, bool f32, bool vec, 
 // xf (FP64 storage, not with rhs_mode or tl_dc2): kStoreNoQ, the stage
 // stores qw in place and the edge columns of its output, not q (qout unused);
 // kStageRecon (stages 2-4), the stage input is qin + beta_r * qw, its qw goes
-// to qwo (not qw) and its q to qout.  Tile shapes other than 32x8 and 16x16
-// are not compiled for these: requested ones fall back to the default.
+// to qwo (not qw) and its q to qout.  These, c2f, divout and
+// tl_dc2 are compiled for 64x8, 32x8 and 16x16 tiles: other requested shapes
+// fall back to the default.
 constexpr int kStoreNoQ = 1, kStageRecon = 2;
 hipError_t launch_stage(const DevTables& T, const void* qin, void* qout, void* qw, bool f32, const double* gxp,
                         const double* gyp, const double* gxv, const double* gyv, int stage, double dt, int rhs_mode,
