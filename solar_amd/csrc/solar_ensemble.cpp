@@ -58,9 +58,10 @@ struct solar_ens {
   struct GatherGroup {
     int* table = nullptr;
     int nm = 0, nblocks = 0, n = 0;
+    int chunks = 0;  // radial chunks per receiver edge
   };
   std::vector<GatherGroup> gg;
-  int gchunks = 4;  // radial chunks per receiver edge in the gathers
+  int gchunks = 0;  // > 0: the chunks of every group (launch-shape sweeps)
   int persist = 0;   // > 0: grid cap of the work-list launches
   std::vector<void*> allocs;
   std::vector<void*> list_allocs;  // work lists, rebuilt by the autotuner
@@ -181,21 +182,25 @@ int build_lists(solar_ens* e) {
 // ecols, from which the next gather reads its column strips (compact lines
 // instead of three values from every row of the state); the step's first
 // gather reads the filtered state.
+// The stages run the stored-q schedule of the single grid: q is stored after
+// stages 2, 4 and 5 only, and stages 2 and 4 rebuild their input as q + beta
+// qw (48 members as the batched workload draws them: 35.3 -> 32.9 ms per step, with
+// the gather chunks below).
 int enqueue_step(solar_ens* e) {
-  int cur = 0;
+  // q and qw buffer of each stage's input
+  static const int kQ[5] = {0, 0, 1, 1, 0}, kW[5] = {0, 0, 1, 1, 0};
   for (int s = 0; s < 5; ++s) {
+    const bool rebuilt = s == 1 || s == 3;
     for (const auto& G : e->gg)
-      ENSCHK(solar::launch_gather_ens(e->dmem, G.table, G.nm, G.nblocks, G.n, true, cur, s > 0, e->gchunks,
-                                      e->stream));
+      ENSCHK(solar::launch_gather_ens(e->dmem, G.table, G.nm, G.nblocks, G.n, true, kQ[s], s > 0, G.chunks, e->stream,
+                                      rebuilt ? kW[s] : -1, rebuilt ? solar::kBetaRk4[s - 1] : 0.0));
     for (const Launch& L : e->stage_l)
-      ENSCHK(solar::launch_stage_ens(e->dmem, L.items, L.nitems, L.grid, L.ti, L.tj, s, cur, e->stream));
-    cur ^= 1;
+      ENSCHK(solar::launch_stage_ens(e->dmem, L.items, L.nitems, L.grid, L.ti, L.tj, s, kQ[s], kW[s], e->stream));
   }
   for (const auto& G : e->gg)
-    ENSCHK(solar::launch_gather_ens(e->dmem, G.table, G.nm, G.nblocks, G.n, false, cur, true, e->gchunks,
-                                    e->stream));
+    ENSCHK(solar::launch_gather_ens(e->dmem, G.table, G.nm, G.nblocks, G.n, false, 1, true, G.chunks, e->stream));
   for (const Launch& L : e->filter_l)
-    ENSCHK(solar::launch_filter_ens(e->dmem, L.items, L.nitems, L.grid, L.ti, L.tj, cur, e->stream));
+    ENSCHK(solar::launch_filter_ens(e->dmem, L.items, L.nitems, L.grid, L.ti, L.tj, 1, e->stream));
   return SOLAR_OK;
 }
 
@@ -204,7 +209,8 @@ int clear_state(solar_ens* e) {
     const size_t b = static_cast<size_t>(e->n[m]) * e->n[m] * e->nr[m] * 30 * sizeof(double);
     ENSCHK(hipMemsetAsync(e->mem[m].q[0], 0, b, e->stream));
     ENSCHK(hipMemsetAsync(e->mem[m].q[1], 0, b, e->stream));
-    ENSCHK(hipMemsetAsync(e->mem[m].qw, 0, b, e->stream));
+    ENSCHK(hipMemsetAsync(e->mem[m].qw[0], 0, b, e->stream));
+    ENSCHK(hipMemsetAsync(e->mem[m].qw[1], 0, b, e->stream));
   }
   ENSCHK(hipStreamSynchronize(e->stream));
   return SOLAR_OK;
@@ -280,23 +286,24 @@ int solar_ens_create(solar_ens** out, int nmembers, const int* n, const int* nr,
     if (rc) return bail(rc);
     const size_t nq = static_cast<size_t>(n[m]) * n[m] * nr[m] * 30;
     const size_t ng = static_cast<size_t>(12) * nr[m] * n[m] * 3;
-    void* p[10];
-    const size_t sz[10] = {nq, nq, nq, ng, ng, ng, ng, 5 * ng, 5 * ng, solar::edge_cols_elems(n[m], nr[m])};
-    for (int a = 0; a < 10; ++a) {
+    void* p[11];
+    const size_t sz[11] = {nq, nq, nq, nq, ng, ng, ng, ng, 5 * ng, 5 * ng, solar::edge_cols_elems(n[m], nr[m])};
+    for (int a = 0; a < 11; ++a) {
       if ((rc = ens_alloc(e, &p[a], sz[a] * sizeof(double), &e->allocs))) return bail(rc);
       if (hipMemset(p[a], 0, sz[a] * sizeof(double)) != hipSuccess)
         return bail(solar::set_error(SOLAR_ERR_HIP, "solar_ens_create: hipMemset failed"));
     }
     M.q[0] = static_cast<double*>(p[0]);
     M.q[1] = static_cast<double*>(p[1]);
-    M.qw = static_cast<double*>(p[2]);
-    M.gxp = static_cast<double*>(p[3]);
-    M.gyp = static_cast<double*>(p[4]);
-    M.gxv = static_cast<double*>(p[5]);
-    M.gyv = static_cast<double*>(p[6]);
-    M.fgx = static_cast<double*>(p[7]);
-    M.fgy = static_cast<double*>(p[8]);
-    M.ecols = static_cast<double*>(p[9]);
+    M.qw[0] = static_cast<double*>(p[2]);
+    M.qw[1] = static_cast<double*>(p[3]);
+    M.gxp = static_cast<double*>(p[4]);
+    M.gyp = static_cast<double*>(p[5]);
+    M.gxv = static_cast<double*>(p[6]);
+    M.gyv = static_cast<double*>(p[7]);
+    M.fgx = static_cast<double*>(p[8]);
+    M.fgy = static_cast<double*>(p[9]);
+    M.ecols = static_cast<double*>(p[10]);
     M.dt = dt[m];
     e->choice[m] = default_choice(n[m], nr[m]);
   }
@@ -312,12 +319,17 @@ int solar_ens_create(solar_ens** out, int nmembers, const int* n, const int* nr,
     solar_ens::GatherGroup G;
     G.n = kv.first;
     G.nm = static_cast<int>(kv.second.size());
+    // about four blocks a CU: a block marches its planes one after the other,
+    // so a group of few members needs short chunks (eight members, two to four
+    // a group: 4 chunks 4.79 ms per step, 8 4.51, 16 4.41, 32 4.40), and one
+    // of many is fastest with long ones (48 members: 4 chunks)
+    G.chunks = e->gchunks > 0 ? e->gchunks : std::min(32, std::max(4, (1024 + 24 * G.nm - 1) / (24 * G.nm)));
     std::vector<int> table(2 * G.nm);
     for (int x = 0; x < G.nm; ++x) {
       const int m = kv.second[x];
       table[x] = G.nblocks;
       table[G.nm + x] = m;
-      G.nblocks += 24 * solar::gather_blocks_per_edge(nr[m], e->gchunks);
+      G.nblocks += 24 * solar::gather_blocks_per_edge(nr[m], G.chunks);
     }
     if ((rc = ens_alloc(e, &d, table.size() * sizeof(int), &e->allocs))) return bail(rc);
     G.table = static_cast<int*>(d);
@@ -381,7 +393,7 @@ int solar_ens_autotune(solar_ens* e, int reps) {
         if ((rc = make_launch(e, sh[0], sh[1], items, &L))) return rc;
         float ms = 0.f;
         if ((rc = time_launch(e, reps, [&]() {
-               return solar::launch_stage_ens(e->dmem, L.items, L.nitems, L.grid, L.ti, L.tj, 2, 0, e->stream);
+               return solar::launch_stage_ens(e->dmem, L.items, L.nitems, L.grid, L.ti, L.tj, 1, 0, 0, e->stream);
              }, &ms)))
           return rc;
         if (ms < best_s) {

@@ -323,7 +323,7 @@ struct StageArgs {
   S* ecols;
   const EnsMember* M;
   const int4* items;
-  int nitems, cur;
+  int nitems, cur, wcur;
 };
 
 // Flags of a stage instantiation beyond kStoreNoQ and kStageRecon.
@@ -347,7 +347,7 @@ constexpr int kStageWaves = 3;
 // tile, one barrier per plane.
 //   KIND 0: first stage (qw taken as 0, written), 1: middle stage (qw read and
 //   written), 2: last stage (qw read, not written back).
-//   FL: kStoreNoQ (FP64, single grid): the stage stores qw (in place) and the
+//   FL: kStoreNoQ (FP64): the stage stores qw (in place) and the
 //   edge columns of q, but not q itself.  kStageRecon (KIND 1): the stage
 //   input is qin + beta_r * qw, rebuilt wherever it is read (own point, halo
 //   cells, radial window) with the expression the previous stage rounded when
@@ -355,8 +355,9 @@ constexpr int kStageWaves = 3;
 //   other than qw (other blocks still read qw's halo cells).  kStageRhs,
 //   kStageAux: above.
 //   MODE 1: ensemble launch.  The block walks a list of work items (member,
-//   tile, panel, plane range) with a grid-sized stride; the state ping-pongs
-//   between M.q[cur] and M.q[1-cur].  MODE 2: tangent-linear stage (tl_dc2,
+//   tile, panel, plane range) with a grid-sized stride; q is read from
+//   M.q[cur] and stored to M.q[1-cur], qw is read from M.qw[wcur] and stored
+//   there or (kStageRecon) to M.qw[1-wcur].  MODE 2: tangent-linear stage (tl_dc2,
 //   tl_div used).
 //   ecols (optional; in an ensemble the member's): the stage also stores its
 //   output at the edge columns i = 1..3 and n-4..n-2 in the edge_cols layout,
@@ -395,7 +396,7 @@ void k_stage(StageArgs<S> A) {
   constexpr bool NOQ = (FL & kStoreNoQ) != 0, RECON = (FL & kStageRecon) != 0;
   constexpr bool RHS = (FL & kStageRhs) != 0, AUX = (FL & (kStageRhs | kStageAux)) != 0;
   constexpr bool ENS = MODE == 1, TL = MODE == 2, WIDE = sizeof(S) == 8;
-  static_assert(!(NOQ || RECON) || (MODE == 0 && WIDE), "the stored-q schedule variants are FP64, single grid");
+  static_assert(!(NOQ || RECON) || (MODE != 2 && WIDE), "the stored-q schedule variants are FP64, not tangent-linear");
   static_assert(!RECON || (KIND == 1 && !NOQ), "a rebuilt input is a middle stage's");
   static_assert(!NOQ || KIND != 2, "the last stage stores q");
   static_assert(!RHS || (KIND == 0 && MODE == 0 && !NOQ), "an RHS evaluation is of kind 0");
@@ -451,9 +452,9 @@ void k_stage(StageArgs<S> A) {
   const size_t ps = plane * sizeof(S), fs = nf * sizeof(S), pbase = (size_t)P * 5 * nf;
   const auto bytes = [](const void* p) { return (GlobalBytes)p; };
   const GlobalBytes qb = bytes((ENS ? reinterpret_cast<const S*>(E.q[A.cur]) : A.qin) + pbase);
-  const GlobalBytes wb = bytes((ENS ? reinterpret_cast<const S*>(E.qw) : A.qw) + pbase);
+  const GlobalBytes wb = bytes((ENS ? reinterpret_cast<const S*>(E.qw[A.wcur]) : A.qw) + pbase);
   const GlobalBytes ob = bytes((ENS ? reinterpret_cast<const S*>(E.q[1 - A.cur]) : A.qout) + pbase);
-  const GlobalBytes wob = RECON ? bytes(A.qwo + pbase) : wb;
+  const GlobalBytes wob = RECON ? bytes((ENS ? reinterpret_cast<const S*>(E.qw[1 - A.wcur]) : A.qwo) + pbase) : wb;
   // edge-column copy: layer l = i (W) or n-1-i (E); the others store none
   const int ecl = i <= 3 ? i : n - 1 - i;
   const S* const ecols = RHS ? nullptr : ENS ? reinterpret_cast<const S*>(E.ecols) : A.ecols;
@@ -1133,7 +1134,8 @@ __global__ __launch_bounds__(TI* TJ) __attribute__((amdgpu_waves_per_eu(6))) voi
 // in M); blockIdx.y selects the field.
 template <bool VEC, int NI>
 __global__ __launch_bounds__(gather_threads_max(NI)) void k_gather_ens(const EnsMember* __restrict__ M, const int* __restrict__ table,
-                                                     int nmem, int cur, int cols, int chunks) {
+                                                     int nmem, int cur, int cols, int chunks, int wcur,
+                                                     double betar) {
   extern __shared__ double sline[];
   const int b = blockIdx.x;
   int lo = 0, hi = nmem - 1;  // last member whose first block is <= b
@@ -1149,9 +1151,10 @@ __global__ __launch_bounds__(gather_threads_max(NI)) void k_gather_ens(const Ens
   const int k0 = (li / 24) * kc, edge = li % 24, k1 = min(k0 + kc, nr);
   const long long fs = 12LL * nr * E.T.n * 3;
   const double* ec = cols ? E.ecols : nullptr;
+  const double* qwr = VEC && wcur >= 0 ? E.qw[wcur] : nullptr;
   if (VEC)
     gather_edge<true, double, NI>(E.T, edge / 4, edge % 4, k0, k1, blockIdx.y, E.q[cur], ec, 4, E.gxp, E.gyp,
-                                  E.gxv, E.gyv, fs, sline, nullptr, 0.0);
+                                  E.gxv, E.gyv, fs, sline, qwr, betar);
   else
     gather_edge<false, double, NI>(E.T, edge / 4, edge % 4, k0, k1, blockIdx.y, E.q[cur], ec, 0, E.fgx, E.fgy,
                                    nullptr, nullptr, fs, sline, nullptr, 0.0);
@@ -1553,32 +1556,36 @@ hipError_t launch_place(const double* src, void* dst, bool f32, size_t nf, int d
 
 template <int TI, int TJ>
 static hipError_t launch_stage_ens_t(const EnsMember* M, const int4* items, int nitems, int grid, int stage, int cur,
-                                     hipStream_t st) {
+                                     int wcur, hipStream_t st) {
   StageArgs<double> a{};
   a.alpha = kAlphaRk4[stage];
   a.beta = kBetaRk4[stage];
+  a.beta_r = stage > 0 ? kBetaRk4[stage - 1] : 0.0;
   a.M = M;
   a.items = items;
   a.nitems = nitems;
   a.cur = cur;
+  a.wcur = wcur;
   const dim3 g(grid), block(TI, TJ);
   if (stage == 0)
-    hipLaunchKernelGGL((k_stage<TI, TJ, 0, double, 1>), g, block, 0, st, a);
+    hipLaunchKernelGGL((k_stage<TI, TJ, 0, double, 1, false, kStoreNoQ>), g, block, 0, st, a);
+  else if (stage == 2)
+    hipLaunchKernelGGL((k_stage<TI, TJ, 1, double, 1, false, kStoreNoQ>), g, block, 0, st, a);
   else if (stage < 4)
-    hipLaunchKernelGGL((k_stage<TI, TJ, 1, double, 1>), g, block, 0, st, a);
+    hipLaunchKernelGGL((k_stage<TI, TJ, 1, double, 1, false, kStageRecon>), g, block, 0, st, a);
   else
     hipLaunchKernelGGL((k_stage<TI, TJ, 2, double, 1>), g, block, 0, st, a);
   return hipGetLastError();
 }
 
 hipError_t launch_stage_ens(const EnsMember* M, const int* items, int nitems, int grid, int ti, int tj, int stage,
-                            int cur, hipStream_t st) {
+                            int cur, int wcur, hipStream_t st) {
   const int4* it = reinterpret_cast<const int4*>(items);
   if (nitems <= 0) return hipSuccess;
   if (stage < 0 || stage > 4) return hipErrorInvalidValue;
-  if (ti == 64 && tj == 8) return launch_stage_ens_t<64, 8>(M, it, nitems, grid, stage, cur, st);
-  if (ti == 32 && tj == 8) return launch_stage_ens_t<32, 8>(M, it, nitems, grid, stage, cur, st);
-  if (ti == 16 && tj == 16) return launch_stage_ens_t<16, 16>(M, it, nitems, grid, stage, cur, st);
+  if (ti == 64 && tj == 8) return launch_stage_ens_t<64, 8>(M, it, nitems, grid, stage, cur, wcur, st);
+  if (ti == 32 && tj == 8) return launch_stage_ens_t<32, 8>(M, it, nitems, grid, stage, cur, wcur, st);
+  if (ti == 16 && tj == 16) return launch_stage_ens_t<16, 16>(M, it, nitems, grid, stage, cur, wcur, st);
   return hipErrorInvalidValue;
 }
 
@@ -1599,26 +1606,26 @@ hipError_t launch_filter_ens(const EnsMember* M, const int* items, int nitems, i
 
 template <bool VEC, int NI>
 static hipError_t launch_gather_ens_v(const EnsMember* M, const int* table, int nmem, int nblocks, int maxn, int cur,
-                                      int cols, int chunks, hipStream_t st) {
+                                      int cols, int chunks, hipStream_t st, int wcur, double betar) {
   const int nt = gather_threads(maxn, NI);
   const size_t lds = sizeof(double) * 2 * 3 * (VEC ? 3 : 1) * (size_t)maxn;
   hipError_t e = gather_lds(&k_gather_ens<VEC, NI>, lds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((k_gather_ens<VEC, NI>), dim3(nblocks, VEC ? 1 : 5), dim3(nt), lds, st, M, table, nmem, cur,
-                     cols, chunks);
+                     cols, chunks, wcur, betar);
   return hipGetLastError();
 }
 
 hipError_t launch_gather_ens(const EnsMember* M, const int* table, int nmem, int nblocks, int maxn, bool vec, int cur,
-                             bool cols, int chunks, hipStream_t st) {
+                             bool cols, int chunks, hipStream_t st, int wcur, double betar) {
   const bool two = 3 * maxn > 1024;  // n > 341: two strip points per thread
   const int c = cols ? 1 : 0;
   if (chunks < 1) return hipErrorInvalidValue;
   if (vec)
-    return two ? launch_gather_ens_v<true, 2>(M, table, nmem, nblocks, maxn, cur, c, chunks, st)
-               : launch_gather_ens_v<true, 1>(M, table, nmem, nblocks, maxn, cur, c, chunks, st);
-  return two ? launch_gather_ens_v<false, 2>(M, table, nmem, nblocks, maxn, cur, c, chunks, st)
-             : launch_gather_ens_v<false, 1>(M, table, nmem, nblocks, maxn, cur, c, chunks, st);
+    return two ? launch_gather_ens_v<true, 2>(M, table, nmem, nblocks, maxn, cur, c, chunks, st, wcur, betar)
+               : launch_gather_ens_v<true, 1>(M, table, nmem, nblocks, maxn, cur, c, chunks, st, wcur, betar);
+  return two ? launch_gather_ens_v<false, 2>(M, table, nmem, nblocks, maxn, cur, c, chunks, st, wcur, betar)
+             : launch_gather_ens_v<false, 1>(M, table, nmem, nblocks, maxn, cur, c, chunks, st, wcur, betar);
 }
 
 }  // namespace solar

@@ -30,13 +30,13 @@ struct DevTables {
 };
 
 // One member of a batched ensemble (FP64): its tables, state ping-pong
-// buffers, 2N accumulator, ghost strips, edge-column copies (written by
+// buffers, the two 2N accumulators of the stored-q schedule, ghost strips, edge-column copies (written by
 // every stage, read by the next gather, edge_cols_elems(n, nr) values) and
 // time step.
 struct EnsMember {
   DevTables T;
   double* q[2];
-  double* qw;
+  double* qw[2];
   double *gxp, *gyp, *gxv, *gyv;
   double *fgx, *fgy;
   double* ecols;
@@ -89,9 +89,12 @@ hipError_t launch_filter(const DevTables& T, const void* qin, void* qout, bool f
 // Ensemble launches.  items: 4 ints per work item, (member, bi | bj << 16,
 // P (stage) or 5P+F (filter) | k0 << 8, k1); grid blocks walk the list with a
 // grid-sized stride.  Stage ti x tj in {64x8, 32x8, 16x16}, filter in
-// {32x16, 16x16, 32x8}.  The state goes from M.q[cur] to M.q[1-cur].
+// {32x16, 16x16, 32x8}.  The state goes from M.q[cur] to M.q[1-cur].  The
+// stages run the stored-q schedule (kStoreNoQ for stages 0 and 2, kStageRecon
+// for 1 and 3): qw is read from M.qw[wcur], and a rebuilding stage writes its
+// own to M.qw[1-wcur].
 hipError_t launch_stage_ens(const EnsMember* M, const int* items, int nitems, int grid, int ti, int tj, int stage,
-                            int cur, hipStream_t st);
+                            int cur, int wcur, hipStream_t st);
 hipError_t launch_filter_ens(const EnsMember* M, const int* items, int nitems, int grid, int ti, int tj, int cur,
                              hipStream_t st);
 // A gather over a group of members: table[x] = first block of the group's
@@ -100,9 +103,10 @@ hipError_t launch_filter_ens(const EnsMember* M, const int* items, int nitems, i
 // (block size and LDS).  vec:
 // the stage ghosts (p', velocity), else the filter's five scalars.  cols:
 // the W/E column strips come from the members' edge-column copies (every
-// gather but the first of a step, whose source no stage wrote).
+// gather but the first of a step, whose source no stage wrote).  wcur >= 0
+// (vec): the source is q + betar * M.qw[wcur], a rebuilding stage's input.
 hipError_t launch_gather_ens(const EnsMember* M, const int* table, int nmem, int nblocks, int maxn, bool vec, int cur,
-                             bool cols, int chunks, hipStream_t st);
+                             bool cols, int chunks, hipStream_t st, int wcur = -1, double betar = 0.0);
 // Planes per gather block (about 32 chunks per receiver edge), and gather
 // blocks per receiver edge.
 constexpr int gather_kc(int nr, int chunks = 32) { return (nr + chunks - 1) / chunks; }
