@@ -811,23 +811,28 @@ struct FilterLds {
 // The tile (bi, bj) of field F of panel P (PF = 5P + F) over planes [k0, k1).
 // PART: the tile may reach past the panel edge; threads past it store nothing,
 // and tile cells beyond the panel's three ghost layers stay 0.
-// PAIR: FILTER_XI tasks of two adjacent outputs (below).
-template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4)>
+// PAIR: FILTER_XI tasks of two adjacent outputs (below).  R: adjacent rows
+// per thread (blocks of TI x TJ / R), whose FILTER_ETA sums share R + 6 reads
+// where single rows take 7 each.
+template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4), int R = 1>
 __device__ __forceinline__ void filter_tile(const DevTables& T, int bi, int bj, int PF, int k0, int k1,
                                             const S* __restrict__ qin, S* __restrict__ qout,
                                             const double* __restrict__ fgx, const double* __restrict__ fgy,
                                             FilterLds<TI, TJ>& lds) {
-  constexpr int NT = TI * TJ;
+  constexpr int NT = TI * TJ / R;
   constexpr int NCELL = (TJ + 6) * (TI + 6);
   constexpr int NC = (NCELL + NT - 1) / NT;
+  static_assert(R == 1 || PAIR, "several rows per thread: paired FILTER_XI tasks");
   auto& sq = lds.sq;
   auto& sx = lds.sx;
   const int n = T.n, nr = T.nr;
   const int P = PF / 5, F = PF % 5;
-  const int tx = threadIdx.x, ty = threadIdx.y;
+  const int tx = threadIdx.x, ty = threadIdx.y * R;  // this thread's first row
   const int i0 = bi * TI, j0 = bj * TJ;
   const int i = i0 + tx, j = j0 + ty;
-  const bool own_in = !PART || (i < n && j < n);
+  bool own_in[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) own_in[r] = !PART || (i < n && j + r < n);
 
   const size_t plane = (size_t)n * n, nf = plane * nr;
   const S* g = qin + (size_t)PF * nf;
@@ -836,14 +841,17 @@ __device__ __forceinline__ void filter_tile(const DevTables& T, int bi, int bj, 
   const size_t fstride = (size_t)12 * gx_side;
   const double* gxW = fgx + F * fstride + (size_t)(P * 2) * gx_side;
   const double* gyS = fgy + F * fstride + (size_t)(P * 2) * gy_side;
-  const size_t ij = own_in ? (size_t)j * n + i : 0;
+  const size_t ij = own_in[0] ? (size_t)j * n + i : 0;
 
   // 2-D case (nr == 1): FILTER_R returns its input (filter.f90:647-650)
   const bool twod = nr == 1;
   // filter.f90:652,726-777: the five planes at each end are zero.
-  if (own_in && !twod)
+  if (!twod)
     for (int k = k0; k < k1; ++k)
-      if (k < kNstr || k >= nr - kNstr) o[(size_t)k * plane + ij] = static_cast<S>(0.0);
+      if (k < kNstr || k >= nr - kNstr)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          if (own_in[r]) o[(size_t)k * plane + ij + (size_t)r * n] = static_cast<S>(0.0);
   const int a = twod ? 0 : max(k0, kNstr), bnd = twod ? 1 : min(k1, nr - kNstr);
   if (a >= bnd) return;
 
@@ -856,7 +864,7 @@ __device__ __forceinline__ void filter_tile(const DevTables& T, int bi, int bj, 
   // a ghost cell the strip's first element.  Kind-0 cells (the corners beyond
   // the panel in both directions, cells past a partial tile's ghost layers)
   // feed only outputs that are not stored, so they keep whatever was loaded.
-  const int tid = ty * TI + tx;
+  const int tid = threadIdx.y * TI + tx;
   unsigned foff[NC];
   const double* gp[NC];
   int kind[NC];
@@ -1014,10 +1022,13 @@ __device__ __forceinline__ void filter_tile(const DevTables& T, int bi, int bj, 
     __syncthreads();
     xi_pass();
     __syncthreads();
-    double v = 0.0;  // stored: the reference's sum from 0.0
 #pragma unroll
-    for (int q = 0; q < 7; ++q) v = v + T.filt[q] * sx[ty + q][tx];
-    if (own_in) o[ij] = static_cast<S>(v);
+    for (int r = 0; r < R; ++r) {
+      double v = 0.0;  // stored: the reference's sum from 0.0
+#pragma unroll
+      for (int q = 0; q < 7; ++q) v = v + T.filt[q] * sx[ty + r + q][tx];
+      if (own_in[r]) o[ij + (size_t)r * n] = static_cast<S>(v);
+    }
     return;
   }
 
@@ -1028,9 +1039,11 @@ __device__ __forceinline__ void filter_tile(const DevTables& T, int bi, int bj, 
   // pending outputs: acc[d] is output plane kk - 5 + d, which takes the term
   // q = 10 - d of plane kk, the same order and the same products as the
   // sum over a window of the last eleven planes with 6 multiplies instead of 11.
-  double acc[11];
+  double acc[R][11];
 #pragma unroll
-  for (int q = 0; q < 11; ++q) acc[q] = 0.0;
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int q = 0; q < 11; ++q) acc[r][q] = 0.0;
 
   const int kbeg = a - kNstr, kend = bnd + kNstr;  // kend - kbeg >= 11
   // store: the step completes an output plane (every step from the 11th on)
@@ -1046,20 +1059,26 @@ __device__ __forceinline__ void filter_tile(const DevTables& T, int bi, int bj, 
     __syncthreads();
     // FILTER_ETA (filter.f90:448-629), from the first product, as FILTER_XI:
     // FILTER_R's sum from 0.0 does not see the sign of a zero input.
-    double v = T.filt[0] * sx[ty][tx];
+    double e[R + 6];  // the column's R + 6 rows
 #pragma unroll
-    for (int q = 1; q < 7; ++q) v = v + T.filt[q] * sx[ty + q][tx];
-    double pr[6];
+    for (int q = 0; q < R + 6; ++q) e[q] = sx[ty + q][tx];
 #pragma unroll
-    for (int m = 0; m < 6; ++m) pr[m] = T.filtr[m] * v;
+    for (int r = 0; r < R; ++r) {
+      double v = T.filt[0] * e[r];
 #pragma unroll
-    for (int d = 0; d < 10; ++d) acc[d] = acc[d] + pr[d < 6 ? d : 10 - d];
-    acc[10] = 0.0 + pr[0];
-    if constexpr (decltype(store)::value) {
-      if (own_in) o[(size_t)(kk - kNstr) * plane + ij] = static_cast<S>(acc[0]);
+      for (int q = 1; q < 7; ++q) v = v + T.filt[q] * e[r + q];
+      double pr[6];
+#pragma unroll
+      for (int m = 0; m < 6; ++m) pr[m] = T.filtr[m] * v;
+#pragma unroll
+      for (int d = 0; d < 10; ++d) acc[r][d] = acc[r][d] + pr[d < 6 ? d : 10 - d];
+      acc[r][10] = 0.0 + pr[0];
+      if constexpr (decltype(store)::value) {
+        if (own_in[r]) o[(size_t)(kk - kNstr) * plane + ij + (size_t)r * n] = static_cast<S>(acc[r][0]);
+      }
+#pragma unroll
+      for (int d = 0; d < 10; ++d) acc[r][d] = acc[r][d + 1];
     }
-#pragma unroll
-    for (int d = 0; d < 10; ++d) acc[d] = acc[d + 1];
   };
   // Branch-free memory traffic per iteration (a fixed warm-up, then pairs of
   // storing steps, then at most one more), so the waits before each LDS
@@ -1086,11 +1105,13 @@ __device__ __forceinline__ void filter_tile(const DevTables& T, int bi, int bj, 
 // runs five waves, two blocks per CU, which leaves the barriers of each
 // plane less to overlap with; at 80 it does not spill (the 32x16 and 16x16
 // tiles; the other shapes spill 36 bytes and keep no floor).
-template <int TI, int TJ, typename S>
-constexpr int filter_waves() { return (sizeof(S) == 4 && TI * TJ >= 256 && !(TI == 64 && TJ == 4) && !(TI == 32 && TJ == 8)) ? 6 : 1; }
+// Two rows per thread take 118 registers: four waves (five spill and take
+// three times as long).
+template <int TI, int TJ, typename S, int R>
+constexpr int filter_waves() { return R > 1 ? 4 : (sizeof(S) == 4 && TI * TJ >= 256 && !(TI == 64 && TJ == 4) && !(TI == 32 && TJ == 8)) ? 6 : 1; }
 
-template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4)>
-__global__ __launch_bounds__(TI* TJ) __attribute__((amdgpu_waves_per_eu(filter_waves<TI, TJ, S>())))
+template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4), int R = 1>
+__global__ __launch_bounds__(TI* TJ / R) __attribute__((amdgpu_waves_per_eu(filter_waves<TI, TJ, S, R>())))
 void k_filter(DevTables T, const S* __restrict__ qin,
                                                     S* __restrict__ qout, const double* __restrict__ fgx,
                                                     const double* __restrict__ fgy, int kchunk, int nkch) {
@@ -1108,7 +1129,7 @@ void k_filter(DevTables T, const S* __restrict__ qin,
   const int k0 = ch * kchunk;
   const int k1 = min(k0 + kchunk, nr);
   if (k0 >= nr) return;
-  filter_tile<TI, TJ, S, PART, PAIR>(T, bi, bj, PF, k0, k1, qin, qout, fgx, fgy, lds);
+  filter_tile<TI, TJ, S, PART, PAIR, R>(T, bi, bj, PF, k0, k1, qin, qout, fgx, fgy, lds);
 }
 
 // Ensemble FILTER_EXP: work items (member, tile, 5P+F, plane range), q[cur] -> q[1-cur].
@@ -1470,22 +1491,22 @@ hipError_t launch_stage(const DevTables& T, const void* qin, void* qout, void* q
   return f32 ? go(stage_args<float>(T, qin, qout, qw, qwo, ecols)) : go(stage_args<double>(T, qin, qout, qw, qwo, ecols));
 }
 
-template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4)>
+template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4), int R = 1>
 static hipError_t launch_filter_t(const DevTables& T, const S* qin, S* qout, const double* fgx, const double* fgy,
                                   hipStream_t st, const LaunchShape& ls) {
   const int tiles = ((T.n + TI - 1) / TI) * ((T.n + TJ - 1) / TJ) * 30;
   // radial chunks of >= 64 planes (each re-reads 10 halo planes), ~4k blocks: a single chunk per
   // column at 6x256^2x384 leaves a long tail (3.45 ms against 2.96 ms with two)
-  int nkch = chunks_for(tiles, T.nr, 4096, 64);
+  int nkch = R > 1 ? small_grid_chunks(tiles, T.nr, 2.0 * kNstr, 2, 1.5) : chunks_for(tiles, T.nr, 4096, 64);
   // a chunk re-reads ten planes, so a small grid is split less far than the
   // stages (us, before -> after: 6x16^2x96 55 -> 16, 6x32^2x64 48 -> 25,
   // 6x48^2x100 66 -> 44; from 1620 blocks on, 6x96^2x192, all splits into
   // 32 to 96 planes measured within 2%)
-  if (tiles * nkch < 1536) nkch = small_grid_chunks(tiles, T.nr, 2.0 * kNstr, 1, 1.5);
+  if (R == 1 && tiles * nkch < 1536) nkch = small_grid_chunks(tiles, T.nr, 2.0 * kNstr, 1, 1.5);
   if (ls.filter_chunks > 0) nkch = ls.filter_chunks;
   const int kchunk = (T.nr + nkch - 1) / nkch;
-  dim3 grid(tiles * nkch), block(TI, TJ);
-  hipLaunchKernelGGL((k_filter<TI, TJ, S, PART, PAIR>), grid, block, 0, st, T, qin, qout, fgx, fgy, kchunk, nkch);
+  dim3 grid(tiles * nkch), block(TI, TJ / R);
+  hipLaunchKernelGGL((k_filter<TI, TJ, S, PART, PAIR, R>), grid, block, 0, st, T, qin, qout, fgx, fgy, kchunk, nkch);
   return hipGetLastError();
 }
 
@@ -1502,6 +1523,16 @@ static hipError_t launch_filter_s(const DevTables& T, const S* qin, S* qout, con
                 : launch_filter_t<16, 16, S, true, false>(T, qin, qout, fgx, fgy, st, ls);
   }
   int ti = ls.filter_ti, tj = ls.filter_tj;
+  // FP64 on panels from 128: 64x16 tiles with two rows a thread.  Fewer halo
+  // cells (1.50 tile cells a point against 1.63, and whole lines of them) and
+  // LDS reads: 6x256^2x384 2.94 -> 2.58 ms, 6x128^2x256 489 -> 456 us.  The
+  // FP32-state filter is bound by its FP64 arithmetic instead and keeps one
+  // row (6x256^2x384 2.28 against 2.40 ms); so do smaller panels (6x64^2x128
+  // 73.2 against 72.2 us).
+  if constexpr (sizeof(S) == 8) {
+    if (T.n % 64 == 0 && T.n >= 128 && !fits(T.n, ti, tj))
+      return launch_filter_t<64, 16, S, false, true, 2>(T, qin, qout, fgx, fgy, st, ls);
+  }
   if (!fits(T.n, ti, tj)) {  // measured best: 32x16 (n%32==0), 16x16
     ti = T.n % 32 == 0 ? 32 : 16;
     tj = 16;
