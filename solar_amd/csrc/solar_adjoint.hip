@@ -41,6 +41,11 @@
 
 namespace solar {
 
+// Occupancy floor of the adjoint stage in waves per SIMD: it takes 186 to 204
+// registers; at three waves it spills 60 to 136 bytes a lane (gradient
+// 6x96^2x192 212 -> 255 ms).
+constexpr int kAdjWaves = 2;
+
 namespace {
 
 __device__ __forceinline__ int strip_index_a(int e, int l, int a, int n) {
@@ -101,25 +106,37 @@ __device__ __forceinline__ void adj_radial(const Row& row, bool bc, double c2rho
 
 }  // namespace
 
-// One reverse RK stage of the adjoint (or L^T alone in RHS mode).
+// One reverse RK stage of the adjoint (or L^T alone, kAdjRhs).
 //   W    : W^(s) = the adjoint of the stage's 2N accumulator (5 fields)
 //   Yin  : Ybar^(s) (5 fields); Yout = Ybar^(s-1) = Yin + dt L^T W (may alias Yin)
-//   Wout : W^(s-1) = alpha*W + beta*Yout when mode & kAdjWriteW
-//   divs : div(v) of the forward stage input, for the gradient (mode & kAdjGrad)
+//   Wout : W^(s-1) = alpha*W + beta*Yout when write_w
+//   divs : div(v) of the forward stage input, for the gradient
 //   gc2  : c^2 gradient accumulator (n,n,nr,6)
 //   gxa_*, gya_* : dt-scaled ghost adjoints written by edge tiles
-// In RHS mode (mode & kAdjRhsOnly) Yout = L^T W and dt must be 1.
-// D32: divs holds FP32 divergences (a template parameter, so the plane
-// prefetch holds a single load path).
-template <int TI, int TJ, bool D32>
-__global__ __launch_bounds__(TI* TJ) void k_adj_stage(DevTables T, const double* __restrict__ W,
-                                                       const double* Yin, double* Yout,  // may alias
-                                                       double* __restrict__ Wout, const double* __restrict__ divs,
-                                                       double* __restrict__ gc2, const double* __restrict__ c2f,
-                                                       double* __restrict__ gxa_p, double* __restrict__ gya_p,
-                                                       double* __restrict__ gxa_v, double* __restrict__ gya_v,
-                                                       double dt, double alpha, double beta, double wscale,
-                                                       int kchunk, int nkch, int mode) {
+// KIND: kAdjStep, kAdjGrad64 or kAdjGrad32 (with the gradient, from FP64 or
+// FP32 divergences), kAdjRhs (Yout = L^T W; dt must be 1).
+//
+// Bound by memory where the grid fills the chip (6x96^2x192, mean of a step's
+// five: 170 bytes a point at 4.5 TB/s, where a march of as many streams with
+// no arithmetic reaches 4.8 to 5.0), by the instructions of its serial plane
+// chain on small grids.  As in the forward stage, addresses
+// are a uniform base plus a lane offset, one thread loads one halo cell (y
+// halos by the first waves), and a plane's loads come in two groups: W, the
+// halo cells and the plane entering the radial window, consumed at its start
+// and loaded again before the barrier; Ybar, div(v) and the c^2 gradient,
+// needed at its end and loaded at the end of the plane before.  Against one
+// prefetched copy of a whole plane: 595 -> 462 vector instructions a plane,
+// 240 -> 204 registers, 6x96^2x192 431 -> 403 us, 6x48^2x100 71 -> 66 us.
+constexpr int kAdjStep = 0, kAdjGrad64 = 1, kAdjGrad32 = 2, kAdjRhs = 3;
+
+template <int TI, int TJ, int KIND>
+__global__ __launch_bounds__(TI* TJ) __attribute__((amdgpu_waves_per_eu(kAdjWaves))) void k_adj_stage(
+    DevTables T, const double* __restrict__ W, const double* Yin, double* Yout,  // may alias
+    double* __restrict__ Wout, const double* __restrict__ divs, double* __restrict__ gc2,
+    const double* __restrict__ c2f, double* __restrict__ gxa_p, double* __restrict__ gya_p,
+    double* __restrict__ gxa_v, double* __restrict__ gya_v, double dt, double alpha, double beta, double wscale,
+    int kchunk, int nkch, int write_w) {
+  constexpr bool RHS = KIND == kAdjRhs, GRAD = KIND == kAdjGrad64 || KIND == kAdjGrad32, D32 = KIND == kAdjGrad32;
   // Transposed-stencil inputs with i halos (x) and j halos (y); two buffers
   // alternating by plane, so one barrier per plane suffices.
   __shared__ double sxv[2][TJ][TI + 6], sxp[2][TJ][TI + 6];
@@ -127,9 +144,10 @@ __global__ __launch_bounds__(TI* TJ) void k_adj_stage(DevTables T, const double*
   // DRP taps for the edge tiles' ghost adjoints, which index them per
   // thread: from LDS, a dynamic index into the kernel argument would be a
   // vector load that the plane loop waits on together with the prefetch
-  __shared__ double sfc[2][7];
-  constexpr int NT = TI * TJ, NHX = 6 * TJ, NH = 6 * TJ + 6 * TI;
-  static_assert(NH <= NT, "one halo cell per thread at most");
+  __shared__ double sfc[7];
+  // halo cells: 6 rows of TI (y), then TJ rows of 6 (x) from a wave boundary on
+  constexpr int NT = TI * TJ, HY = (6 * TI + 63) / 64 * 64;
+  static_assert(HY + 6 * TJ <= NT, "one halo cell per thread at most");
 
   const int n = T.n, nr = T.nr;
   const int nti = n / TI, ntj = n / TJ;
@@ -141,20 +159,24 @@ __global__ __launch_bounds__(TI* TJ) void k_adj_stage(DevTables T, const double*
   const int P = b % 6;
   const int ch = b / 6;
   const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * TI + tx;
+  const bool hx = __builtin_amdgcn_readfirstlane(tid & ~63) >= HY;  // this wave's halo cells: x or y
   const int i0 = bi * TI, j0 = bj * TJ;
   const int i = i0 + tx, j = j0 + ty;
   const int k0 = ch * kchunk;
   const int k1 = min(k0 + kchunk, nr);
   if (k0 >= nr) return;
 
-  const size_t plane = (size_t)n * n, nf = plane * nr;
-  const size_t ij = (size_t)j * n + i;
+  const size_t plane = (size_t)n * n, nf = plane * nr, ps = plane * sizeof(double), fs = nf * sizeof(double);
+  const unsigned cell = (unsigned)(j * n + i), off = cell * 8u;
+  const auto bytes = [](const void* p) { return (GlobalBytes)p; };
   // W^(s), or wscale * Ybar when the stage starts from Ybar alone (W == nullptr)
-  const double* w0 = (W ? W : Yin) + (size_t)(P * 5) * nf;
+  const GlobalBytes wb = bytes((W ? W : Yin) + (size_t)(P * 5) * nf);
+  const GlobalBytes yb = bytes(RHS ? W : Yin + (size_t)(P * 5) * nf);
+  const GlobalBytes yob = bytes(Yout + (size_t)(P * 5) * nf), wob = bytes(Wout + (size_t)(P * 5) * nf);
+  const GlobalBytes c2b = bytes(c2f + (size_t)P * nf);  // read only with c2f
   const double ws = W ? 1.0 : wscale;
   const CRadialRows rows = const_rows(T.rad);
   auto c2rho0_of = [&](const auto& row, double c2) { return c2f ? c2 * row.rho0 : row.c2rho0; };
-  auto c2_at = [&](int k, size_t cell) { return c2f ? c2f[(size_t)P * nf + (size_t)k * plane + cell] : 0.0; };
 
   // Radial inputs (u_rv, u_rp) of plane k at this column, loaded on demand
   // (the window fill and the closure planes).
@@ -164,109 +186,109 @@ __global__ __launch_bounds__(TI* TJ) void k_adj_stage(DevTables T, const double*
       up = 0.0;
       return;
     }
-    const size_t c = (size_t)k * plane + ij;
-    adj_radial(rows[k], k == 0 || k == nr - 1, c2rho0_of(rows[k], c2_at(k, ij)), ws * w0[c], ws * w0[3 * nf + c],
-               ws * w0[4 * nf + c], uv, up);
+    const size_t kp = (size_t)k * ps;
+    const unsigned o = lane_offset(off);
+    const double c2 = c2f ? load_at<double>(c2b + kp, o) : 0.0;
+    adj_radial(rows[k], k == 0 || k == nr - 1, c2rho0_of(rows[k], c2), ws * load_at<double>(wb + kp, o),
+               ws * load_at<double>(wb + kp + 3 * fs, o), ws * load_at<double>(wb + kp + 4 * fs, o), uv, up);
   };
+
+  // The halo cell this thread fills (at most one): its LDS cell, and its offset
+  // in a field plane.  Beyond the panel edge the transposed stencil reads 0.
+  int hrow, hcol, hi, hj;
+  bool has_h;
+  if (hx) {
+    const int c6 = (tid - HY) % 6;
+    hrow = (tid - HY) / 6;
+    has_h = hrow < TJ;
+    hcol = c6 < 3 ? c6 : TI + c6;
+    hi = i0 - 3 + hcol;
+    hj = j0 + hrow;
+  } else {
+    const int r6 = tid / TI;
+    has_h = r6 < 6;
+    hcol = tid % TI;
+    hrow = r6 < 3 ? r6 : TJ + r6;
+    hi = i0 + hcol;
+    hj = j0 - 3 + hrow;
+  }
+  const bool h_in = has_h && hi >= 0 && hi < n && hj >= 0 && hj < n;
+  const unsigned hcell = h_in ? (unsigned)(hj * n + hi) : 0u, hoff = hcell * 8u;
+
+  // What a plane's start needs, loaded a plane ahead: W at the own point, the
+  // halo cell and the plane entering the radial window (k+3 for plane k), and
+  // c^2 there with c2f.
+  double w_n[5], hw[4], rw[3], c2o = 0.0, c2h = 0.0, c2r = 0.0;
+  auto load_start = [&](int k) {
+    const size_t kp = (size_t)k * ps, ke = (size_t)min(k + 3, nr - 1) * ps;
+    const unsigned o = lane_offset(off), h = lane_offset(hoff);
+    rw[0] = load_at<double>(wb + ke, o);
+    rw[1] = load_at<double>(wb + ke + 3 * fs, o);
+    rw[2] = load_at<double>(wb + ke + 4 * fs, o);
+#pragma unroll
+    for (int f = 0; f < 5; ++f) w_n[f] = load_at<double>(wb + kp + f * fs, o);
+    hw[0] = load_at<double>(wb + kp, h);
+    hw[1] = load_at<double>(wb + kp + fs, h);
+    hw[2] = load_at<double>(wb + kp + 2 * fs, h);
+    hw[3] = load_at<double>(wb + kp + 4 * fs, h);
+    if (c2f) {
+      c2o = load_at<double>(c2b + kp, o);
+      c2h = load_at<double>(c2b + kp, h);
+      c2r = load_at<double>(c2b + ke, o);
+    }
+  };
+  // What its end needs.
+  double y_n[5] = {}, g_n = 0.0, dv_n = 0.0;
+  float dvf_n = 0.f;  // D32: as loaded (a conversion at the load would wait for it)
+  auto load_update = [&](int k) {
+    const size_t kp = (size_t)k * ps;
+    const unsigned o = lane_offset(off);
+    if constexpr (!RHS) {
+#pragma unroll
+      for (int f = 0; f < 5; ++f) y_n[f] = load_at_nt<double>(yb + kp + f * fs, o);
+    }
+    if constexpr (GRAD) {
+      const size_t gk = (size_t)P * nf + (size_t)k * plane;
+      g_n = load_at<double>(bytes(gc2) + gk * 8, o);
+      if constexpr (D32)
+        dvf_n = load_at_nt<float>(bytes(divs) + gk * 4, lane_offset(cell * 4u));
+      else
+        dv_n = load_at_nt<double>(bytes(divs) + gk * 8, o);
+    }
+  };
+
+  load_start(k0);
   // Radial window over planes k-3..k+3.
   double rv[7], rp[7];
 #pragma unroll
   for (int q = 0; q < 7; ++q) radial_u(k0 - 3 + q, rv[q], rp[q]);
-
-  // The halo cell this thread fills (at most one per thread when NH <= NT):
-  // x halos first (TJ rows x 6 columns), then y halos (6 rows x TI columns).
-  // hcell < 0: beyond the panel edge, where the transposed stencil reads 0.
-  const bool has_h = tid < NH;
-  bool hx = false;
-  int hrow = 0, hcol = 0, hi_ = 0, hj_ = 0;
-  if (has_h) {
-    if (tid < NHX) {
-      hx = true;
-      hrow = tid / 6;
-      const int c6 = tid % 6;
-      hcol = c6 < 3 ? c6 : TI + c6;
-      hi_ = i0 - 3 + hcol;
-      hj_ = j0 + hrow;
-    } else {
-      const int h = tid - NHX;
-      const int r6 = h / TI;
-      hcol = h % TI;
-      hrow = r6 < 3 ? r6 : TJ + r6;
-      hi_ = i0 + hcol;
-      hj_ = j0 - 3 + hrow;
-    }
-  }
-  const bool h_in = has_h && hi_ >= 0 && hi_ < n && hj_ >= 0 && hj_ < n;
-  const size_t hcell = h_in ? (size_t)hj_ * n + hi_ : 0;
-
   // Loop-invariant metric of the own point and, for the halo cell, the three
   // factors its one transposed-stencil input needs: x halos take
   // (dc/C, D, XY/C) for u_xv, u_xp; y halos (dc/D, XY/D, C) for u_yv, u_yp.
-  const double Ci = T.ci[i], Dj = T.dj[j];
-  const double4 mq = *reinterpret_cast<const double4*>(T.adj_metric + ij * 4);
-  const double tdx = T.tdx[ij], tde = T.tde[ij];
-  double hA = 0.0, hB = 0.0, hC = 0.0;
-  if (h_in) {
-    const double4 hm = *reinterpret_cast<const double4*>(T.adj_metric + hcell * 4);
-    hA = hx ? hm.x : hm.y;
-    hB = hx ? T.dj[hj_] : hm.w;
-    hC = hx ? hm.z : T.ci[hi_];
-  }
-
-  const double sig_dt = (mode & kAdjRhsOnly) ? 1.0 : dt;
-  const size_t gx_side = (size_t)nr * n * 3, gy_side = (size_t)nr * 3 * n;
-
-  // W values of one plane, loaded a plane ahead: own point, halo cell, and
-  // the plane entering the radial window (k+3 for plane k); Ybar, div(v), the
-  // c^2 gradient and c^2 come with them.  Every load is issued whatever the
-  // mode (unused inputs read a fixed in-bounds address), so no branch sits
-  // between the loads and the waits before their use count exactly what is
-  // still in flight.
-  const bool upd = !(mode & kAdjRhsOnly), grad = (mode & kAdjGrad) != 0;
-  const double* yi = upd ? Yin + (size_t)(P * 5) * nf : w0;
-  const double* dvb = grad ? divs : w0;
-  const double* gcb = grad ? gc2 : w0;
-  const double* c2b = c2f ? c2f + (size_t)P * nf : w0;
-  struct AdjPlane {
-    double w[5], hw[4], rw[3], y[5], dv, g, c2o, c2h, c2r;
-    float dvf;  // D32: the divergence as loaded, widened where it is used (a conversion at
-                // the load would wait on every load in flight)
-  };
-  auto load_plane = [&](int k, AdjPlane& L) {
-    const size_t x = (size_t)k * plane + ij;
+  double Ci = T.ci[i], Dj = T.dj[j];
+  double4 mq = *reinterpret_cast<const double4*>(T.adj_metric + (size_t)cell * 4);
+  double tdx = T.tdx[cell], tde = T.tde[cell];
+  const double4 hm = *reinterpret_cast<const double4*>(T.adj_metric + (size_t)hcell * 4);
+  double hA = hx ? hm.x : hm.y;
+  double hB = hx ? T.dj[h_in ? hj : 0] : hm.w;
+  double hC = hx ? hm.z : T.ci[h_in ? hi : 0];
+  if (threadIdx.y == 0 && threadIdx.x < 7) sfc[threadIdx.x] = T.fcx[threadIdx.x];  // read after the first barrier
+  // Everything loaded so far arrives before the loop, so that the waits inside
+  // it are those of its own loads.
+  asm volatile("" : "+v"(Ci), "+v"(Dj), "+v"(mq.x), "+v"(mq.y), "+v"(mq.z), "+v"(mq.w), "+v"(tdx), "+v"(tde));
+  asm volatile("" : "+v"(hA), "+v"(hB), "+v"(hC), "+v"(c2o), "+v"(c2h), "+v"(c2r));
 #pragma unroll
-    for (int f = 0; f < 5; ++f) L.w[f] = w0[(size_t)f * nf + x];
+  for (int q = 0; q < 7; ++q) asm volatile("" : "+v"(rv[q]), "+v"(rp[q]));
 #pragma unroll
-    for (int f = 0; f < 5; ++f) L.y[f] = __builtin_nontemporal_load(yi + (size_t)f * nf + (upd ? x : 0));
-    const size_t g = grad ? (size_t)P * nf + x : 0;
-    if constexpr (D32)
-      L.dvf = __builtin_nontemporal_load(reinterpret_cast<const float*>(dvb) + g);
-    else
-      L.dv = __builtin_nontemporal_load(dvb + g);
-    L.g = gcb[g];
-    const size_t hk = (size_t)k * plane + hcell;
-    L.hw[0] = w0[hk];
-    L.hw[1] = w0[nf + hk];
-    L.hw[2] = w0[2 * nf + hk];
-    L.hw[3] = w0[4 * nf + hk];
-    const size_t ek = (size_t)min(k + 3, nr - 1) * plane + ij;
-    L.rw[0] = w0[ek];
-    L.rw[1] = w0[3 * nf + ek];
-    L.rw[2] = w0[4 * nf + ek];
-    L.c2o = c2b[c2f ? x : 0];
-    L.c2h = c2b[c2f ? hk : 0];
-    L.c2r = c2b[c2f ? ek : 0];
-  };
-  if (threadIdx.y == 0 && threadIdx.x < 7) {  // read after the first plane's barrier
-    sfc[0][threadIdx.x] = T.fcx[threadIdx.x];
-    sfc[1][threadIdx.x] = T.fcy[threadIdx.x];
-  }
-  AdjPlane nxt;
-  load_plane(k0, nxt);
+  for (int f = 0; f < 5; ++f) asm volatile("" : "+v"(w_n[f]));
+  asm volatile("" : "+v"(hw[0]), "+v"(hw[1]), "+v"(hw[2]), "+v"(hw[3]), "+v"(rw[0]), "+v"(rw[1]), "+v"(rw[2]));
+  load_update(k0);
+
+  const double c4 = T.fcx[4], c5 = T.fcx[5], c6 = T.fcx[6];  // antisymmetric taps (checked at upload)
+  const double sig_dt = RHS ? 1.0 : dt;
+  const size_t gx_side = (size_t)nr * n * 3, gy_side = gx_side;
 
   for (int k = k0; k < k1; ++k) {
-    const AdjPlane cur = nxt;
-    load_plane(min(k + 1, k1 - 1), nxt);  // the last plane's prefetch is loaded and not used
     const auto& row = rows[k];
     const bool bck = k == 0 || k == nr - 1;
     if (k > k0) {
@@ -276,68 +298,79 @@ __global__ __launch_bounds__(TI* TJ) void k_adj_stage(DevTables T, const double*
         rp[q] = rp[q + 1];
       }
       const int ke = k + 3;
-      if (ke < nr) {
-        const auto& re = rows[ke];
-        adj_radial(re, ke == nr - 1, c2rho0_of(re, cur.c2r), ws * cur.rw[0], ws * cur.rw[1], ws * cur.rw[2], rv[6],
-                   rp[6]);
-      } else {
+      const auto& re = rows[min(ke, nr - 1)];
+      adj_radial(re, ke >= nr - 1, c2rho0_of(re, c2r), ws * rw[0], ws * rw[1], ws * rw[2], rv[6], rp[6]);
+      if (ke >= nr) {
+        asm volatile("");  // stays a branch
         rv[6] = 0.0;
         rp[6] = 0.0;
       }
     }
-    const size_t kp = (size_t)k * plane;
     const int bf = (k - k0) & 1;
     // own point
-    const double w1 = ws * cur.w[0], w2 = ws * cur.w[1], w3 = ws * cur.w[2], w4 = ws * cur.w[3], w5 = ws * cur.w[4];
+    const double w1 = ws * w_n[0], w2 = ws * w_n[1], w3 = ws * w_n[2], w4 = ws * w_n[3], w5 = ws * w_n[4];
     AdjU u;
-    adj_point(row, bck, Ci, Dj, mq, c2rho0_of(row, cur.c2o), w1, w2, w3, w4, w5, u);
+    adj_point(row, bck, Ci, Dj, mq, c2rho0_of(row, c2o), w1, w2, w3, w4, w5, u);
     sxv[bf][ty][tx + 3] = u.uxv;
     sxp[bf][ty][tx + 3] = u.uxp;
     syv[bf][ty + 3][tx] = u.uyv;
     syp[bf][ty + 3][tx] = u.uyp;
-    if (has_h) {
-      double hv = 0.0, hp = 0.0;
-      if (h_in) {  // the halo cell's one input: u_xv, u_xp (x halo) or u_yv, u_yp (y halo)
-        const double b1 = bck ? 0.0 : ws * cur.hw[0], b2 = bck ? 0.0 : ws * cur.hw[1],
-                     b3 = bck ? 0.0 : ws * cur.hw[2], b5 = bck ? 0.0 : ws * cur.hw[3];
-        const double divb = -row.rho0 * b1 - c2rho0_of(row, cur.c2h) * b5;
-        const double gxb = -b2 * row.inv_rho0, geb = -b3 * row.inv_rho0;
-        hv = row.inv_r * hA * divb;
-        hp = row.inv_r * (hB * gxb + hC * geb);
+    {  // the halo cell's one input: u_xv, u_xp (x halo) or u_yv, u_yp (y halo)
+      const double h1 = ws * hw[0], h2 = ws * hw[1], h3 = ws * hw[2], h5 = ws * hw[3];
+      const double divb = -row.rho0 * h1 - c2rho0_of(row, c2h) * h5;
+      const double gxb = -h2 * row.inv_rho0, geb = -h3 * row.inv_rho0;
+      double hv = row.inv_r * hA * divb;
+      double hp = row.inv_r * (hB * gxb + hC * geb);
+      if (!h_in || bck) {
+        hv = 0.0;
+        hp = 0.0;
       }
-      if (hx) {
-        sxv[bf][hrow][hcol] = hv;
-        sxp[bf][hrow][hcol] = hp;
-      } else {
-        syv[bf][hrow][hcol] = hv;
-        syp[bf][hrow][hcol] = hp;
+      if (has_h) {
+        if (hx) {
+          sxv[bf][hrow][hcol] = hv;
+          sxp[bf][hrow][hcol] = hp;
+        } else {
+          syv[bf][hrow][hcol] = hv;
+          syp[bf][hrow][hcol] = hp;
+        }
       }
     }
+    load_start(min(k + 1, k1 - 1));  // the last plane's is loaded and not used
     __syncthreads();
 
     // Transposed stencils: (D^T u)(i) = sum_q c[6-q] u(i-3+q); one set of
-    // coefficients for xi and eta, whose zero centre tap adds nothing (as in
-    // the forward stage; both checked when the tables are uploaded).
+    // antisymmetric coefficients for xi and eta, whose zero centre tap adds
+    // nothing (as in the forward stage).
+    const double tap[7] = {c6, c5, c4, 0.0, -c4, -c5, -c6};
     double dxv = 0.0, dxp = 0.0, dyv = 0.0, dyp = 0.0;
 #pragma unroll
     for (int q = 0; q < 7; ++q) {
       if (q == 3) continue;
-      dxv += T.fcx[6 - q] * sxv[bf][ty][tx + q];
-      dxp += T.fcx[6 - q] * sxp[bf][ty][tx + q];
-      dyv += T.fcx[6 - q] * syv[bf][ty + q][tx];
-      dyp += T.fcx[6 - q] * syp[bf][ty + q][tx];
+      dxv += tap[q] * sxv[bf][ty][tx + q];
+      dxp += tap[q] * sxp[bf][ty][tx + q];
+      dyv += tap[q] * syv[bf][ty + q][tx];
+      dyp += tap[q] * syp[bf][ty + q][tx];
     }
     // Transposed radial stencil: every row kk whose DDR stencil reads plane k.
     double drv = 0.0, drp = 0.0;
+    if (k >= 6 && k < nr - 6) {  // interior rows: row k-3+q reads plane k with its tap 6-q
 #pragma unroll
-    for (int q = 0; q < 7; ++q) {
-      const int kk = k - 3 + q;
-      if (kk >= 0 && kk < nr) {
-        const int t = k - ddr_base(kk, nr);
-        if (t >= 0 && t <= 6) {
-          const double wt = rows[kk].w[t];
-          drv += wt * rv[q];
-          drp += wt * rp[q];
+      for (int q = 0; q < 7; ++q) {
+        const double wt = rows[k - 3 + q].w[6 - q];
+        drv += wt * rv[q];
+        drp += wt * rp[q];
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 7; ++q) {
+        const int kk = k - 3 + q;
+        if (kk >= 0 && kk < nr) {
+          const int t = k - ddr_base(kk, nr);
+          if (t >= 0 && t <= 6) {
+            const double wt = rows[kk].w[t];
+            drv += wt * rv[q];
+            drp += wt * rp[q];
+          }
         }
       }
     }
@@ -370,24 +403,28 @@ __global__ __launch_bounds__(TI* TJ) void k_adj_stage(DevTables T, const double*
     lt[3] = -row.drho0dr * u.b1 + row.rho0g0 * u.b5 + (2.0 * row.inv_r) * u.divb - sg * w4 + drv;
     lt[4] = -sg * w5 + dxp + dyp + drp;
 
-    const size_t x = kp + ij;
-    double* yo = Yout + (size_t)(P * 5) * nf;
-    if (mode & kAdjRhsOnly) {
+    const size_t kp = (size_t)k * ps;
+    const unsigned o = lane_offset(off);
+    if constexpr (RHS) {
 #pragma unroll
-      for (int f = 0; f < 5; ++f) yo[(size_t)f * nf + x] = lt[f];
+      for (int f = 0; f < 5; ++f) store_at(yob + kp + f * fs, o, lt[f]);
     } else {
-      double* wo = Wout + (size_t)(P * 5) * nf;
       const double wv[5] = {w1, w2, w3, w4, w5};
+      double yn[5], gn = 0.0;
 #pragma unroll
-      for (int f = 0; f < 5; ++f) {
-        const double yn = cur.y[f] + dt * lt[f];
-        __builtin_nontemporal_store(yn, yo + (size_t)f * nf + x);
-        if (mode & kAdjWriteW) __builtin_nontemporal_store(alpha * wv[f] + beta * yn, wo + (size_t)f * nf + x);
-      }
-      if (grad) {
+      for (int f = 0; f < 5; ++f) yn[f] = y_n[f] + dt * lt[f];
+      if constexpr (GRAD) {
         // r5 = -c^2 rho0 div + ...  ->  d r5 / d c^2 = -rho0 div (zero on the BC planes)
-        const double dv = D32 ? static_cast<double>(cur.dvf) : cur.dv;
-        gc2[(size_t)P * nf + x] = cur.g + dt * (-row.rho0 * dv) * u.b5;
+        const double dv = D32 ? static_cast<double>(dvf_n) : dv_n;
+        gn = g_n + dt * (-row.rho0 * dv) * u.b5;
+      }
+      load_update(min(k + 1, k1 - 1));
+      if constexpr (GRAD) store_at(bytes(gc2) + ((size_t)P * nf + (size_t)k * plane) * 8, o, gn);
+#pragma unroll
+      for (int f = 0; f < 5; ++f) store_at_nt(yob + kp + f * fs, o, yn[f]);
+      if (write_w) {
+#pragma unroll
+        for (int f = 0; f < 5; ++f) store_at_nt(wob + kp + f * fs, o, alpha * wv[f] + beta * yn[f]);
       }
     }
 
@@ -397,45 +434,45 @@ __global__ __launch_bounds__(TI* TJ) void k_adj_stage(DevTables T, const double*
       const int l = tx + 1;
       double gp = 0.0, gv = 0.0;
       for (int ii = 0; ii <= 3 - l; ++ii) {
-        gp += sfc[0][3 - l - ii] * sxp[bf][ty][3 + ii];
-        gv += sfc[0][3 - l - ii] * sxv[bf][ty][3 + ii];
+        gp += sfc[3 - l - ii] * sxp[bf][ty][3 + ii];
+        gv += sfc[3 - l - ii] * sxv[bf][ty][3 + ii];
       }
-      const size_t o = (size_t)(P * 2) * gx_side + ((size_t)k * n + j) * 3 + (l - 1);
-      gxa_p[o] = sig_dt * gp;
-      gxa_v[o] = sig_dt * gv;
+      const size_t x = (size_t)(P * 2) * gx_side + ((size_t)k * n + j) * 3 + (l - 1);
+      gxa_p[x] = sig_dt * gp;
+      gxa_v[x] = sig_dt * gv;
     }
     if (bi == nti - 1 && tx >= TI - 3) {
       const int l = tx - (TI - 3) + 1;
       double gp = 0.0, gv = 0.0;
       for (int ii = n - 4 + l; ii <= n - 1; ++ii) {
-        gp += sfc[0][n + 2 + l - ii] * sxp[bf][ty][3 + ii - i0];
-        gv += sfc[0][n + 2 + l - ii] * sxv[bf][ty][3 + ii - i0];
+        gp += sfc[n + 2 + l - ii] * sxp[bf][ty][3 + ii - i0];
+        gv += sfc[n + 2 + l - ii] * sxv[bf][ty][3 + ii - i0];
       }
-      const size_t o = (size_t)(P * 2 + 1) * gx_side + ((size_t)k * n + j) * 3 + (l - 1);
-      gxa_p[o] = sig_dt * gp;
-      gxa_v[o] = sig_dt * gv;
+      const size_t x = (size_t)(P * 2 + 1) * gx_side + ((size_t)k * n + j) * 3 + (l - 1);
+      gxa_p[x] = sig_dt * gp;
+      gxa_v[x] = sig_dt * gv;
     }
     if (bj == 0 && ty < 3) {
       const int l = ty + 1;
       double gp = 0.0, gv = 0.0;
       for (int jj = 0; jj <= 3 - l; ++jj) {
-        gp += sfc[1][3 - l - jj] * syp[bf][3 + jj][tx];
-        gv += sfc[1][3 - l - jj] * syv[bf][3 + jj][tx];
+        gp += sfc[3 - l - jj] * syp[bf][3 + jj][tx];
+        gv += sfc[3 - l - jj] * syv[bf][3 + jj][tx];
       }
-      const size_t o = (size_t)(P * 2) * gy_side + ((size_t)k * 3 + (l - 1)) * n + i;
-      gya_p[o] = sig_dt * gp;
-      gya_v[o] = sig_dt * gv;
+      const size_t x = (size_t)(P * 2) * gy_side + ((size_t)k * 3 + (l - 1)) * n + i;
+      gya_p[x] = sig_dt * gp;
+      gya_v[x] = sig_dt * gv;
     }
     if (bj == ntj - 1 && ty >= TJ - 3) {
       const int l = ty - (TJ - 3) + 1;
       double gp = 0.0, gv = 0.0;
       for (int jj = n - 4 + l; jj <= n - 1; ++jj) {
-        gp += sfc[1][n + 2 + l - jj] * syp[bf][3 + jj - j0][tx];
-        gv += sfc[1][n + 2 + l - jj] * syv[bf][3 + jj - j0][tx];
+        gp += sfc[n + 2 + l - jj] * syp[bf][3 + jj - j0][tx];
+        gv += sfc[n + 2 + l - jj] * syv[bf][3 + jj - j0][tx];
       }
-      const size_t o = (size_t)(P * 2 + 1) * gy_side + ((size_t)k * 3 + (l - 1)) * n + i;
-      gya_p[o] = sig_dt * gp;
-      gya_v[o] = sig_dt * gv;
+      const size_t x = (size_t)(P * 2 + 1) * gy_side + ((size_t)k * 3 + (l - 1)) * n + i;
+      gya_p[x] = sig_dt * gp;
+      gya_v[x] = sig_dt * gv;
     }
   }
 }
@@ -869,7 +906,7 @@ __global__ void k_inject(double* __restrict__ lam, const long long* __restrict__
 
 static int adj_ti(int n) { return (n % 32 == 0) ? 32 : 16; }
 
-template <int TI, int TJ, bool D32>
+template <int TI, int TJ>
 static hipError_t launch_adj_stage_t(const DevTables& T, const AdjStageArgs& a, hipStream_t st) {
   const int tiles = (T.n / TI) * (T.n / TJ) * 6;
   // chunks of >= 24 planes, as many as fit in three rounds of the GPU's blocks
@@ -885,17 +922,25 @@ static hipError_t launch_adj_stage_t(const DevTables& T, const AdjStageArgs& a, 
   if (tiles * nkch < 1024) nkch = small_grid_chunks(tiles, T.nr, 1.5, 2, 1.25);
   if (a.chunks > 0) nkch = std::min(a.chunks, T.nr);
   const int kchunk = (T.nr + nkch - 1) / nkch;
-  hipLaunchKernelGGL((k_adj_stage<TI, TJ, D32>), dim3(tiles * nkch), dim3(TI, TJ), 0, st, T, a.W, a.Yin, a.Yout,
-                     a.Wout, a.divs, a.gc2, a.c2f, a.gxa_p, a.gya_p, a.gxa_v, a.gya_v, a.dt, a.alpha, a.beta, a.wscale,
-                     kchunk, nkch, a.mode);
+#define SOLAR_ADJ_LAUNCH(KIND)                                                                                    \
+  hipLaunchKernelGGL((k_adj_stage<TI, TJ, KIND>), dim3(tiles * nkch), dim3(TI, TJ), 0, st, T, a.W, a.Yin, a.Yout, \
+                     a.Wout, a.divs, a.gc2, a.c2f, a.gxa_p, a.gya_p, a.gxa_v, a.gya_v, a.dt, a.alpha, a.beta,     \
+                     a.wscale, kchunk, nkch, (a.mode & kAdjWriteW) != 0)
+  if (a.mode & kAdjRhsOnly)
+    SOLAR_ADJ_LAUNCH(kAdjRhs);
+  else if (!(a.mode & kAdjGrad))
+    SOLAR_ADJ_LAUNCH(kAdjStep);
+  else if (a.div32)
+    SOLAR_ADJ_LAUNCH(kAdjGrad32);
+  else
+    SOLAR_ADJ_LAUNCH(kAdjGrad64);
+#undef SOLAR_ADJ_LAUNCH
   return hipGetLastError();
 }
 
 hipError_t launch_adj_stage(const DevTables& T, const AdjStageArgs& a, hipStream_t st) {
-  const bool d32 = a.div32 && a.divs && (a.mode & kAdjGrad);
-  if (adj_ti(T.n) == 32)
-    return d32 ? launch_adj_stage_t<32, 8, true>(T, a, st) : launch_adj_stage_t<32, 8, false>(T, a, st);
-  return d32 ? launch_adj_stage_t<16, 16, true>(T, a, st) : launch_adj_stage_t<16, 16, false>(T, a, st);
+  if (adj_ti(T.n) == 32) return launch_adj_stage_t<32, 8>(T, a, st);
+  return launch_adj_stage_t<16, 16>(T, a, st);
 }
 
 template <bool VEC, bool RADF, int NI, bool HASW>

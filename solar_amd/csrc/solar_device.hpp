@@ -24,6 +24,32 @@ __device__ __forceinline__ global_ptr<T> to_global(T* p) {
   return (global_ptr<T>)p;
 }
 
+// Accesses that name global memory with a wave-uniform base and a 32-bit lane
+// offset: the address costs no vector instruction.  lane_offset hides that an
+// offset does not change in a loop: widened to 64 bits outside the loop, it
+// would cost an add at every access.
+__device__ __forceinline__ unsigned lane_offset(unsigned v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+using GlobalBytes = const __attribute__((address_space(1))) char*;
+template <typename V>
+__device__ __forceinline__ V load_at(GlobalBytes base, unsigned off) {
+  return *(const __attribute__((address_space(1))) V*)(base + off);
+}
+template <typename V>
+__device__ __forceinline__ V load_at_nt(GlobalBytes base, unsigned off) {
+  return __builtin_nontemporal_load((const __attribute__((address_space(1))) V*)(base + off));
+}
+template <typename V>
+__device__ __forceinline__ void store_at_nt(GlobalBytes base, unsigned off, V v) {
+  __builtin_nontemporal_store(v, (__attribute__((address_space(1))) V*)const_cast<__attribute__((address_space(1))) char*>(base + off));
+}
+template <typename V>
+__device__ __forceinline__ void store_at(GlobalBytes base, unsigned off, V v) {
+  *(__attribute__((address_space(1))) V*)const_cast<__attribute__((address_space(1))) char*>(base + off) = v;
+}
+
 // Block index remap so that consecutive logical blocks (neighbouring tiles,
 // whose halos overlap) run on the same XCD and share its L2.  Hardware
 // dispatches block b to XCD b % 8; XCD x receives nb / 8 blocks, one more
