@@ -20,7 +20,8 @@ HIP_FLAGS = [
 ]
 HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-I/opt/rocm/include"]
 SOURCES_HIP = ["solar_kernels.hip", "solar_adjoint.hip", "solar_noalloc.hip"]
-SOURCES_HOST = ["solar_tables.cpp", "solar_ic.cpp", "solar_capi.cpp", "solar_ensemble.cpp", "solar_io.cpp"]
+SOURCES_HOST = ["solar_tables.cpp", "solar_ic.cpp", "solar_capi.cpp", "solar_ensemble.cpp", "solar_io.cpp",
+                "solar_hostcopy.cpp"]
 
 
 def hipcc():

@@ -69,6 +69,7 @@ struct solar_ctx {
   std::vector<hipEvent_t> ev;
   double ktime[5] = {0, 0, 0, 0, 0};
   size_t bytes = 0;
+  solar::HostCopy host;  // large copies from and to the caller's arrays
   // sensitivity / adjoint state, allocated on first use
   double* c2f = nullptr;  // optional 3-D c^2 (n,n,nr,6); points at c2f_buf when set
   double* c2f_buf = nullptr;
@@ -404,7 +405,7 @@ int solar_finalize(solar_ctx* c) {
 // Host double array -> device buffer in the handle's storage type.
 static int upload_state(solar_ctx* c, void* dst, const double* src, size_t count) {
   if (!c->f32) {
-    HIPCHK(hipMemcpyAsync(dst, src, count * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c->host.to_device(dst, src, count * sizeof(double), c->device, c->stream));
   } else {
     std::vector<float> tmp(src, src + count);
     HIPCHK(hipMemcpyAsync(dst, tmp.data(), count * sizeof(float), hipMemcpyHostToDevice, c->stream));
@@ -416,8 +417,7 @@ static int upload_state(solar_ctx* c, void* dst, const double* src, size_t count
 // Device buffer in the handle's storage type -> host double array.
 static int download_state(solar_ctx* c, double* dst, const void* src, size_t count) {
   if (!c->f32) {
-    HIPCHK(hipMemcpyAsync(dst, src, count * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(c->host.to_host(dst, src, count * sizeof(double), c->device, c->stream));
   } else {
     std::vector<float> tmp(count);
     HIPCHK(hipMemcpyAsync(tmp.data(), src, count * sizeof(float), hipMemcpyDeviceToHost, c->stream));
@@ -743,12 +743,11 @@ static int adj_alloc(solar_ctx* c) {
 }
 
 static int upload_f64(solar_ctx* c, double* dst, const double* src, size_t count) {
-  HIPCHK(hipMemcpyAsync(dst, src, count * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c->host.to_device(dst, src, count * sizeof(double), c->device, c->stream));
   return SOLAR_OK;
 }
 static int download_f64(solar_ctx* c, double* dst, const double* src, size_t count) {
-  HIPCHK(hipMemcpyAsync(dst, src, count * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
+  HIPCHK(c->host.to_host(dst, src, count * sizeof(double), c->device, c->stream));
   return SOLAR_OK;
 }
 

@@ -66,6 +66,8 @@ struct solar_ens {
   std::vector<void*> allocs;
   std::vector<void*> list_allocs;  // work lists, rebuilt by the autotuner
   size_t bytes = 0;
+  int device = 0;
+  solar::HostCopy host;  // large copies from and to the caller's arrays
   hipStream_t stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -255,6 +257,7 @@ int solar_ens_create(solar_ens** out, int nmembers, const int* n, const int* nr,
     delete e;
     return code;
   };
+  (void)hipGetDevice(&e->device);
   e->nm = nmembers;
   e->n.assign(n, n + nmembers);
   e->nr.assign(nr, nr + nmembers);
@@ -455,16 +458,14 @@ int solar_ens_autotune(solar_ens* e, int reps) {
 int solar_ens_set_state(solar_ens* e, int m, const double* q) {
   if (!e || !q || m < 0 || m >= e->nm) return solar::set_error(SOLAR_ERR_ARG, "solar_ens_set_state: invalid argument");
   const size_t b = static_cast<size_t>(e->n[m]) * e->n[m] * e->nr[m] * 30 * sizeof(double);
-  ENSCHK(hipMemcpyAsync(e->mem[m].q[0], q, b, hipMemcpyHostToDevice, e->stream));
-  ENSCHK(hipStreamSynchronize(e->stream));
+  ENSCHK(e->host.to_device(e->mem[m].q[0], q, b, e->device, e->stream));
   return SOLAR_OK;
 }
 
 int solar_ens_get_state(solar_ens* e, int m, double* q) {
   if (!e || !q || m < 0 || m >= e->nm) return solar::set_error(SOLAR_ERR_ARG, "solar_ens_get_state: invalid argument");
   const size_t b = static_cast<size_t>(e->n[m]) * e->n[m] * e->nr[m] * 30 * sizeof(double);
-  ENSCHK(hipMemcpyAsync(q, e->mem[m].q[0], b, hipMemcpyDeviceToHost, e->stream));
-  ENSCHK(hipStreamSynchronize(e->stream));
+  ENSCHK(e->host.to_host(q, e->mem[m].q[0], b, e->device, e->stream));
   return SOLAR_OK;
 }
 

@@ -1,0 +1,118 @@
+// Large copies between pageable host memory and the device.
+//
+// A caller's array is pageable and often fresh: the runtime's own copy of
+// 830 MB into new arrays runs at 9 GB/s, one thread faulting their pages in.
+// Here a few threads each take a contiguous part of the array through two
+// pinned pieces of their own: while one piece is on the link, the other is
+// copied to or from the array.  Measured on 830 MB of ensemble states: into
+// new arrays 90 -> 27 ms, from arrays 29 -> 19 ms (eight threads 25 and 20).
+#include "solar_internal.hpp"
+
+#include <algorithm>
+#include <cstring>
+#include <new>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+namespace solar {
+
+namespace {
+
+constexpr int kThreads = 4;
+constexpr size_t kPiece = size_t(4) << 20;
+constexpr size_t kLeast = size_t(32) << 20;  // below, starting the threads costs more than it gives
+
+}  // namespace
+
+struct HostCopy::Staging {
+  char* buf = nullptr;  // pinned, kThreads x 2 pieces
+  hipEvent_t ev[kThreads][2] = {};
+  int made = 0;
+
+  hipError_t make() {
+    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&buf), kThreads * 2 * kPiece, hipHostMallocDefault);
+    for (int x = 0; x < 2 * kThreads && e == hipSuccess; ++x, ++made)
+      e = hipEventCreateWithFlags(&ev[x / 2][x % 2], hipEventDisableTiming);
+    return e;
+  }
+  ~Staging() {
+    for (int x = 0; x < made; ++x) (void)hipEventDestroy(ev[x / 2][x % 2]);
+    if (buf) (void)hipHostFree(buf);
+  }
+};
+
+HostCopy::~HostCopy() { delete s_; }
+
+// One thread's part: pieces in order, alternating between the two buffers.
+hipError_t HostCopy::part(int t, char* host, char* dev, size_t bytes, bool down, int device, hipStream_t st) {
+  hipError_t e = hipSetDevice(device);
+  const size_t np = (bytes + kPiece - 1) / kPiece;
+  char* buf[2] = {s_->buf + (2 * t) * kPiece, s_->buf + (2 * t + 1) * kPiece};
+  auto size = [&](size_t p) { return std::min(kPiece, bytes - p * kPiece); };
+  // down: piece p is on the link while piece p - 1 is copied out; up: piece p
+  // is copied in while piece p - 1 is on the link
+  for (size_t p = 0; p < np + (down ? 1 : 2) && e == hipSuccess; ++p) {
+    if (down) {
+      if (p < np) {
+        e = hipMemcpyAsync(buf[p & 1], dev + p * kPiece, size(p), hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess) e = hipEventRecord(s_->ev[t][p & 1], st);
+      }
+      if (p > 0 && e == hipSuccess) {
+        e = hipEventSynchronize(s_->ev[t][(p - 1) & 1]);
+        if (e == hipSuccess) std::memcpy(host + (p - 1) * kPiece, buf[(p - 1) & 1], size(p - 1));
+      }
+    } else {
+      if (p >= 2) e = hipEventSynchronize(s_->ev[t][p & 1]);  // piece p - 2 has left its buffer
+      if (p < np && e == hipSuccess) {
+        std::memcpy(buf[p & 1], host + p * kPiece, size(p));
+        e = hipMemcpyAsync(dev + p * kPiece, buf[p & 1], size(p), hipMemcpyHostToDevice, st);
+        if (e == hipSuccess) e = hipEventRecord(s_->ev[t][p & 1], st);
+      }
+    }
+  }
+  return e;
+}
+
+hipError_t HostCopy::run(void* host, void* dev, size_t bytes, bool down, int device, hipStream_t st) {
+  auto plain = [&]() {
+    const hipError_t e = down ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st)
+                              : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
+    return e == hipSuccess ? hipStreamSynchronize(st) : e;
+  };
+  if (bytes < kLeast) return plain();
+  if (!s_) {
+    Staging* s = new (std::nothrow) Staging();
+    if (!s || s->make() != hipSuccess) {
+      (void)hipGetLastError();
+      delete s;
+      return plain();
+    }
+    s_ = s;
+  }
+  const size_t each = (bytes / kThreads + kPiece - 1) / kPiece * kPiece;
+  hipError_t err[kThreads] = {};
+  auto work = [&](int t) {
+    const size_t a = std::min(bytes, each * t), b = t == kThreads - 1 ? bytes : std::min(bytes, each * (t + 1));
+    err[t] = part(t, static_cast<char*>(host) + a, static_cast<char*>(dev) + a, b - a, down, device, st);
+  };
+  std::thread th[kThreads];
+  for (int t = 1; t < kThreads; ++t) {
+    try {
+      th[t] = std::thread(work, t);
+    } catch (const std::system_error&) {  // no thread to be had: this one does the part
+      work(t);
+    }
+  }
+  work(0);
+  for (int t = 1; t < kThreads; ++t)
+    if (th[t].joinable()) th[t].join();
+  for (hipError_t e : err)
+    if (e != hipSuccess) {
+      (void)hipStreamSynchronize(st);  // nothing of the copy is in flight on return
+      return e;
+    }
+  return hipSuccess;
+}
+
+}  // namespace solar

@@ -24,4 +24,28 @@ int upload_tables(const Tables& t, DevTables* d, std::vector<void*>* allocs, siz
 size_t scratch_bytes();
 hipError_t scratch_address(int device, void** addr);
 
+// Copies between a caller's host array and the device, synchronous, ordered
+// after the work on `st` (solar_hostcopy.cpp).  Large ones go through pinned
+// staging that the object makes on the first of them and keeps (32 MiB); it is
+// for one thread at a time, as the handle that owns it.
+class HostCopy {
+ public:
+  HostCopy() = default;
+  HostCopy(const HostCopy&) = delete;
+  HostCopy& operator=(const HostCopy&) = delete;
+  ~HostCopy();
+  hipError_t to_device(void* dev, const void* host, size_t bytes, int device, hipStream_t st) {
+    return run(const_cast<void*>(host), dev, bytes, false, device, st);
+  }
+  hipError_t to_host(void* host, const void* dev, size_t bytes, int device, hipStream_t st) {
+    return run(host, const_cast<void*>(dev), bytes, true, device, st);
+  }
+
+ private:
+  struct Staging;
+  Staging* s_ = nullptr;
+  hipError_t run(void* host, void* dev, size_t bytes, bool down, int device, hipStream_t st);
+  hipError_t part(int t, char* host, char* dev, size_t bytes, bool down, int device, hipStream_t st);
+};
+
 }  // namespace solar
