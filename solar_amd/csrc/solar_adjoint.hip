@@ -114,7 +114,8 @@ __device__ __forceinline__ void adj_radial(const Row& row, bool bc, double c2rho
 //   gc2  : c^2 gradient accumulator (n,n,nr,6)
 //   gxa_*, gya_* : dt-scaled ghost adjoints written by edge tiles
 // KIND: kAdjStep, kAdjGrad64 or kAdjGrad32 (with the gradient, from FP64 or
-// FP32 divergences), kAdjRhs (Yout = L^T W; dt must be 1).
+// FP32 divergences), kAdjRhs (Yout = L^T W; dt must be 1).  STREAM: the Ybar
+// and W streams are non-temporal (stream_past_cache).
 //
 // Bound by memory where the grid fills the chip (6x96^2x192, mean of a step's
 // five: 170 bytes a point at 4.5 TB/s, where a march of as many streams with
@@ -129,7 +130,7 @@ __device__ __forceinline__ void adj_radial(const Row& row, bool bc, double c2rho
 // 240 -> 204 registers, 6x96^2x192 431 -> 403 us, 6x48^2x100 71 -> 66 us.
 constexpr int kAdjStep = 0, kAdjGrad64 = 1, kAdjGrad32 = 2, kAdjRhs = 3;
 
-template <int TI, int TJ, int KIND>
+template <int TI, int TJ, int KIND, bool STREAM>
 __global__ __launch_bounds__(TI* TJ) __attribute__((amdgpu_waves_per_eu(kAdjWaves))) void k_adj_stage(
     DevTables T, const double* __restrict__ W, const double* Yin, double* Yout,  // may alias
     double* __restrict__ Wout, const double* __restrict__ divs, double* __restrict__ gc2,
@@ -245,7 +246,8 @@ __global__ __launch_bounds__(TI* TJ) __attribute__((amdgpu_waves_per_eu(kAdjWave
     const unsigned o = lane_offset(off);
     if constexpr (!RHS) {
 #pragma unroll
-      for (int f = 0; f < 5; ++f) y_n[f] = load_at_nt<double>(yb + kp + f * fs, o);
+      for (int f = 0; f < 5; ++f)
+        y_n[f] = STREAM ? load_at_nt<double>(yb + kp + f * fs, o) : load_at<double>(yb + kp + f * fs, o);
     }
     if constexpr (GRAD) {
       const size_t gk = (size_t)P * nf + (size_t)k * plane;
@@ -420,11 +422,17 @@ __global__ __launch_bounds__(TI* TJ) __attribute__((amdgpu_waves_per_eu(kAdjWave
       }
       load_update(min(k + 1, k1 - 1));
       if constexpr (GRAD) store_at(bytes(gc2) + ((size_t)P * nf + (size_t)k * plane) * 8, o, gn);
+      const auto put = [&](GlobalBytes p, double v) {
+        if constexpr (STREAM)
+          store_at_nt(p, o, v);
+        else
+          store_at(p, o, v);
+      };
 #pragma unroll
-      for (int f = 0; f < 5; ++f) store_at_nt(yob + kp + f * fs, o, yn[f]);
+      for (int f = 0; f < 5; ++f) put(yob + kp + f * fs, yn[f]);
       if (write_w) {
 #pragma unroll
-        for (int f = 0; f < 5; ++f) store_at_nt(wob + kp + f * fs, o, alpha * wv[f] + beta * yn[f]);
+        for (int f = 0; f < 5; ++f) put(wob + kp + f * fs, alpha * wv[f] + beta * yn[f]);
       }
     }
 
@@ -922,18 +930,28 @@ static hipError_t launch_adj_stage_t(const DevTables& T, const AdjStageArgs& a, 
   if (tiles * nkch < 1024) nkch = small_grid_chunks(tiles, T.nr, 1.5, 2, 1.25);
   if (a.chunks > 0) nkch = std::min(a.chunks, T.nr);
   const int kchunk = (T.nr + nkch - 1) / nkch;
-#define SOLAR_ADJ_LAUNCH(KIND)                                                                                    \
-  hipLaunchKernelGGL((k_adj_stage<TI, TJ, KIND>), dim3(tiles * nkch), dim3(TI, TJ), 0, st, T, a.W, a.Yin, a.Yout, \
-                     a.Wout, a.divs, a.gc2, a.c2f, a.gxa_p, a.gya_p, a.gxa_v, a.gya_v, a.dt, a.alpha, a.beta,     \
-                     a.wscale, kchunk, nkch, (a.mode & kAdjWriteW) != 0)
-  if (a.mode & kAdjRhsOnly)
-    SOLAR_ADJ_LAUNCH(kAdjRhs);
-  else if (!(a.mode & kAdjGrad))
-    SOLAR_ADJ_LAUNCH(kAdjStep);
-  else if (a.div32)
-    SOLAR_ADJ_LAUNCH(kAdjGrad32);
-  else
-    SOLAR_ADJ_LAUNCH(kAdjGrad64);
+  // plain streams where the buffers stay in the last-level cache, as in the
+  // forward stages (gradient 6x48^2x100 75.1 -> 71.9 ms, 6x96^2x192 201 against 212)
+  const bool nt = stream_past_cache((size_t)30 * T.n * T.n * T.nr * sizeof(double));
+#define SOLAR_ADJ_LAUNCH(KIND, NT)                                                                             \
+  hipLaunchKernelGGL((k_adj_stage<TI, TJ, KIND, NT>), dim3(tiles * nkch), dim3(TI, TJ), 0, st, T, a.W, a.Yin, \
+                     a.Yout, a.Wout, a.divs, a.gc2, a.c2f, a.gxa_p, a.gya_p, a.gxa_v, a.gya_v, a.dt, a.alpha, \
+                     a.beta, a.wscale, kchunk, nkch, (a.mode & kAdjWriteW) != 0)
+#define SOLAR_ADJ_KIND(KIND)      \
+  if (nt)                         \
+    SOLAR_ADJ_LAUNCH(KIND, true); \
+  else                            \
+    SOLAR_ADJ_LAUNCH(KIND, false);
+  if (a.mode & kAdjRhsOnly) {
+    SOLAR_ADJ_KIND(kAdjRhs)
+  } else if (!(a.mode & kAdjGrad)) {
+    SOLAR_ADJ_KIND(kAdjStep)
+  } else if (a.div32) {
+    SOLAR_ADJ_KIND(kAdjGrad32)
+  } else {
+    SOLAR_ADJ_KIND(kAdjGrad64)
+  }
+#undef SOLAR_ADJ_KIND
 #undef SOLAR_ADJ_LAUNCH
   return hipGetLastError();
 }

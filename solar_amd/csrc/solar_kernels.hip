@@ -289,7 +289,7 @@ struct StageArgs {
   const double *gxp, *gyp, *gxv, *gyv;
   double alpha, beta, beta_r, dt;
   int kchunk, nkch, rhs_mode;
-  int tile_w, whole;  // PART only; whole: rows and tiles are of whole 64-byte segments
+  int tile_w;  // PART only
   const double* c2f;
   double* divout;
   int div32;
@@ -303,6 +303,10 @@ struct StageArgs {
 // Flags of a stage instantiation beyond kStoreNoQ and kStageRecon.
 constexpr int kStageRhs = 4;  // evaluates the RHS alone (rhs_mode holds its flags), KIND 0
 constexpr int kStageAux = 8;  // c2f or divout is given
+// The streams that no other block reads (q and qw stores; rho' and qw loads)
+// are non-temporal; kStagePlain: they are not (launch_stage_t).  Partial tiles
+// load plainly either way: they share 128-byte lines with their neighbours.
+constexpr int kStagePlain = 16;
 
 // Reciprocal-based quotients (div_group) in the FP32-state stages only.
 template <typename S>
@@ -368,6 +372,7 @@ template <int TI, int TJ, int KIND, typename S, int MODE = 0, bool PART = false,
 __global__ __launch_bounds__(TI* TJ) __attribute__((amdgpu_waves_per_eu(kStageWaves)))
 void k_stage(StageArgs<S> A) {
   constexpr bool NOQ = (FL & kStoreNoQ) != 0, RECON = (FL & kStageRecon) != 0;
+  constexpr bool STREAM = (FL & kStagePlain) == 0;
   constexpr bool RHS = (FL & kStageRhs) != 0, AUX = (FL & (kStageRhs | kStageAux)) != 0;
   constexpr bool ENS = MODE == 1, TL = MODE == 2, WIDE = sizeof(S) == 8;
   static_assert(!(NOQ || RECON) || (MODE != 2 && WIDE), "the stored-q schedule variants are FP64, not tangent-linear");
@@ -528,10 +533,11 @@ void k_stage(StageArgs<S> A) {
   double c2_n = 0.0, tdc2 = 0.0, tdiv = 0.0;
   auto load_update = [&](int k) {
     const unsigned o = lane_offset(off);
-    q1_n = load_at_nt<S>(qb + (size_t)k * ps, o);
+    const auto get = [&](GlobalBytes p) { return STREAM && !PART ? load_at_nt<S>(p, o) : load_at<S>(p, o); };
+    q1_n = get(qb + (size_t)k * ps);
 #pragma unroll
     for (int f = 0; f < 5; ++f)
-      if (KIND != 0 && !(RECON && (f == 1 || f == 2))) w_n[f] = load_at_nt<S>(wb + (size_t)k * ps + f * fs, o);
+      if (KIND != 0 && !(RECON && (f == 1 || f == 2))) w_n[f] = get(wb + (size_t)k * ps + f * fs);
     const size_t dk = ((size_t)P * nf + (size_t)k * plane) * sizeof(double);
     const unsigned o8 = lane_offset(cell * 8u);
     if (AUX || TL) {
@@ -737,23 +743,16 @@ void k_stage(StageArgs<S> A) {
       }
       load_update(min(k + 1, k1 - 1));
       if (own_in) {
-        // Non-temporal stores, except where rows or tiles begin inside a
-        // 64-byte segment: a neighbouring tile completes that segment in L2
-        // (stage, 6x204^2x100: 1.03 -> 0.95 ms; with whole segments,
-        // 6x200^2x150, plain stores are slower: 1.17 -> 1.24 ms).
-        if (PART && !A.whole) {
-          asm volatile("");  // stays a branch
+        const auto put = [&](GlobalBytes p, S v) {
+          if constexpr (STREAM)
+            store_at_nt(p, o, v);
+          else
+            store_at(p, o, v);
+        };
 #pragma unroll
-          for (int f = 0; f < 5; ++f) {
-            if (!NOQ) store_at(ob + kp + f * fs, o, qn[f]);
-            if (KIND != 2) store_at(wob + kp + f * fs, o, wn[f]);
-          }
-        } else {
-#pragma unroll
-          for (int f = 0; f < 5; ++f) {
-            if (!NOQ) store_at_nt(ob + kp + f * fs, o, qn[f]);
-            if (KIND != 2) store_at_nt(wob + kp + f * fs, o, wn[f]);
-          }
+        for (int f = 0; f < 5; ++f) {
+          if (!NOQ) put(ob + kp + f * fs, qn[f]);
+          if (KIND != 2) put(wob + kp + f * fs, wn[f]);
         }
       }
       if (ec_on) {
@@ -1301,7 +1300,15 @@ static hipError_t launch_stage_t(StageArgs<S> a, int stage, int xf, hipStream_t 
   // against 318 at 20 planes, 308 at 16)
   if (tiles * nkch < 1536) nkch = small_grid_chunks(tiles, T.nr, 1.0, 3, 1.25);
   if (ls.stage_chunks > 0) nkch = ls.stage_chunks;
-  a.whole = T.n * sizeof(S) % 64 == 0 && W * sizeof(S) % 64 == 0;
+  // Non-temporal streams, but not where the step's buffers stay in the 256 MB
+  // last-level cache between launches (stream_past_cache), and in partial
+  // tiles only where rows and tiles are of whole 64-byte segments: else a
+  // neighbouring tile completes the segment in L2 (stage, 6x204^2x100: 1.03 ->
+  // 0.95 ms; with whole segments, 6x200^2x150, plain stores are slower: 1.17 ->
+  // 1.24 ms; plain loads there: step 7.41 -> 7.18 ms).  A template flag: chosen
+  // by a branch in the plane loop it cost the large grids 1 to 2%.
+  const bool plain = !stream_past_cache((size_t)30 * T.n * T.n * T.nr * sizeof(S)) ||
+                     (PART && (T.n * sizeof(S) % 64 != 0 || W * sizeof(S) % 64 != 0));
   a.nkch = nkch;
   a.kchunk = (T.nr + nkch - 1) / nkch;
   const dim3 grid(tiles * nkch), block = PART ? dim3(part_threads(W, TJ)) : dim3(TI, TJ);
@@ -1320,17 +1327,21 @@ static hipError_t launch_stage_t(StageArgs<S> a, int stage, int xf, hipStream_t 
   if constexpr (kMain && sizeof(S) == 8) {
     if (xf) {
       if (a.tl_dc2) return hipErrorInvalidValue;
-#define SOLAR_STAGE_XF(AUX)                                     \
-  if (xf == kStoreNoQ && kind == 0)                             \
-    SOLAR_STAGE_LAUNCH(0, 0, kStoreNoQ | (AUX));                \
-  else if (xf == kStoreNoQ && kind == 1)                        \
-    SOLAR_STAGE_LAUNCH(1, 0, kStoreNoQ | (AUX));                \
-  else if (xf == kStageRecon && kind == 1 && a.qwo)             \
-    SOLAR_STAGE_LAUNCH(1, 0, kStageRecon | (AUX));              \
-  else                                                          \
+#define SOLAR_STAGE_XF(FL)                          \
+  if (xf == kStoreNoQ && kind == 0)                 \
+    SOLAR_STAGE_LAUNCH(0, 0, kStoreNoQ | (FL));     \
+  else if (xf == kStoreNoQ && kind == 1)            \
+    SOLAR_STAGE_LAUNCH(1, 0, kStoreNoQ | (FL));     \
+  else if (xf == kStageRecon && kind == 1 && a.qwo) \
+    SOLAR_STAGE_LAUNCH(1, 0, kStageRecon | (FL));   \
+  else                                              \
     return hipErrorInvalidValue;
-      if (aux) {
+      if (aux && plain) {
+        SOLAR_STAGE_XF(kStageAux | kStagePlain)
+      } else if (aux) {
         SOLAR_STAGE_XF(kStageAux)
+      } else if (plain) {
+        SOLAR_STAGE_XF(kStagePlain)
       } else {
         SOLAR_STAGE_XF(0)
       }
@@ -1357,15 +1368,18 @@ static hipError_t launch_stage_t(StageArgs<S> a, int stage, int xf, hipStream_t 
     SOLAR_STAGE_LAUNCH(1, 0, FL); \
   else                            \
     SOLAR_STAGE_LAUNCH(2, 0, FL);
-  if (aux) {
-    if constexpr (kMain) {
+  if constexpr (kMain) {
+    if (aux) {
       SOLAR_STAGE_KIND(kStageAux)
-    } else {
-      return hipErrorInvalidValue;
+      return hipGetLastError();
     }
-  } else {
-    SOLAR_STAGE_KIND(0)
+    if (plain) {
+      SOLAR_STAGE_KIND(kStagePlain)
+      return hipGetLastError();
+    }
   }
+  if (aux) return hipErrorInvalidValue;
+  SOLAR_STAGE_KIND(0)
 #undef SOLAR_STAGE_KIND
 #undef SOLAR_STAGE_LAUNCH
   return hipGetLastError();

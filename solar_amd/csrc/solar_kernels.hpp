@@ -52,6 +52,14 @@ struct LaunchShape {
   int adj_stage_chunks = 0, adj_filter_chunks = 0;  // sensitivity kernels
 };
 
+// Whether a step's own-point streams bypass the caches (non-temporal): the
+// states of one buffer (bytes) are too large for the step's four to stay in
+// the 256 MB last-level cache from one launch to the next.  Measured step
+// times, non-temporal against plain: 63 MB 6x64^2x64 327 / 306 us, FP32 state
+// 6x64^2x128 413 / 370 us, 16 MB 6x32^2x64 148 / 129 us; 94 MB FP32 state
+// 6x64^2x192 569 / 604 us, 126 MB 6x64^2x128 604 / 622 us.
+constexpr bool stream_past_cache(size_t bytes) { return bytes > (size_t(64) << 20); }
+
 // Radial chunks of a march whose tiles do not fill the chip (solar_kernels.hip).
 int small_grid_chunks(int tiles, int nr, double warm, int resident, double alone);
 

@@ -37,8 +37,11 @@ def test_partial_tiles_match_the_oracle(n, nr, bits):
     assert np.array_equal(got, want)
 
 
-def test_wide_tiles_with_a_c2_field_match_the_oracle():
-    n, nr = 128, 13
+# 13 planes: the step's buffers stay in the last-level cache (plain stores);
+# 24: they do not (non-temporal)
+@pytest.mark.parametrize("nr", [13, 24])
+def test_wide_tiles_with_a_c2_field_match_the_oracle(nr):
+    n = 128
     bg, q, length, dt = _inputs(n, nr)
     c2 = bg[1][None, :, None, None] * (1 + 0.02 * np.random.default_rng(3).random((6, nr, n, n)))
     o = oracle.Oracle(n, nr, *bg, length, 0.1)
@@ -50,8 +53,9 @@ def test_wide_tiles_with_a_c2_field_match_the_oracle():
         assert np.array_equal(s.get_state(), o.rk4(q, 1, dt)[0])
 
 
-def test_wide_tiles_gradient_and_tangent_linear(monkeypatch):
-    n, nr, steps = 128, 14, 3
+@pytest.mark.parametrize("nr", [14, 24])
+def test_wide_tiles_gradient_and_tangent_linear(nr, monkeypatch):
+    n, steps = 128, 3
     bg, q, length, dt = _inputs(n, nr)
     rng = np.random.default_rng(8)
     rec = np.array([[p, 6, 5 + p, 100] for p in range(6)])
