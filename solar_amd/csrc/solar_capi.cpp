@@ -174,12 +174,14 @@ int enqueue_step(solar_ctx* c, double dt, bool timed, double* const* divp = null
     for (int s = 0; s < 5; ++s) {
       const St& x = sch[s];
       if (timed) HIPCHK(hipEventRecord(c->ev[e++], c->stream));
-      HIPCHK(solar::launch_gather(T, x.qg, false, true, 4, 1, c->gxp, c->gyp, c->gxv, c->gyv, c->stream,
-                                  s > 0 ? c->ecols : nullptr, x.wg, x.bg));
+      const bool own = solar::stage_gathers(T, false, s, x.xf, c->shape, c->c2f, divp ? divp[s] : nullptr, nullptr);
+      if (!own)
+        HIPCHK(solar::launch_gather(T, x.qg, false, true, 4, 1, c->gxp, c->gyp, c->gxv, c->gyv, c->stream,
+                                    s > 0 ? c->ecols : nullptr, x.wg, x.bg));
       if (timed) HIPCHK(hipEventRecord(c->ev[e++], c->stream));
       HIPCHK(solar::launch_stage(T, x.qin, x.qout, x.qw, false, c->gxp, c->gyp, c->gxv, c->gyv, s, dt,
                                  0, c->stream, c->shape, c->c2f, divp ? divp[s] : nullptr, c->div_bits == 32,
-                                 nullptr, nullptr, c->ecols, x.xf, x.qwo, x.bg));
+                                 nullptr, nullptr, c->ecols, x.xf, x.qwo, x.bg, own));
     }
     if (timed) HIPCHK(hipEventRecord(c->ev[e++], c->stream));
     HIPCHK(solar::launch_gather(T, B, false, false, 0, 5, c->fgx, c->fgy, nullptr, nullptr, c->stream, c->ecols));
@@ -192,12 +194,14 @@ int enqueue_step(solar_ctx* c, double dt, bool timed, double* const* divp = null
   // the next gather reads its W/E strips; the first gather reads the state.
   for (int s = 0; s < 5; ++s) {
     if (timed) HIPCHK(hipEventRecord(c->ev[e++], c->stream));
-    HIPCHK(solar::launch_gather(T, cur, c->f32, true, 4, 1, c->gxp, c->gyp, c->gxv, c->gyv, c->stream,
-                                s > 0 ? c->ecols : nullptr));
+    const bool own = solar::stage_gathers(T, c->f32, s, 0, c->shape, c->c2f, divp ? divp[s] : nullptr, tl_dc2);
+    if (!own)
+      HIPCHK(solar::launch_gather(T, cur, c->f32, true, 4, 1, c->gxp, c->gyp, c->gxv, c->gyv, c->stream,
+                                  s > 0 ? c->ecols : nullptr));
     if (timed) HIPCHK(hipEventRecord(c->ev[e++], c->stream));
     HIPCHK(solar::launch_stage(T, cur, nxt, qw, c->f32, c->gxp, c->gyp, c->gxv, c->gyv, s, dt, 0, c->stream,
                                c->shape, c->c2f, divp ? divp[s] : nullptr, c->div_bits == 32, tl_dc2,
-                               tl_dc2 ? tl_divp[s] : nullptr, c->ecols));
+                               tl_dc2 ? tl_divp[s] : nullptr, c->ecols, 0, nullptr, 0.0, own));
     void* t = cur;
     cur = nxt;
     nxt = t;
@@ -286,6 +290,13 @@ int solar::upload_tables(const Tables& t, DevTables* d, std::vector<void*>* allo
     return rc;
   for (int p = 0; p < 6; ++p)
     for (int e = 0; e < 4; ++e) d->inv_route[p * 4 + e] = t.inv_route[p][e];
+  for (int p = 0; p < 6; ++p) {
+    d->route_bits[p] = 0;
+    for (int e = 0; e < 4; ++e) {
+      const Route& r = t.route[p][e];
+      d->route_bits[p] |= (r.sender << 2 | r.sender_edge | (r.reverse ? 32 : 0)) << (6 * e);
+    }
+  }
   for (int q = 0; q < 7; ++q) {
     d->fcx[q] = t.fcx[q];
     d->fcy[q] = t.fcy[q];

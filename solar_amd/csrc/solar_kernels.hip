@@ -258,6 +258,124 @@ __device__ __forceinline__ void gather_edge(const DevTables& T, int P, int e, in
   }
 }
 
+// Planes whose source strips a tile has in LDS at a time (6x32^2x64 step: 114 us
+// with two, 116 with one).
+constexpr int kGatherPlanes = 2;
+
+// The ghost cells of one stage tile (columns i0.. of wi, rows j0.. of wj) of
+// panel P over planes [k0, k1), p' and the velocity across the edge, by
+// k_gather's expressions in its order: the same bits.  The tile's threads
+// stage the source points of every panel edge the tile's halo crosses -- per
+// edge three lines, as far as the nine-point sums reach -- converted to
+// (p', theta, phi), for NP planes at a time, and each thread whose halo cell (hi, hj)
+// is a ghost (ghost, on edge e) sums its own: ghosts[plane][p', v][thread].
+// What bounds it is latency, so the block's weights load before its strips,
+// and its radial windows after them (held meanwhile they made the rebuilding
+// stage spill: 8.8 -> 13.1 us at 6x16^2x24).  Stage with its ghosts against
+// gather and stage, us: 6x16^2x24 7.2 to 8.8 against 4.4 + 5.5 to 7.4;
+// 6x32^2x64 14 to 20 against 5.3 + 12 to 18; and a launch less.
+//   q, w: the stage's input and, REC, the accumulator it is rebuilt from.
+//   strips: NP x 3 x (staged points) doubles.
+template <typename S, bool REC, int NP>
+__device__ __forceinline__ void gather_tile(const DevTables& T, int P, int i0, int j0, int wi, int wj, int k0, int k1,
+                                            const S* __restrict__ q, const S* w, double betar, int tid, int nth,
+                                            bool ghost, int e, int hi, int hj, double* ghosts, double* strips) {
+  const int n = T.n, nr = T.nr;
+  const size_t plane = (size_t)n * n, nf = plane * nr;
+  // Per edge the tile's ghosts reach (W, E, S, N): the first along-edge index
+  // of its ghosts in the sender's order, and the strip's first point and end
+  // in the list of staged points (empty for the others).
+  const int routes = T.route_bits[P];
+  const bool on[4] = {i0 == 0, i0 + wi + 3 > n, j0 == 0, j0 + wj + 3 > n};
+  int first[4], from[4], start[4], D = 0;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    const int m0 = x < 2 ? j0 : i0, len = x < 2 ? wj : wi;
+    first[x] = routes >> (6 * x) & 32 ? n - m0 - len : m0;
+    from[x] = max(first[x] - 4, 0);
+    start[x] = D;
+    D += on[x] ? 3 * (min(first[x] + len + 4, n) - from[x]) : 0;
+  }
+  if (D == 0) return;  // block-uniform
+  const auto pick = [](const int (&v)[4], int x) { return x == 0 ? v[0] : x == 1 ? v[1] : x == 2 ? v[2] : v[3]; };
+  // this thread's ghost cell: its weights, the staged points they apply to, its transform
+  double wt[9], ab0 = 0.0, ab1 = 0.0;
+  int base = 0, mp = 0;
+  if (ghost) {
+    const int r = routes >> (6 * e);
+    const int lo = e == kW ? -hi - 1 : e == kE ? hi - n : e == kS ? -hj - 1 : hj - n;
+    const int m = e < 2 ? hj : hi;
+    mp = r & 32 ? n - 1 - m : m;
+    base = pick(start, e) + lo - 3 * pick(from, e);
+    const double* g = T.gw + ((size_t)lo * n + mp) * 9;
+#pragma unroll
+    for (int tp = 0; tp < 9; ++tp) wt[tp] = g[tp];
+    const double* abp = T.trans + (((size_t)(r & 31) * 3 + lo) * n + mp) * 2;  // [sender][sender edge][l][m]
+    ab0 = abp[0];
+    ab1 = abp[1];
+  }
+  for (int kg = k0; kg < k1; kg += NP) {
+    if (kg != k0) __syncthreads();  // the strips are read
+    for (int t = tid; t < D; t += nth) {
+      const int x = (t >= start[1]) + (t >= start[2]) + (t >= start[3]);
+      const int u = t - pick(start, x), r = routes >> (6 * x) & 31, sender = r >> 2;
+      const int pidx = strip_index(r & 3, u % 3 + 1, pick(from, x) + u / 3, n);
+      const double* cv = T.conv + ((size_t)(sender < 4 ? 0 : sender - 3) * plane + pidx) * 6;
+      const size_t o = (size_t)sender * 5 * nf + pidx;
+      double c[6];
+#pragma unroll
+      for (int y = 0; y < 6; ++y) c[y] = cv[y];
+      S v[NP][3], vw[NP][3];
+#pragma unroll
+      for (int kk = 0; kk < NP; ++kk) {
+        if (kg + kk >= k1) break;
+        const size_t ok = o + (size_t)(kg + kk) * plane;
+        v[kk][0] = q[ok + 4 * nf];
+        v[kk][1] = q[ok + nf];
+        v[kk][2] = q[ok + 2 * nf];
+        if constexpr (REC) {
+          vw[kk][0] = w[ok + 4 * nf];
+          vw[kk][1] = w[ok + nf];
+          vw[kk][2] = w[ok + 2 * nf];
+        }
+      }
+#pragma unroll
+      for (int kk = 0; kk < NP; ++kk) {
+        if (kg + kk >= k1) break;
+        double d[3];
+#pragma unroll
+        for (int y = 0; y < 3; ++y) {
+          d[y] = static_cast<double>(v[kk][y]);
+          if constexpr (REC) d[y] = d[y] + betar * static_cast<double>(vw[kk][y]);
+        }
+        double* ln = strips + kk * 3 * D + t;
+        ln[0] = d[0];
+        ln[D] = c[0] * (c[1] * d[1] + c[2] * d[2]);
+        ln[2 * D] = c[3] * (c[4] * d[1] + c[5] * d[2]);
+      }
+    }
+    __syncthreads();
+    if (ghost) {
+#pragma unroll
+      for (int kk = 0; kk < NP; ++kk) {
+        if (kg + kk >= k1) break;
+        const double* ln = strips + kk * 3 * D + base;
+        double ps = 0.0, ths = 0.0, phs = 0.0;
+#pragma unroll
+        for (int tp = 0; tp < 9; ++tp) {
+          const int a = 3 * clampi(mp - 4 + tp, 0, n - 1);
+          ps = ps + ln[a] * wt[tp];
+          ths = ths + ln[D + a] * wt[tp];
+          phs = phs + ln[2 * D + a] * wt[tp];
+        }
+        double* g = ghosts + (kg + kk - k0) * 2 * nth + tid;
+        g[0] = ps;
+        g[nth] = ab0 * ths + ab1 * phs;
+      }
+    }
+  }
+}
+
 // blockIdx.x = (chunk of planes)*24 + (receiver panel P)*4 + (receiver edge e);
 // blockIdx.y selects a field offset (the filter's five scalars).
 // The FP32-state vector gather at six waves per SIMD (80 registers, a 12-byte
@@ -298,6 +416,8 @@ struct StageArgs {
   const EnsMember* M;
   const int4* items;
   int nitems, cur, wcur;
+  bool gather;    // host only: the stage is to compute its ghost cells if it can,
+  bool* gathers;  // or (not null): only say whether it can
 };
 
 // Flags of a stage instantiation beyond kStoreNoQ and kStageRecon.
@@ -307,6 +427,14 @@ constexpr int kStageAux = 8;  // c2f or divout is given
 // are non-temporal; kStagePlain: they are not (launch_stage_t).  Partial tiles
 // load plainly either way: they share 128-byte lines with their neighbours.
 constexpr int kStagePlain = 16;
+// The stage computes its tiles' ghost cells itself (gather_tile): no gather
+// launch before it.  Short chunks of planes only (launch_stage_t).
+constexpr int kStageGather = 32;
+// One shell (nr == 1), with kStageGather: the radial windows hold one plane
+// and the LDS tiles one buffer, so 96 registers and 20 KB where there were 130
+// and 40, and the grid is resident at once (us per launch, 6x204^2: first 14.1
+// -> 10.1, rebuilding 19.3 -> 12.8; step 104 -> 77).
+constexpr int kStageShell = 64;
 
 // Reciprocal-based quotients (div_group) in the FP32-state stages only.
 template <typename S>
@@ -317,6 +445,10 @@ constexpr bool kStageRcp = sizeof(S) == 4;
 // measured within 1% of three in every case but one (four, where the divergences
 // are kept, makes the rebuilding stage spill: gradient 218 -> 229 ms).
 constexpr int kStageWaves = 3;
+// Four where a plain stage computes its ghost cells: left alone it takes 130
+// registers, and of blocks of five waves only one fits a CU (6x40^2x30: 19 us
+// a stage against 13).
+constexpr int kGatherWaves = 4;
 
 // One RK stage (or one RHS evaluation, kStageRhs), one pass over HBM.  A
 // block owns a TI x TJ column tile of one panel and marches through a chunk
@@ -369,21 +501,25 @@ constexpr int kStageWaves = 3;
 // two; us per launch in 32x8 tiles, 6x128^2x256: first 558 -> 462, rebuilding
 // 978 -> 902; 6x256^2x384 FP32 state, middle 2866 -> 2661, last 2494 -> 2002.
 template <int TI, int TJ, int KIND, typename S, int MODE = 0, bool PART = false, int FL = 0>
-__global__ __launch_bounds__(TI* TJ) __attribute__((amdgpu_waves_per_eu(kStageWaves)))
+__global__ __launch_bounds__(TI* TJ) __attribute__((amdgpu_waves_per_eu(PART && (FL & kStageGather) && !(FL & kStageRecon) ? kGatherWaves : kStageWaves)))
 void k_stage(StageArgs<S> A) {
   constexpr bool NOQ = (FL & kStoreNoQ) != 0, RECON = (FL & kStageRecon) != 0;
-  constexpr bool STREAM = (FL & kStagePlain) == 0;
+  constexpr bool STREAM = (FL & kStagePlain) == 0, GATH = (FL & kStageGather) != 0;
+  constexpr bool SHELL = (FL & kStageShell) != 0;
   constexpr bool RHS = (FL & kStageRhs) != 0, AUX = (FL & (kStageRhs | kStageAux)) != 0;
   constexpr bool ENS = MODE == 1, TL = MODE == 2, WIDE = sizeof(S) == 8;
   static_assert(!(NOQ || RECON) || (MODE != 2 && WIDE), "the stored-q schedule variants are FP64, not tangent-linear");
   static_assert(!RECON || (KIND == 1 && !NOQ), "a rebuilt input is a middle stage's");
   static_assert(!NOQ || KIND != 2, "the last stage stores q");
+  static_assert(!SHELL || GATH, "a shell's chunk is short");
+  static_assert(!GATH || (MODE == 0 && !AUX && !STREAM), "own ghost cells: plain stages of one grid");
   static_assert(!RHS || (KIND == 0 && MODE == 0 && !NOQ), "an RHS evaluation is of kind 0");
   // halo cells: 6 rows of TI (y), then TJ rows of 6 (x) from a wave boundary on
   constexpr int NT = TI * TJ, NHC = PART ? 1 : ((6 * TI + 63) / 64 * 64 + 6 * TJ + NT - 1) / NT;
-  __shared__ double sp[2][TJ + 6][TI + 6];
-  __shared__ double svx[2][TJ][TI + 6];
-  __shared__ double sve[2][TJ + 6][TI + 6];
+  constexpr int NB = SHELL ? 1 : 2;
+  __shared__ double sp[NB][TJ + 6][TI + 6];
+  __shared__ double svx[NB][TJ][TI + 6];
+  __shared__ double sve[NB][TJ + 6][TI + 6];
 
   const int W = PART ? A.tile_w : TI, HY = (6 * W + 63) / 64 * 64;
   const int tid = PART ? threadIdx.x : threadIdx.y * TI + threadIdx.x;
@@ -489,7 +625,7 @@ void k_stage(StageArgs<S> A) {
 
   // what plane k's start needs, loaded a plane ahead; in the storage type
   // (a conversion at the load would wait for it there)
-  S vx_n, ve_n, pn, rn, hp[NHC], hv[NHC];
+  S vx_n, ve_n, pn = 0, rn = 0, hp[NHC], hv[NHC];
   double gp[NHC] = {}, gv[NHC] = {};
   S w1_n = 0, w2_n = 0, wpn = 0, wrn = 0, rp[NHC] = {}, rv[NHC] = {};  // RECON: qw at the same points
   auto load_start = [&](int k) {
@@ -497,16 +633,18 @@ void k_stage(StageArgs<S> A) {
     const size_t kn = (size_t)min(k + 3, nr - 1) * ps;  // the plane entering the windows before plane k
 #pragma unroll
     for (int c = 0; c < NHC; ++c)
-      if (wave_g[c]) {
+      if (!GATH && wave_g[c]) {
         const size_t kg = (size_t)k * gs;
         const unsigned g = lane_offset(goff[c]);
         gp[c] = load_at<double>((xh[c] ? gxp : gyp) + kg, g);
         gv[c] = load_at<double>((xh[c] ? gxv : gyv) + kg, g);
       }
     const unsigned o = lane_offset(off);
-    pn = load_at<S>(qb + kn + 4 * fs, o);
-    rn = load_at<S>(qb + kn + 3 * fs, o);
-    if constexpr (RECON) {
+    if constexpr (!SHELL) {
+      pn = load_at<S>(qb + kn + 4 * fs, o);
+      rn = load_at<S>(qb + kn + 3 * fs, o);
+    }
+    if constexpr (RECON && !SHELL) {
       wpn = load_at<S>(wb + kn + 4 * fs, o);
       wrn = load_at<S>(wb + kn + 3 * fs, o);
     }
@@ -553,11 +691,22 @@ void k_stage(StageArgs<S> A) {
   double Ci = to_global(ENS ? E.T.ci : A.T.ci)[ic], Dj = to_global(ENS ? E.T.dj : A.T.dj)[jc];
   double dc = to_global(ENS ? E.T.dc : A.T.dc)[cell], tdx = to_global(ENS ? E.T.tdx : A.T.tdx)[cell],
          tde = to_global(ENS ? E.T.tde : A.T.tde)[cell], xy = to_global(ENS ? E.T.xy : A.T.xy)[cell];
+  // GATH: the tile's ghost cells first.
+  extern __shared__ double ghost_lds[];  // ghost values [plane][p', v][thread], then source strips
+  const int nth = PART ? (int)blockDim.x : NT;
+  if constexpr (GATH) {
+    static_assert(NHC == 1, "one halo cell per thread");
+    const int hi = i0 - 3 + hcol[0], hj = j0 - 3 + hrow[0];
+    gather_tile<S, RECON, SHELL ? 1 : kGatherPlanes>(A.T, P, i0, j0, wi, wj, k0, k1, A.qin, A.qw, A.beta_r, tid, nth, hg[0],
+                          hi < 0 ? kW : hi >= n ? kE : hj < 0 ? kS : kN, hi, hj, ghost_lds,
+                          ghost_lds + (size_t)A.kchunk * 2 * nth);
+  }
   // Radial windows of p' and v_r over planes kb..kb+6.
   double pw[7], rw[7];
   int kb = clampi(k0 - 3, 0, nr - 7);
+  const int q0 = SHELL ? 3 : 0, q1 = SHELL ? 4 : 7;  // a shell: slot 3 holds its plane
 #pragma unroll
-  for (int q = 0; q < 7; ++q) {  // (nr == 1, the 2-D case: every slot holds plane 0, with DDR weights 0)
+  for (int q = q0; q < q1; ++q) {  // (nr == 1 otherwise: every slot holds plane 0, with DDR weights 0)
     const size_t kq = (size_t)min(kb + q, nr - 1) * ps;
     pw[q] = load_at<S>(qb + kq + 4 * fs, off);
     rw[q] = load_at<S>(qb + kq + 3 * fs, off);
@@ -572,9 +721,11 @@ void k_stage(StageArgs<S> A) {
   // it are those of its own loads.
   asm volatile("" : "+v"(dc), "+v"(tdx), "+v"(tde), "+v"(xy), "+v"(Ci), "+v"(Dj));
 #pragma unroll
-  for (int q = 0; q < 7; ++q) asm volatile("" : "+v"(pw[q]), "+v"(rw[q]));
-  asm volatile("" : "+v"(pn), "+v"(rn), "+v"(vx_n), "+v"(ve_n));
-  if constexpr (RECON) asm volatile("" : "+v"(wpn), "+v"(wrn), "+v"(w1_n), "+v"(w2_n));
+  for (int q = q0; q < q1; ++q) asm volatile("" : "+v"(pw[q]), "+v"(rw[q]));
+  asm volatile("" : "+v"(vx_n), "+v"(ve_n));
+  if constexpr (!SHELL) asm volatile("" : "+v"(pn), "+v"(rn));
+  if constexpr (RECON) asm volatile("" : "+v"(w1_n), "+v"(w2_n));
+  if constexpr (RECON && !SHELL) asm volatile("" : "+v"(wpn), "+v"(wrn));
 #pragma unroll
   for (int c = 0; c < NHC; ++c) {
     asm volatile("" : "+v"(hp[c]), "+v"(hv[c]), "+v"(gp[c]), "+v"(gv[c]));
@@ -584,7 +735,7 @@ void k_stage(StageArgs<S> A) {
 
   for (int k = k0; k < k1; ++k) {
     const int want = clampi(k - 3, 0, nr - 7);
-    if (want != kb) {  // slides by exactly one plane: plane k+3 enters
+    if (!SHELL && want != kb) {  // slides by exactly one plane: plane k+3 enters
 #pragma unroll
       for (int q = 0; q < 6; ++q) {
         pw[q] = pw[q + 1];
@@ -597,7 +748,7 @@ void k_stage(StageArgs<S> A) {
     // p', v_r at plane k: window slot k - kb, 3 on interior planes
     const int wk = k - kb;
     double pc = pw[3], rc = rw[3];
-    if (wk != 3) {
+    if (!SHELL && wk != 3) {
       asm volatile("");  // stays a branch
 #pragma unroll
       for (int q = 0; q < 7; ++q) {
@@ -605,7 +756,7 @@ void k_stage(StageArgs<S> A) {
         rc = wk == q ? rw[q] : rc;
       }
     }
-    const int bf = k & 1;
+    const int bf = SHELL ? 0 : k & 1;
     const double vx = RECON ? vx_n + A.beta_r * w1_n : vx_n;
     const double ve = RECON ? ve_n + A.beta_r * w2_n : ve_n;
     const S w1 = w1_n, w2 = w2_n;  // RECON: used by the update as well
@@ -620,6 +771,10 @@ void k_stage(StageArgs<S> A) {
       double p = RECON ? hp[c] + A.beta_r * rp[c] : hp[c];
       double v = RECON ? hv[c] + A.beta_r * rv[c] : hv[c];
       if (wave_g[c]) {
+        if constexpr (GATH) {
+          gp[c] = ghost_lds[(k - k0) * 2 * nth + tid];
+          gv[c] = ghost_lds[((k - k0) * 2 + 1) * nth + tid];
+        }
         p = hg[c] ? gp[c] : p;
         v = hg[c] ? gv[c] : v;
       }
@@ -631,7 +786,7 @@ void k_stage(StageArgs<S> A) {
           sve[bf][hrow[c]][hcol[c]] = v;
       }
     }
-    load_start(min(k + 1, k1 - 1));  // the last plane's is loaded and not used
+    if constexpr (!SHELL) load_start(min(k + 1, k1 - 1));  // the last plane's is loaded and not used
     __syncthreads();
 
     // 7-point DRP stencils, ascending taps from 0 (derivative.f90:137-148,
@@ -653,8 +808,10 @@ void k_stage(StageArgs<S> A) {
         dpx = dpx + tap[q] * sp[bf][ty + 3][tx + q];
         dpe = dpe + tap[q] * sp[bf][ty + q][tx + 3];
       }
-      dvr = dvr + row.w[q] * rw[q];
-      dpr = dpr + row.w[q] * pw[q];
+      if (!SHELL || q == 3) {  // (a shell's weights are 0: one product has the value of the seven's sum)
+        dvr = dvr + row.w[q] * rw[q];
+        dpr = dpr + row.w[q] * pw[q];
+      }
     }
 
     // grad.f90:125-133 and :49-57.
@@ -741,7 +898,7 @@ void k_stage(StageArgs<S> A) {
         qn[f] = static_cast<S>(x[f] + A.beta * wd);
         wn[f] = static_cast<S>(wd);
       }
-      load_update(min(k + 1, k1 - 1));
+      if constexpr (!SHELL) load_update(min(k + 1, k1 - 1));
       if (own_in) {
         const auto put = [&](GlobalBytes p, S v) {
           if constexpr (STREAM)
@@ -763,6 +920,7 @@ void k_stage(StageArgs<S> A) {
           if (KIND == 2 || f == 1 || f == 2 || f == 4) store_at(e + (size_t)f * 3 * n * sizeof(S), eo, qn[f]);
       }
     }
+    if constexpr (SHELL) break;
   }
   if constexpr (ENS) __syncthreads();  // the next item rewrites the LDS tiles
   }
@@ -1284,6 +1442,12 @@ constexpr int part_threads(int w, int tj) {
   const int points = (w * tj + 63) / 64 * 64, halo = ((6 * w + 63) / 64 * 64 + 6 * tj + 63) / 64 * 64;
   return points > halo ? points : halo;
 }
+// The longest chunk of planes whose ghost cells a stage computes itself: the
+// LDS that holds them, and the planes in front of which the block stands
+// still, grow with it (us a step, gather launches -> own ghosts: chunks of 1,
+// 6x16^2x24 64 -> 54; 4, 6x32^2x64 129 -> 114; 5, 6x32^2x100 173 -> 160; 8,
+// FP32 state 6x96^2x16 168 -> 174).
+constexpr int kGatherChunk = 6;
 // PART: a.tile_w is the tile width (at most TI).
 template <int TI, int TJ, typename S, bool PART = false>
 static hipError_t launch_stage_t(StageArgs<S> a, int stage, int xf, hipStream_t st, const LaunchShape& ls) {
@@ -1315,15 +1479,36 @@ static hipError_t launch_stage_t(StageArgs<S> a, int stage, int xf, hipStream_t 
   a.alpha = kAlphaRk4[stage < 0 ? 0 : stage];
   a.beta = kBetaRk4[stage < 0 ? 0 : stage];
   const int kind = stage <= 0 ? 0 : (stage < 4 ? 1 : 2);
-#define SOLAR_STAGE_LAUNCH(K, M, FL) hipLaunchKernelGGL((k_stage<TI, TJ, K, S, M, PART, FL>), grid, block, 0, st, a)
+#define SOLAR_STAGE_LAUNCH(K, M, FL) hipLaunchKernelGGL((k_stage<TI, TJ, K, S, M, PART, FL>), grid, block, lds, st, a)
+  // the variants beyond the plain stages: 64x8, 32x8 and 16x16 tiles
+  constexpr bool kMain = (TI == 64 && TJ == 8) || (TI == 32 && TJ == 8) || (TI == 16 && TJ == 16);
+  const bool aux = a.c2f || a.divout;
+  // Stages with their own ghost cells: short chunks on grids whose streams are
+  // plain (there the launch of a gather, 4 to 6 us, is worth more than the
+  // edge blocks' extra work), as long as the LDS leaves as many blocks on a CU
+  // as registers allow and the grid has (6x64^2x48 FP32 state with one block
+  // less: 183 -> 225 us a step).
+  const int nti = (T.n + W - 1) / W, ntj = (T.n + TJ - 1) / TJ;
+  // (a partial tile one short of the last can reach the last's edge too)
+  const size_t strip_points = (nti <= (PART ? 2 : 1) ? 2 : 1) * 3 * (TJ + 8) + (ntj <= (PART ? 2 : 1) ? 2 : 1) * 3 * (W + 8);
+  const size_t tile_lds = sizeof(double) * (T.nr == 1 ? 1 : 2) * (2 * (TJ + 6) + TJ) * (TI + 6);
+  size_t lds = sizeof(double) * ((size_t)a.kchunk * 2 * block.x * block.y +
+                                 (size_t)std::min(a.kchunk, kGatherPlanes) * 3 * strip_points);
+  const int waves = (int)(block.x * block.y + 63) / 64;
+  const int per_cu = std::max(1, std::min(4 * kStageWaves / waves, (tiles * nkch + 255) / 256));
+  const bool gather = kMain && plain && !aux && !a.rhs_mode && !a.tl_dc2 && a.kchunk <= kGatherChunk &&
+                      tile_lds + lds <= 64 * 1024 && (tile_lds + lds + 2048) * per_cu <= 160 * 1024;
+  if (a.gathers) {
+    *a.gathers = gather;
+    return hipSuccess;
+  }
+  if (a.gather && !gather) return hipErrorInvalidValue;
+  if (!a.gather) lds = 0;
   if (a.rhs_mode) {
     if (xf || a.tl_dc2 || a.divout) return hipErrorInvalidValue;
     SOLAR_STAGE_LAUNCH(0, 0, kStageRhs);
     return hipGetLastError();
   }
-  // the variants beyond the plain stages: 64x8, 32x8 and 16x16 tiles
-  constexpr bool kMain = (TI == 64 && TJ == 8) || (TI == 32 && TJ == 8) || (TI == 16 && TJ == 16);
-  const bool aux = a.c2f || a.divout;
   if constexpr (kMain && sizeof(S) == 8) {
     if (xf) {
       if (a.tl_dc2) return hipErrorInvalidValue;
@@ -1336,7 +1521,11 @@ static hipError_t launch_stage_t(StageArgs<S> a, int stage, int xf, hipStream_t 
     SOLAR_STAGE_LAUNCH(1, 0, kStageRecon | (FL));   \
   else                                              \
     return hipErrorInvalidValue;
-      if (aux && plain) {
+      if (a.gather && T.nr == 1) {
+        SOLAR_STAGE_XF(kStageGather | kStagePlain | kStageShell)
+      } else if (a.gather) {
+        SOLAR_STAGE_XF(kStageGather | kStagePlain)
+      } else if (aux && plain) {
         SOLAR_STAGE_XF(kStageAux | kStagePlain)
       } else if (aux) {
         SOLAR_STAGE_XF(kStageAux)
@@ -1369,6 +1558,14 @@ static hipError_t launch_stage_t(StageArgs<S> a, int stage, int xf, hipStream_t 
   else                            \
     SOLAR_STAGE_LAUNCH(2, 0, FL);
   if constexpr (kMain) {
+    if (a.gather && T.nr == 1) {
+      SOLAR_STAGE_KIND(kStageGather | kStagePlain | kStageShell)
+      return hipGetLastError();
+    }
+    if (a.gather) {
+      SOLAR_STAGE_KIND(kStageGather | kStagePlain)
+      return hipGetLastError();
+    }
     if (aux) {
       SOLAR_STAGE_KIND(kStageAux)
       return hipGetLastError();
@@ -1456,10 +1653,28 @@ static StageArgs<S> stage_args(const DevTables& T, const void* qin, void* qout, 
   return a;
 }
 
+bool stage_gathers(const DevTables& T, bool f32, int stage, int xf, const LaunchShape& ls, const double* c2f,
+                   const double* divout, const double* tl_dc2) {
+  bool yes = false;
+  auto ask = [&](auto a) {
+    a.c2f = c2f;
+    a.divout = const_cast<double*>(divout);
+    a.tl_dc2 = tl_dc2;
+    a.gathers = &yes;
+    (void)launch_stage_s(a, stage, xf, nullptr, ls);
+  };
+  if (f32)
+    ask(stage_args<float>(T, nullptr, nullptr, nullptr, nullptr, nullptr));
+  else
+    ask(stage_args<double>(T, nullptr, nullptr, nullptr, nullptr, nullptr));
+  return yes;
+}
+
 hipError_t launch_stage(const DevTables& T, const void* qin, void* qout, void* qw, bool f32, const double* gxp,
                         const double* gyp, const double* gxv, const double* gyv, int stage, double dt, int rhs_mode,
                         hipStream_t st, const LaunchShape& ls, const double* c2f, double* divout, int div32,
-                        const double* tl_dc2, const double* tl_div, void* ecols, int xf, void* qwo, double beta_r) {
+                        const double* tl_dc2, const double* tl_div, void* ecols, int xf, void* qwo, double beta_r,
+                        bool gather) {
   auto go = [&](auto a) {
     a.gxp = gxp;
     a.gyp = gyp;
@@ -1473,6 +1688,7 @@ hipError_t launch_stage(const DevTables& T, const void* qin, void* qout, void* q
     a.div32 = div32;
     a.tl_dc2 = tl_dc2;
     a.tl_div = tl_div;
+    a.gather = gather;
     return launch_stage_s(a, stage, xf, st, ls);
   };
   // (the stored-q schedule variants and the tangent-linear stage are FP64: launch_stage_t refuses others)

@@ -20,6 +20,7 @@ struct DevTables {
   const double* gw;      // gather weights         [3][n][9]
   const double* trans;   // receiver transform     [6][4][3][n][2]
   const Route* route;    // panel routes           [6][4]
+  int route_bits[6];     //   and packed: per edge e of panel P (sender << 2 | sender edge | reverse << 5) << 6 e
   const int* gt_mp;      // transposed gather rows [3][n][kGtWidth]: receiver along index
   const double* gt_w;    //   and weight per entry
   const double* adj_metric;  // adjoint metric factors [n*n][4]
@@ -91,7 +92,12 @@ hipError_t launch_stage(const DevTables& T, const void* qin, void* qout, void* q
                         hipStream_t st, const LaunchShape& ls, const double* c2f = nullptr,
                         double* divout = nullptr, int div32 = 0, const double* tl_dc2 = nullptr,
                         const double* tl_div = nullptr, void* ecols = nullptr, int xf = 0, void* qwo = nullptr,
-                        double beta_r = 0.0);
+                        double beta_r = 0.0, bool gather = false);
+// Whether this stage launch computes the ghost cells of its tiles itself when
+// it is given gather = true (it then reads no ghost strips): grids whose
+// chunks are a few planes.  Any mix of such and other stages is a valid step.
+bool stage_gathers(const DevTables& T, bool f32, int stage, int xf, const LaunchShape& ls, const double* c2f,
+                   const double* divout, const double* tl_dc2);
 hipError_t launch_filter(const DevTables& T, const void* qin, void* qout, bool f32, const double* fgx,
                          const double* fgy, hipStream_t st, const LaunchShape& ls);
 // Ensemble launches.  items: 4 ints per work item, (member, bi | bj << 16,
