@@ -60,11 +60,9 @@ __device__ __forceinline__ unsigned quot_exp(double a) { return (unsigned)(__bui
 // is false) those lanes redo the group by hardware division.  The common
 // path then has no branch per quotient.  Without RCP, hardware division.
 // Measured in one call: the FP32-state step at c3 16.23 -> 16.03 ms against
-// a guard per quotient; the FP64 stages, latency-bound at two waves per
-// SIMD, were no faster at c3 and slower at 6x128^2x256 and 6x96^2x192
-// (+0.5%, +1.6%) than with hardware division, and keep it (a guard per
-// quotient had been slower there too: it drained the prefetch at the
-// loop's back edge).
+// a guard per quotient; the FP64 stages were 0 to 6% slower with it than
+// with hardware division, and keep that (a guard per quotient had been slower
+// there too: it drained the prefetch at the loop's back edge).
 template <bool RCP, int N>
 __device__ __forceinline__ void div_group(const double (&a)[N], const double (&b)[N], const double (&y)[N], bool fast,
                                           double (&q)[N]) {
@@ -1089,10 +1087,10 @@ __device__ __forceinline__ void filter_tile(const DevTables& T, int bi, int bj, 
   // PAIR: a task is two adjacent outputs of one row, read as four aligned
   // 16-byte pairs (eight values for two 7-tap sums), 22 x 16 tasks for a
   // 32 x 16 tile: half the LDS reads of one output per thread (FP32 filter
-  // at c3 2.79 -> 2.61 ms).  The FP64 filter takes pairs on panels up to
-  // 128 (filter 6x128^2x256 -3%, 6x96^2x192 -7%, the ensemble step -0.8%)
-  // and one output per thread on larger ones (6x256^2x384: 2.93 -> 3.14 ms
-  // with pairs).
+  // at c3 2.79 -> 2.61 ms).  With one row per thread the FP64 filter takes
+  // pairs on panels up to 128 (filter 6x128^2x256 -3%, 6x96^2x192 -7%, the
+  // ensemble step -0.8%) and one output per thread on larger ones
+  // (6x256^2x384: 2.93 -> 3.14 ms with pairs).
   typedef double dpair __attribute__((ext_vector_type(2)));  // one 16-byte LDS access
   auto xi_pass = [&]() {
     if constexpr (!PAIR) {
