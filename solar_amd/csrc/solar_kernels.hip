@@ -942,8 +942,8 @@ struct FilterLds {
 // and tile cells beyond the panel's three ghost layers stay 0.
 // PAIR: FILTER_XI tasks of two adjacent outputs (below).  R: adjacent rows
 // per thread (blocks of TI x TJ / R), whose FILTER_ETA sums share R + 6 reads
-// where single rows take 7 each.
-template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4), int R = 1>
+// where single rows take 7 each.  SHELL: nr == 1, the 2-D case.
+template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4), int R = 1, bool SHELL = false>
 __device__ __forceinline__ void filter_tile(const DevTables& T, int bi, int bj, int PF, int k0, int k1,
                                             const S* __restrict__ qin, S* __restrict__ qout,
                                             const double* __restrict__ fgx, const double* __restrict__ fgy,
@@ -972,16 +972,15 @@ __device__ __forceinline__ void filter_tile(const DevTables& T, int bi, int bj, 
   const double* gyS = fgy + F * fstride + (size_t)(P * 2) * gy_side;
   const size_t ij = own_in[0] ? (size_t)j * n + i : 0;
 
-  // 2-D case (nr == 1): FILTER_R returns its input (filter.f90:647-650)
-  const bool twod = nr == 1;
-  // filter.f90:652,726-777: the five planes at each end are zero.
-  if (!twod)
+  // filter.f90:652,726-777: the five planes at each end are zero; in the 2-D
+  // case FILTER_R returns its input (filter.f90:647-650).
+  if constexpr (!SHELL)
     for (int k = k0; k < k1; ++k)
       if (k < kNstr || k >= nr - kNstr)
 #pragma unroll
         for (int r = 0; r < R; ++r)
           if (own_in[r]) o[(size_t)k * plane + ij + (size_t)r * n] = static_cast<S>(0.0);
-  const int a = twod ? 0 : max(k0, kNstr), bnd = twod ? 1 : min(k1, nr - kNstr);
+  const int a = SHELL ? 0 : max(k0, kNstr), bnd = SHELL ? 1 : min(k1, nr - kNstr);
   if (a >= bnd) return;
 
   // Tile cells this thread fills: kind 1 a field cell, 2 a ghost-strip cell,
@@ -1140,7 +1139,7 @@ __device__ __forceinline__ void filter_tile(const DevTables& T, int bi, int bj, 
     }
   };
 
-  if (twod) {  // the one plane: FILTER_XI, FILTER_ETA, stored as they come
+  if constexpr (SHELL) {  // the one plane: FILTER_XI, FILTER_ETA, stored as they come
     FPlane p0;
     load_plane(0, p0);
 #pragma unroll
@@ -1239,8 +1238,8 @@ __device__ __forceinline__ void filter_tile(const DevTables& T, int bi, int bj, 
 template <int TI, int TJ, typename S, int R>
 constexpr int filter_waves() { return R > 1 ? 4 : (sizeof(S) == 4 && TI * TJ >= 256 && !(TI == 64 && TJ == 4) && !(TI == 32 && TJ == 8)) ? 6 : 1; }
 
-template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4), int R = 1>
-__global__ __launch_bounds__(TI* TJ / R) __attribute__((amdgpu_waves_per_eu(filter_waves<TI, TJ, S, R>())))
+template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4), int R = 1, bool SHELL = false>
+__global__ __launch_bounds__(TI* TJ / R) __attribute__((amdgpu_waves_per_eu(SHELL ? 1 : filter_waves<TI, TJ, S, R>())))
 void k_filter(DevTables T, const S* __restrict__ qin,
                                                     S* __restrict__ qout, const double* __restrict__ fgx,
                                                     const double* __restrict__ fgy, int kchunk, int nkch) {
@@ -1258,7 +1257,7 @@ void k_filter(DevTables T, const S* __restrict__ qin,
   const int k0 = ch * kchunk;
   const int k1 = min(k0 + kchunk, nr);
   if (k0 >= nr) return;
-  filter_tile<TI, TJ, S, PART, PAIR, R>(T, bi, bj, PF, k0, k1, qin, qout, fgx, fgy, lds);
+  filter_tile<TI, TJ, S, PART, PAIR, R, SHELL>(T, bi, bj, PF, k0, k1, qin, qout, fgx, fgy, lds);
 }
 
 // Ensemble FILTER_EXP: work items (member, tile, 5P+F, plane range), q[cur] -> q[1-cur].
@@ -1693,7 +1692,7 @@ hipError_t launch_stage(const DevTables& T, const void* qin, void* qout, void* q
   return f32 ? go(stage_args<float>(T, qin, qout, qw, qwo, ecols)) : go(stage_args<double>(T, qin, qout, qw, qwo, ecols));
 }
 
-template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4), int R = 1>
+template <int TI, int TJ, typename S, bool PART = false, bool PAIR = (sizeof(S) == 4), int R = 1, bool SHELL = false>
 static hipError_t launch_filter_t(const DevTables& T, const S* qin, S* qout, const double* fgx, const double* fgy,
                                   hipStream_t st, const LaunchShape& ls) {
   const int tiles = ((T.n + TI - 1) / TI) * ((T.n + TJ - 1) / TJ) * 30;
@@ -1708,7 +1707,7 @@ static hipError_t launch_filter_t(const DevTables& T, const S* qin, S* qout, con
   if (ls.filter_chunks > 0) nkch = ls.filter_chunks;
   const int kchunk = (T.nr + nkch - 1) / nkch;
   dim3 grid(tiles * nkch), block(TI, TJ / R);
-  hipLaunchKernelGGL((k_filter<TI, TJ, S, PART, PAIR, R>), grid, block, 0, st, T, qin, qout, fgx, fgy, kchunk, nkch);
+  hipLaunchKernelGGL((k_filter<TI, TJ, S, PART, PAIR, R, SHELL>), grid, block, 0, st, T, qin, qout, fgx, fgy, kchunk, nkch);
   return hipGetLastError();
 }
 
@@ -1717,6 +1716,12 @@ static hipError_t launch_filter_s(const DevTables& T, const S* qin, S* qout, con
                                   hipStream_t st, const LaunchShape& ls) {
   // FILTER_XI in paired tasks: always for an FP32 state, for FP64 on panels up to 128
   const bool pair = sizeof(S) == 4 || T.n <= 128;
+  // One shell: no radial sums, so 28 registers instead of 76 and eight waves
+  // per SIMD; the smallest tiles fill the chip best (us, 6x204^2: 15.8 -> 13.6,
+  // 32 wide 14.9, 64 wide 17.9; 6x300^2 26.2 -> 21.5; 6x512^2 52.3 -> 48.3).
+  if (T.nr == 1)
+    return T.n % 16 ? launch_filter_t<16, 16, S, true, true, 1, true>(T, qin, qout, fgx, fgy, st, ls)
+                    : launch_filter_t<16, 16, S, false, true, 1, true>(T, qin, qout, fgx, fgy, st, ls);
   if (T.n % 16 != 0) {  // partial tiles
     if (pad_pick_ti(T.n) == 32)
       return pair ? launch_filter_t<32, 16, S, true, true>(T, qin, qout, fgx, fgy, st, ls)
