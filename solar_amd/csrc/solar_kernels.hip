@@ -439,7 +439,7 @@ template <typename S>
 constexpr bool kStageRcp = sizeof(S) == 4;
 
 // Occupancy floor of the stage kernel in waves per SIMD.  Every variant takes
-// 111 to 145 registers and none spills at three; floors of two and four
+// 96 to 167 registers and none spills at three; floors of two and four
 // measured within 1% of three in every case but one (four, where the divergences
 // are kept, makes the rebuilding stage spill: gradient 218 -> 229 ms).
 constexpr int kStageWaves = 3;
