@@ -27,6 +27,7 @@
 
 #include "solar_device.hpp"
 #include "solar_kernels.hpp"
+#include "solar_tiles.hpp"
 
 namespace solar {
 
@@ -59,13 +60,15 @@ __device__ __forceinline__ unsigned quot_exp(double a) { return (unsigned)(__bui
 // sequence; in a wave where some lane's numerators fail the test (or fast
 // is false) those lanes redo the group by hardware division.  The common
 // path then has no branch per quotient.  Without RCP, hardware division.
+// live: the lane's quotients are used (lanes of a partial tile without a point
+// of their own divide what their cells happen to hold).
 // Measured in one call: the FP32-state step at c3 16.23 -> 16.03 ms against
 // a guard per quotient; the FP64 stages were 0 to 6% slower with it than
 // with hardware division, and keep that (a guard per quotient had been slower
 // there too: it drained the prefetch at the loop's back edge).
 template <bool RCP, int N>
 __device__ __forceinline__ void div_group(const double (&a)[N], const double (&b)[N], const double (&y)[N], bool fast,
-                                          double (&q)[N]) {
+                                          bool live, double (&q)[N]) {
   if constexpr (!RCP) {
 #pragma unroll
     for (int t = 0; t < N; ++t) q[t] = a[t] / b[t];
@@ -77,7 +80,7 @@ __device__ __forceinline__ void div_group(const double (&a)[N], const double (&b
     q[t] = quot_rcp(a[t], b[t], y[t]);
     m = max(m, quot_exp(a[t]));
   }
-  const bool slow = !fast || m > 1800u;
+  const bool slow = live && (!fast || m > 1800u);
   if (__builtin_expect(__ballot(slow) != 0, 0)) {
     if (slow) {
 #pragma unroll
@@ -474,7 +477,9 @@ constexpr int kGatherWaves = 4;
 //   PART: the tiles are tile_w <= TI wide, any width, and need not divide n;
 //   the block is one-dimensional.  In the last tile of a row or column the E
 //   (N) halo cells begin at the panel edge, inside the tile; threads without a
-//   point of their own load through an in-panel point and write nothing.
+//   point of their own (beyond the panel, or surplus in the block, part_point)
+//   load through an in-panel point, read cells of the LDS tiles and write
+//   nothing.
 //
 // What bounds it.  At 6x256^2x384 a march of as many streams, with no
 // arithmetic, in the same tiles reaches 4.8 to 5.0 TB/s on this card (one shot
@@ -521,7 +526,8 @@ void k_stage(StageArgs<S> A) {
 
   const int W = PART ? A.tile_w : TI, HY = (6 * W + 63) / 64 * 64;
   const int tid = PART ? threadIdx.x : threadIdx.y * TI + threadIdx.x;
-  const int tx = PART ? tid % W : threadIdx.x, ty = PART ? tid / W : threadIdx.y;
+  const PartPoint pt = PART ? part_point(tid, W, TJ) : PartPoint{(int)threadIdx.x, (int)threadIdx.y, true};
+  const int tx = pt.tx, ty = pt.ty;
   const int wave0 = __builtin_amdgcn_readfirstlane(tid & ~63);  // this wave's first thread
 
   const int n_items = ENS ? A.nitems : 1;
@@ -557,7 +563,7 @@ void k_stage(StageArgs<S> A) {
                c6 = ENS ? E.T.fcx[6] : A.T.fcx[6];
   const int i0 = bi * W, j0 = bj * TJ, i = i0 + tx, j = j0 + ty;
   const int wi = PART ? min(W, n - i0) : TI, wj = PART ? min(TJ, n - j0) : TJ;  // the tile inside the panel
-  const bool own_in = !PART || (tx < wi && ty < wj);
+  const bool own_in = !PART || (pt.own && tx < wi && ty < wj);
   const int ic = PART ? min(i, n - 1) : i, jc = PART ? min(j, n - 1) : j;
   const size_t plane = (size_t)n * n, nf = plane * nr;
   const unsigned cell = (unsigned)(jc * n + ic), off = cell * (unsigned)sizeof(S);
@@ -822,7 +828,7 @@ void k_stage(StageArgs<S> A) {
       const double na[7] = {dvx, dve, 2.0 * rc, xy * dpe, xy * dpx, dpr, q1 * row.g0};
       const double ba[7] = {Ci, Dj, row.r, Dj, Ci, row.rho0, row.rho0};
       const double ya[7] = {yCi, yDj, row.inv_r, yDj, yCi, row.inv_rho0, row.inv_rho0};
-      div_group<kStageRcp<S>>(na, ba, ya, fdiv, qa);
+      div_group<kStageRcp<S>>(na, ba, ya, fdiv, own_in, qa);
     }
     const double div = (row.inv_r * ((dc * (qa[0] + qa[1]) - tdx * vx) - tde * ve) + dvr) + qa[2];
     const double gxi = row.inv_r * (Dj * dpx + qa[3]);
@@ -836,7 +842,7 @@ void k_stage(StageArgs<S> A) {
       const double nb[2] = {gxi, get};
       const double bb[2] = {row.rho0, row.rho0};
       const double yb[2] = {row.inv_rho0, row.inv_rho0};
-      div_group<kStageRcp<S>>(nb, bb, yb, fdiv, qc);
+      div_group<kStageRcp<S>>(nb, bb, yb, fdiv, own_in, qc);
     }
     double r2 = -qc[0];
     double r3 = -qc[1];
@@ -1433,12 +1439,6 @@ hipError_t launch_gather(const DevTables& T, const void* q, bool f32, bool vec, 
                          gxs, gys, gxv, gyv, st, static_cast<const double*>(qwr), betar);
 }
 
-// Threads of a stage block with tiles of width w: its points, and its halo
-// cells (6 w above and below, filled up to a wave, and 6 tj beside).
-constexpr int part_threads(int w, int tj) {
-  const int points = (w * tj + 63) / 64 * 64, halo = ((6 * w + 63) / 64 * 64 + 6 * tj + 63) / 64 * 64;
-  return points > halo ? points : halo;
-}
 // The longest chunk of planes whose ghost cells a stage computes itself: the
 // LDS that holds them, and the planes in front of which the block stands
 // still, grow with it (us a step, gather launches -> own ghosts: chunks of 1,
@@ -1585,28 +1585,6 @@ static hipError_t launch_stage_t(StageArgs<S> a, int stage, int xf, hipStream_t 
 // shape divides n (n not a multiple of 16), the partial-tile kernels run with
 // 32-wide or 16-wide tiles, whichever pads n less (ties to 32).
 static bool fits(int n, int ti, int tj) { return ti > 0 && tj > 0 && n % ti == 0 && n % tj == 0; }
-// Width of a partial-tile panel's stage tiles: from 64 down to 33, the one
-// that leaves the fewest lanes without a point, the widest of near equals (us
-// per stage, 6x200^2x150: 40 wide 1177, 50 1432, 34 1608, 16x16 tiles 1240;
-// 6x250^2x60: 63 wide 771, 50 856, 42 895).  Multiples of 8 where the rows
-// are.  One shell makes too few blocks to fill the chip: there the narrowest
-// of near equals, down to 26 (6x204^2: 30 wide 19.9, 51 22.8; 6x250^2: 32 wide
-// 24.2, 63 26.2).
-static int part_width(int n, int nr) {
-  const int narrow = nr == 1 ? 26 : 33;
-  int best = 0;
-  double least = 0.0;
-  for (int t = (n + 63) / 64; t <= (n + narrow - 1) / narrow || t == (n + 63) / 64; ++t) {
-    int w = (n + t - 1) / t;
-    if (n % 8 == 0) w = (w + 7) / 8 * 8;
-    const double lanes = (double)part_threads(w, 8) * t;
-    if (least == 0.0 || lanes < (nr == 1 ? 1.03 : 0.97) * least) {
-      least = lanes;
-      best = w;
-    }
-  }
-  return best;
-}
 static int pad_pick_ti(int n) { return ((n + 31) / 32) * 32 <= ((n + 15) / 16) * 16 ? 32 : 16; }
 
 template <typename S>
