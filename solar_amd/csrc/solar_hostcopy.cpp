@@ -23,6 +23,30 @@ constexpr int kThreads = 4;
 constexpr size_t kPiece = size_t(4) << 20;
 constexpr size_t kLeast = size_t(32) << 20;  // below, starting the threads costs more than it gives
 
+// Makes `device` current for the calling thread while it lives: events belong
+// to the device that is current when they are made, and the caller's comes back.
+class OnDevice {
+ public:
+  explicit OnDevice(int device) {
+    int cur = -1;
+    status_ = hipGetDevice(&cur);
+    if (status_ == hipSuccess && cur != device) {
+      status_ = hipSetDevice(device);
+      if (status_ == hipSuccess) back_ = cur;
+    }
+  }
+  ~OnDevice() {
+    if (back_ >= 0) (void)hipSetDevice(back_);
+  }
+  OnDevice(const OnDevice&) = delete;
+  OnDevice& operator=(const OnDevice&) = delete;
+  hipError_t status() const { return status_; }
+
+ private:
+  hipError_t status_;
+  int back_ = -1;
+};
+
 }  // namespace
 
 struct HostCopy::Staging {
@@ -46,7 +70,8 @@ HostCopy::~HostCopy() { delete s_; }
 
 // One thread's part: pieces in order, alternating between the two buffers.
 hipError_t HostCopy::part(int t, char* host, char* dev, size_t bytes, bool down, int device, hipStream_t st) {
-  hipError_t e = hipSetDevice(device);
+  const OnDevice on(device);
+  hipError_t e = on.status();
   const size_t np = (bytes + kPiece - 1) / kPiece;
   char* buf[2] = {s_->buf + (2 * t) * kPiece, s_->buf + (2 * t + 1) * kPiece};
   auto size = [&](size_t p) { return std::min(kPiece, bytes - p * kPiece); };
@@ -81,6 +106,11 @@ hipError_t HostCopy::run(void* host, void* dev, size_t bytes, bool down, int dev
     return e == hipSuccess ? hipStreamSynchronize(st) : e;
   };
   if (bytes < kLeast) return plain();
+  const OnDevice on(device);
+  if (on.status() != hipSuccess) {
+    (void)hipGetLastError();
+    return plain();
+  }
   if (!s_) {
     Staging* s = new (std::nothrow) Staging();
     if (!s || s->make() != hipSuccess) {

@@ -1,0 +1,60 @@
+// Checks of solar_hostcopy.cpp on the CPU (hip_stub.hpp); the argument names
+// one, the exit status is 0 if it holds.
+#include "hip_stub.hpp"
+#include "solar_internal.hpp"
+
+#include <cstdio>
+#include <functional>
+#include <string>
+#include <vector>
+
+namespace {
+
+constexpr size_t kBytes = (size_t(41) << 20) + 24;  // above the staging's least size, no whole pieces
+
+int failures = 0;
+void check(bool ok, const char* what) {
+  if (ok) return;
+  std::printf("failed: %s\n", what);
+  ++failures;
+}
+
+struct Arrays {
+  std::vector<char> src, dst;
+  void* dev = nullptr;
+  explicit Arrays(char seed, size_t bytes = kBytes) : src(bytes), dst(bytes) {
+    for (size_t x = 0; x < bytes; ++x) src[x] = static_cast<char>(x * 7 + x / 4096 + seed);
+    (void)hipMalloc(&dev, bytes);
+  }
+  ~Arrays() { (void)hipFree(dev); }
+  bool round_trip(solar::HostCopy& h, int device = 0) {
+    const hipStream_t st = stub::stream_of(device);
+    if (h.to_device(dev, src.data(), src.size(), device, st) != hipSuccess) return false;
+    if (h.to_host(dst.data(), dev, dst.size(), device, st) != hipSuccess) return false;
+    return src == dst;
+  }
+};
+
+// A handle of another device than the caller's current one.
+void other_device() {
+  solar::HostCopy h;
+  Arrays a(1);
+  stub::device = 0;
+  check(a.round_trip(h, 1), "copies for device 1 while device 0 is current");
+  check(stub::device == 0, "the caller's current device stays");
+  check(hipGetLastError() == hipSuccess, "no error left behind");
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::vector<std::pair<std::string, std::function<void()>>> all = {
+      {"other_device", other_device},
+  };
+  for (const auto& c : all)
+    if (argc == 2 && c.first == argv[1]) {
+      c.second();
+      return failures != 0;
+    }
+  return 2;
+}
