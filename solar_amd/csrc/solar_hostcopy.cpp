@@ -1,6 +1,8 @@
 // Large copies between pageable host memory and the device.
 //
-// A caller's array is pageable and often fresh: the runtime's own copy of
+// An array that the runtime knows (pinned, managed, a device's) is copied by it
+// alone: staged, 35 MB of pinned memory took 1.0 ms instead of 0.63, 1 GB 21.5
+// instead of 17.5.  A caller's array is mostly pageable and often fresh: the runtime's own copy of
 // 830 MB into new arrays runs at 9 GB/s, one thread faulting their pages in.
 // Here a few threads each take a contiguous part of the array through two
 // pinned pieces of their own: while one piece is on the link, the other is
@@ -46,6 +48,14 @@ class OnDevice {
   hipError_t status_;
   int back_ = -1;
 };
+
+// Whether the runtime can put the memory at p on the link as it is.
+bool runtime_knows(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+  (void)hipGetLastError();  // an ordinary array
+  return false;
+}
 
 }  // namespace
 
@@ -105,7 +115,7 @@ hipError_t HostCopy::run(void* host, void* dev, size_t bytes, bool down, int dev
                               : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
     return e == hipSuccess ? hipStreamSynchronize(st) : e;
   };
-  if (bytes < kLeast) return plain();
+  if (bytes < kLeast || runtime_knows(host)) return plain();
   const OnDevice on(device);
   if (on.status() != hipSuccess) {
     (void)hipGetLastError();

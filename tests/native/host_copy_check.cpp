@@ -45,11 +45,38 @@ void other_device() {
   check(hipGetLastError() == hipSuccess, "no error left behind");
 }
 
+// Host arrays that are pinned, or memory of a device: the runtime copies those
+// by itself, in one piece.
+void known_memory() {
+  solar::HostCopy h;
+  Arrays a(2);
+  void* mem[2] = {nullptr, nullptr};
+  (void)hipHostMalloc(&mem[0], kBytes, 0);
+  (void)hipMalloc(&mem[1], kBytes);
+  for (void* p : mem) {
+    const size_t from = 4096;  // the middle of the allocation
+    stub::watch = static_cast<char*>(p) + from;
+    stub::watch_bytes = kBytes - from;
+    std::memcpy(static_cast<char*>(p) + from, a.src.data(), kBytes - from);
+    stub::copies = stub::direct = 0;
+    check(h.to_device(a.dev, stub::watch, kBytes - from, 0, stub::stream_of(0)) == hipSuccess, "to the device");
+    check(stub::copies == 1 && stub::direct == 1, "one copy from the array itself");
+    std::memset(static_cast<char*>(p) + from, 0, kBytes - from);
+    check(h.to_host(static_cast<char*>(p) + from, a.dev, kBytes - from, 0, stub::stream_of(0)) == hipSuccess, "back");
+    check(stub::copies == 2 && stub::direct == 2, "one copy into the array itself");
+    check(std::memcmp(stub::watch, a.src.data(), kBytes - from) == 0, "the same bytes");
+  }
+  stub::watch = nullptr;
+  (void)hipHostFree(mem[0]);
+  (void)hipFree(mem[1]);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::vector<std::pair<std::string, std::function<void()>>> all = {
       {"other_device", other_device},
+      {"known_memory", known_memory},
   };
   for (const auto& c : all)
     if (argc == 2 && c.first == argv[1]) {
