@@ -66,8 +66,10 @@ struct HostCopy::Staging {
 
   hipError_t make() {
     hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&buf), kThreads * 2 * kPiece, hipHostMallocDefault);
-    for (int x = 0; x < 2 * kThreads && e == hipSuccess; ++x, ++made)
-      e = hipEventCreateWithFlags(&ev[x / 2][x % 2], hipEventDisableTiming);
+    while (made < 2 * kThreads && e == hipSuccess) {
+      e = hipEventCreateWithFlags(&ev[made / 2][made % 2], hipEventDisableTiming);
+      if (e == hipSuccess) ++made;
+    }
     return e;
   }
   ~Staging() {
@@ -124,8 +126,8 @@ hipError_t HostCopy::run(void* host, void* dev, size_t bytes, bool down, int dev
   if (!s_) {
     Staging* s = new (std::nothrow) Staging();
     if (!s || s->make() != hipSuccess) {
-      (void)hipGetLastError();
       delete s;
+      (void)hipGetLastError();  // no failure of the staging for a later launch to report
       return plain();
     }
     s_ = s;

@@ -71,12 +71,28 @@ void known_memory() {
   (void)hipFree(mem[1]);
 }
 
+// The staging cannot be made: the copy goes on without it, and nothing of the
+// failure stays behind.
+void events_fail() {
+  for (int k : {0, 3, 7}) {
+    solar::HostCopy h;
+    Arrays a(3);
+    stub::fail_event = k;
+    check(a.round_trip(h), "copies while an event creation fails");
+    check(hipGetLastError() == hipSuccess, "no error left for the next launch to report");
+    stub::fail_event = -1;
+    check(a.round_trip(h), "copies afterwards");
+  }
+  check(stub::events.empty() && stub::pinned.empty(), "everything is given back");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::vector<std::pair<std::string, std::function<void()>>> all = {
       {"other_device", other_device},
       {"known_memory", known_memory},
+      {"events_fail", events_fail},
   };
   for (const auto& c : all)
     if (argc == 2 && c.first == argv[1]) {
