@@ -13,7 +13,6 @@
 #include <algorithm>
 #include <cstring>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -142,7 +141,7 @@ hipError_t HostCopy::run(void* host, void* dev, size_t bytes, bool down, int dev
   for (int t = 1; t < kThreads; ++t) {
     try {
       th[t] = std::thread(work, t);
-    } catch (const std::system_error&) {  // no thread to be had: this one does the part
+    } catch (...) {  // no thread to be had, or no memory for it: this one does the part
       work(t);
     }
   }

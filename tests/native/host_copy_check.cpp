@@ -5,8 +5,19 @@
 
 #include <cstdio>
 #include <functional>
+#include <new>
 #include <string>
 #include <vector>
+
+// Allocations of this thread until one fails (once).
+static thread_local int fail_new = -1;
+void* operator new(size_t n) {
+  if (fail_new >= 0 && fail_new-- == 0) throw std::bad_alloc();
+  if (void* p = std::malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 namespace {
 
@@ -86,6 +97,22 @@ void events_fail() {
   check(stub::events.empty() && stub::pinned.empty(), "everything is given back");
 }
 
+// No memory for a thread's record: the calling thread does that part itself.
+void no_thread() {
+  solar::HostCopy h;
+  Arrays a(4);
+  check(a.round_trip(h), "with threads");
+  for (int k = 0; k < 3; ++k) {
+    fail_new = k;
+    check(h.to_device(a.dev, a.src.data(), kBytes, 0, stub::stream_of(0)) == hipSuccess, "to the device");
+    fail_new = k;
+    check(h.to_host(a.dst.data(), a.dev, kBytes, 0, stub::stream_of(0)) == hipSuccess, "back");
+    fail_new = -1;
+    check(a.src == a.dst, "the same bytes");
+    std::fill(a.dst.begin(), a.dst.end(), 0);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -93,6 +120,7 @@ int main(int argc, char** argv) {
       {"other_device", other_device},
       {"known_memory", known_memory},
       {"events_fail", events_fail},
+      {"no_thread", no_thread},
   };
   for (const auto& c : all)
     if (argc == 2 && c.first == argv[1]) {
