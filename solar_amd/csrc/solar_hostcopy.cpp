@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <thread>
 #include <vector>
@@ -117,6 +118,8 @@ hipError_t HostCopy::run(void* host, void* dev, size_t bytes, bool down, int dev
     return e == hipSuccess ? hipStreamSynchronize(st) : e;
   };
   if (bytes < kLeast || runtime_knows(host)) return plain();
+  const std::unique_lock<std::mutex> lock(mu_, std::try_to_lock);
+  if (!lock) return plain();  // another thread's copy has the staging
   const OnDevice on(device);
   if (on.status() != hipSuccess) {
     (void)hipGetLastError();

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime_api.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -26,8 +27,8 @@ hipError_t scratch_address(int device, void** addr);
 
 // Copies between a caller's host array and the device, synchronous, ordered
 // after the work on `st` (solar_hostcopy.cpp).  Large ones go through pinned
-// staging that the object makes on the first of them and keeps (32 MiB); it is
-// for one thread at a time, as the handle that owns it.
+// staging that the object makes on the first of them and keeps (32 MiB); a copy
+// that comes while another thread's has the staging goes without it.
 class HostCopy {
  public:
   HostCopy() = default;
@@ -44,6 +45,7 @@ class HostCopy {
  private:
   struct Staging;
   Staging* s_ = nullptr;
+  std::mutex mu_;  // held by the copy that uses s_
   hipError_t run(void* host, void* dev, size_t bytes, bool down, int device, hipStream_t st);
   hipError_t part(int t, char* host, char* dev, size_t bytes, bool down, int device, hipStream_t st);
 };

@@ -7,6 +7,7 @@
 #include <functional>
 #include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 // Allocations of this thread until one fails (once).
@@ -113,6 +114,30 @@ void no_thread() {
   }
 }
 
+// A second thread's copy in the middle of the first one's, on the same object.
+solar::HostCopy* shared_copy;
+Arrays* shared_array;
+bool shared_ok;
+void copy_meanwhile() {
+  std::thread([] { shared_ok = shared_array->round_trip(*shared_copy); }).join();
+}
+void two_threads() {
+  solar::HostCopy h;
+  Arrays a(5), b(6);
+  check(a.round_trip(h), "alone");
+  shared_copy = &h;
+  shared_array = &b;
+  for (int down = 0; down < 2; ++down) {
+    shared_ok = false;
+    stub::on_copy = copy_meanwhile;
+    std::memset(down ? static_cast<void*>(a.dst.data()) : a.dev, 0, kBytes);
+    check((down ? h.to_host(a.dst.data(), a.dev, kBytes, 0, stub::stream_of(0))
+                : h.to_device(a.dev, a.src.data(), kBytes, 0, stub::stream_of(0))) == hipSuccess, "the first copy");
+    check(std::memcmp(down ? static_cast<void*>(a.dst.data()) : a.dev, a.src.data(), kBytes) == 0, "the first array is whole");
+    check(shared_ok, "the second array is whole");
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -121,6 +146,7 @@ int main(int argc, char** argv) {
       {"known_memory", known_memory},
       {"events_fail", events_fail},
       {"no_thread", no_thread},
+      {"two_threads", two_threads},
   };
   for (const auto& c : all)
     if (argc == 2 && c.first == argv[1]) {
