@@ -11,7 +11,6 @@
 #include <cstring>
 #include <map>
 #include <mutex>
-#include <set>
 
 namespace stub {
 
@@ -20,6 +19,12 @@ inline thread_local hipError_t pending = hipSuccess;
 inline std::mutex mu;
 inline std::map<const char*, size_t> pinned, on_device;  // allocations: address, size
 inline std::map<hipEvent_t, int> events;                 // device of each
+// what was asked of the streams, in order: kinds of copies, kWait
+constexpr int kWait = -1;
+inline int asked[1024], n_asked = 0;
+inline void ask(int what) {
+  if (n_asked < 1024) asked[n_asked++] = what;
+}
 inline std::atomic<int> copies{0}, direct{0};  // all copies; those from or to the array `watch`
 inline const char* watch = nullptr;
 inline size_t watch_bytes = 0;
@@ -100,8 +105,12 @@ inline __attribute__((used)) hipError_t hipEventRecord(hipEvent_t e, hipStream_t
   return hipSuccess;
 }
 inline __attribute__((used)) hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-inline __attribute__((used)) hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-inline __attribute__((used)) hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+inline __attribute__((used)) hipError_t hipStreamSynchronize(hipStream_t) {
+  std::lock_guard<std::mutex> l(stub::mu);
+  stub::ask(stub::kWait);
+  return hipSuccess;
+}
+inline __attribute__((used)) hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind kind, hipStream_t) {
   std::memcpy(d, s, n);
   ++stub::copies;
   const auto in = [](const void* p) {
@@ -112,6 +121,7 @@ inline __attribute__((used)) hipError_t hipMemcpyAsync(void* d, const void* s, s
   void (*f)() = nullptr;
   {
     std::lock_guard<std::mutex> l(stub::mu);
+    stub::ask(kind);
     std::swap(f, stub::on_copy);
   }
   if (f) f();

@@ -3,6 +3,7 @@
 #include "hip_stub.hpp"
 #include "solar_internal.hpp"
 
+#include <algorithm>
 #include <cstdio>
 #include <functional>
 #include <new>
@@ -138,6 +139,22 @@ void two_threads() {
   }
 }
 
+// Before its pieces, a staged copy waits for the stream and sends two small
+// uploads, each waited for.
+void settled_stream() {
+  solar::HostCopy h;
+  Arrays a(7);
+  check(a.round_trip(h), "a first round trip");
+  for (bool down : {true, false}) {
+    stub::n_asked = 0;
+    check((down ? h.to_host(a.dst.data(), a.dev, kBytes, 0, stub::stream_of(0))
+                : h.to_device(a.dev, a.src.data(), kBytes, 0, stub::stream_of(0))) == hipSuccess, "a copy");
+    const int want[] = {stub::kWait, hipMemcpyHostToDevice, stub::kWait, hipMemcpyHostToDevice, stub::kWait};
+    check(stub::n_asked > 5 && std::equal(want, want + 5, stub::asked),
+          "wait, upload, wait, upload, wait");
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -147,6 +164,7 @@ int main(int argc, char** argv) {
       {"events_fail", events_fail},
       {"no_thread", no_thread},
       {"two_threads", two_threads},
+      {"settled_stream", settled_stream},
   };
   for (const auto& c : all)
     if (argc == 2 && c.first == argv[1]) {
