@@ -27,7 +27,7 @@ hipError_t scratch_address(int device, void** addr);
 
 // Copies between a caller's host array and the device, synchronous, ordered
 // after the work on `st` (solar_hostcopy.cpp).  Large ones go through pinned
-// staging that the object makes on the first of them and keeps (32 MiB); a copy
+// staging (32 MiB) that the object makes when they are worth it and keeps; a copy
 // that comes while another thread's has the staging goes without it.
 class HostCopy {
  public:
@@ -45,7 +45,8 @@ class HostCopy {
  private:
   struct Staging;
   Staging* s_ = nullptr;
-  std::mutex mu_;  // held by the copy that uses s_
+  size_t owed_ = 0;  // bytes of plain copies that the staging would have sped up, weighted
+  std::mutex mu_;  // held by the copy that uses them
   hipError_t run(void* host, void* dev, size_t bytes, bool down, int device, hipStream_t st);
   hipError_t part(int t, char* host, char* dev, size_t bytes, bool down, int device, hipStream_t st);
 };

@@ -40,6 +40,8 @@ struct Arrays {
     (void)hipMalloc(&dev, bytes);
   }
   ~Arrays() { (void)hipFree(dev); }
+  // two of them have the staging made
+  bool round_trips(solar::HostCopy& h, int device = 0) { return round_trip(h, device) && round_trip(h, device); }
   bool round_trip(solar::HostCopy& h, int device = 0) {
     const hipStream_t st = stub::stream_of(device);
     if (h.to_device(dev, src.data(), src.size(), device, st) != hipSuccess) return false;
@@ -53,7 +55,7 @@ void other_device() {
   solar::HostCopy h;
   Arrays a(1);
   stub::device = 0;
-  check(a.round_trip(h, 1), "copies for device 1 while device 0 is current");
+  check(a.round_trips(h, 1) && a.round_trip(h, 1), "copies for device 1 while device 0 is current");
   check(stub::device == 0, "the caller's current device stays");
   check(hipGetLastError() == hipSuccess, "no error left behind");
 }
@@ -91,10 +93,10 @@ void events_fail() {
     solar::HostCopy h;
     Arrays a(3);
     stub::fail_event = k;
-    check(a.round_trip(h), "copies while an event creation fails");
+    check(a.round_trips(h), "copies while an event creation fails");
     check(hipGetLastError() == hipSuccess, "no error left for the next launch to report");
     stub::fail_event = -1;
-    check(a.round_trip(h), "copies afterwards");
+    check(a.round_trips(h), "copies afterwards");
   }
   check(stub::events.empty() && stub::pinned.empty(), "everything is given back");
 }
@@ -103,7 +105,7 @@ void events_fail() {
 void no_thread() {
   solar::HostCopy h;
   Arrays a(4);
-  check(a.round_trip(h), "with threads");
+  check(a.round_trips(h), "with threads");
   for (int k = 0; k < 3; ++k) {
     fail_new = k;
     check(h.to_device(a.dev, a.src.data(), kBytes, 0, stub::stream_of(0)) == hipSuccess, "to the device");
@@ -125,7 +127,7 @@ void copy_meanwhile() {
 void two_threads() {
   solar::HostCopy h;
   Arrays a(5), b(6);
-  check(a.round_trip(h), "alone");
+  check(a.round_trips(h), "alone");
   shared_copy = &h;
   shared_array = &b;
   for (int down = 0; down < 2; ++down) {
@@ -144,7 +146,7 @@ void two_threads() {
 void settled_stream() {
   solar::HostCopy h;
   Arrays a(7);
-  check(a.round_trip(h), "a first round trip");
+  check(a.round_trips(h), "round trips");
   for (bool down : {true, false}) {
     stub::n_asked = 0;
     check((down ? h.to_host(a.dst.data(), a.dev, kBytes, 0, stub::stream_of(0))
@@ -153,6 +155,35 @@ void settled_stream() {
     check(stub::n_asked > 5 && std::equal(want, want + 5, stub::asked),
           "wait, upload, wait, upload, wait");
   }
+}
+
+// The staging is made when copies without it have cost about as much as making
+// it does, not by the first of them.
+void first_copy() {
+  for (bool down : {false, true}) {
+    solar::HostCopy h;
+    Arrays a(8);
+    char* host = down ? a.dst.data() : a.src.data();
+    stub::watch = host;
+    stub::watch_bytes = kBytes;
+    int plain = 0;
+    for (; plain < 100; ++plain) {
+      stub::direct = 0;
+      check((down ? h.to_host(host, a.dev, kBytes, 0, stub::stream_of(0))
+                  : h.to_device(a.dev, host, kBytes, 0, stub::stream_of(0))) == hipSuccess, "a copy");
+      if (stub::direct == 0) break;
+    }
+    check(plain >= 1, "the first copy of a new object goes without the staging");
+    check(plain <= (down ? 2 : 12), "many copies make it");
+    stub::watch = nullptr;
+  }
+  solar::HostCopy h;
+  Arrays a(9, size_t(90) << 20);
+  stub::watch = a.dst.data();
+  stub::watch_bytes = a.dst.size();
+  stub::direct = 0;
+  check(h.to_host(a.dst.data(), a.dev, a.dst.size(), 0, stub::stream_of(0)) == hipSuccess, "a large download");
+  check(stub::direct == 0, "a download that pays for the staging by itself makes it");
 }
 
 }  // namespace
@@ -165,6 +196,7 @@ int main(int argc, char** argv) {
       {"no_thread", no_thread},
       {"two_threads", two_threads},
       {"settled_stream", settled_stream},
+      {"first_copy", first_copy},
   };
   for (const auto& c : all)
     if (argc == 2 && c.first == argv[1]) {

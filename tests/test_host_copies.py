@@ -19,7 +19,7 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("case", ["other_device", "known_memory", "events_fail", "no_thread", "two_threads", "settled_stream"])
+@pytest.mark.parametrize("case", ["other_device", "known_memory", "events_fail", "no_thread", "two_threads", "settled_stream", "first_copy"])
 def test_host_copy(program, case):
     r = subprocess.run([program, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
