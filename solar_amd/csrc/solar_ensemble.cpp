@@ -61,6 +61,7 @@ struct solar_ens {
     int chunks = 0;  // radial chunks per receiver edge
   };
   std::vector<GatherGroup> gg;
+  bool stored_q = false;  // the stored-q schedule (every member has its second accumulator)
   int gchunks = 0;  // > 0: the chunks of every group (launch-shape sweeps)
   int persist = 0;   // > 0: grid cap of the work-list launches
   std::vector<void*> allocs;
@@ -184,20 +185,25 @@ int build_lists(solar_ens* e) {
 // ecols, from which the next gather reads its column strips (compact lines
 // instead of three values from every row of the state); the step's first
 // gather reads the filtered state.
-// The stages run the stored-q schedule of the single grid: q is stored after
-// stages 2, 4 and 5 only, and stages 2 and 4 rebuild their input as q + beta
-// qw (48 members as the batched workload draws them: 35.3 -> 32.9 ms per step, with
-// the gather chunks below).
+// With a second accumulator the stages run the stored-q schedule of the single
+// grid: q is stored after stages 2, 4 and 5 only, and stages 2 and 4 rebuild
+// their input as q + beta qw (48 members as the batched workload draws them:
+// 35.3 -> 32.9 ms per step, with the gather chunks below).  Without one, q is
+// stored after every stage; the same bits.
 int enqueue_step(solar_ens* e) {
   // q and qw buffer of each stage's input
-  static const int kQ[5] = {0, 0, 1, 1, 0}, kW[5] = {0, 0, 1, 1, 0};
+  static const int kStoredQ[5] = {0, 0, 1, 1, 0}, kStoredW[5] = {0, 0, 1, 1, 0};
+  static const int kAllQ[5] = {0, 1, 0, 1, 0}, kAllW[5] = {0, 0, 0, 0, 0};
+  const int* const kQ = e->stored_q ? kStoredQ : kAllQ;
+  const int* const kW = e->stored_q ? kStoredW : kAllW;
   for (int s = 0; s < 5; ++s) {
-    const bool rebuilt = s == 1 || s == 3;
+    const bool rebuilt = e->stored_q && (s == 1 || s == 3);
     for (const auto& G : e->gg)
       ENSCHK(solar::launch_gather_ens(e->dmem, G.table, G.nm, G.nblocks, G.n, true, kQ[s], s > 0, G.chunks, e->stream,
                                       rebuilt ? kW[s] : -1, rebuilt ? solar::kBetaRk4[s - 1] : 0.0));
     for (const Launch& L : e->stage_l)
-      ENSCHK(solar::launch_stage_ens(e->dmem, L.items, L.nitems, L.grid, L.ti, L.tj, s, kQ[s], kW[s], e->stream));
+      ENSCHK(solar::launch_stage_ens(e->dmem, L.items, L.nitems, L.grid, L.ti, L.tj, s, kQ[s], kW[s], e->stored_q,
+                                     e->stream));
   }
   for (const auto& G : e->gg)
     ENSCHK(solar::launch_gather_ens(e->dmem, G.table, G.nm, G.nblocks, G.n, false, 1, true, G.chunks, e->stream));
@@ -212,10 +218,42 @@ int clear_state(solar_ens* e) {
     ENSCHK(hipMemsetAsync(e->mem[m].q[0], 0, b, e->stream));
     ENSCHK(hipMemsetAsync(e->mem[m].q[1], 0, b, e->stream));
     ENSCHK(hipMemsetAsync(e->mem[m].qw[0], 0, b, e->stream));
-    ENSCHK(hipMemsetAsync(e->mem[m].qw[1], 0, b, e->stream));
+    if (e->mem[m].qw[1]) ENSCHK(hipMemsetAsync(e->mem[m].qw[1], 0, b, e->stream));
   }
   ENSCHK(hipStreamSynchronize(e->stream));
   return SOLAR_OK;
+}
+
+// The members' second accumulators, one more state's worth each.  Taken where
+// they leave at least as much device memory free as they need, for what the
+// program allocates after them: an ensemble that nearly fills the card is made
+// without them, as is one under SOLAR_STEP_STORE_ALL.
+void add_accumulators(solar_ens* e) {
+  const char* all = std::getenv("SOLAR_STEP_STORE_ALL");
+  if (all && all[0] && std::strcmp(all, "0") != 0) return;
+  std::vector<size_t> size(e->nm);
+  size_t total = 0, freeb = 0, cap = 0;
+  for (int m = 0; m < e->nm; ++m)
+    total += size[m] = static_cast<size_t>(e->n[m]) * e->n[m] * e->nr[m] * 30 * sizeof(double);
+  if (hipMemGetInfo(&freeb, &cap) != hipSuccess || total > freeb / 2) {
+    (void)hipGetLastError();
+    return;
+  }
+  std::vector<void*> got;
+  for (int m = 0; m < e->nm; ++m) {
+    void* p = nullptr;
+    if (hipMalloc(&p, size[m]) != hipSuccess) break;
+    got.push_back(p);
+  }
+  if (got.size() < static_cast<size_t>(e->nm)) {  // in pieces the memory was not to be had
+    for (void* p : got) (void)hipFree(p);
+    (void)hipGetLastError();
+    return;
+  }
+  for (int m = 0; m < e->nm; ++m) e->mem[m].qw[1] = static_cast<double*>(got[m]);
+  e->allocs.insert(e->allocs.end(), got.begin(), got.end());
+  e->bytes += total;
+  e->stored_q = true;
 }
 
 // Mean time (ms) of reps launches of `launch` on the ensemble's stream.
@@ -289,9 +327,9 @@ int solar_ens_create(solar_ens** out, int nmembers, const int* n, const int* nr,
     if (rc) return bail(rc);
     const size_t nq = static_cast<size_t>(n[m]) * n[m] * nr[m] * 30;
     const size_t ng = static_cast<size_t>(12) * nr[m] * n[m] * 3;
-    void* p[11];
-    const size_t sz[11] = {nq, nq, nq, nq, ng, ng, ng, ng, 5 * ng, 5 * ng, solar::edge_cols_elems(n[m], nr[m])};
-    for (int a = 0; a < 11; ++a) {
+    void* p[10];
+    const size_t sz[10] = {nq, nq, nq, ng, ng, ng, ng, 5 * ng, 5 * ng, solar::edge_cols_elems(n[m], nr[m])};
+    for (int a = 0; a < 10; ++a) {
       if ((rc = ens_alloc(e, &p[a], sz[a] * sizeof(double), &e->allocs))) return bail(rc);
       if (hipMemset(p[a], 0, sz[a] * sizeof(double)) != hipSuccess)
         return bail(solar::set_error(SOLAR_ERR_HIP, "solar_ens_create: hipMemset failed"));
@@ -299,14 +337,14 @@ int solar_ens_create(solar_ens** out, int nmembers, const int* n, const int* nr,
     M.q[0] = static_cast<double*>(p[0]);
     M.q[1] = static_cast<double*>(p[1]);
     M.qw[0] = static_cast<double*>(p[2]);
-    M.qw[1] = static_cast<double*>(p[3]);
-    M.gxp = static_cast<double*>(p[4]);
-    M.gyp = static_cast<double*>(p[5]);
-    M.gxv = static_cast<double*>(p[6]);
-    M.gyv = static_cast<double*>(p[7]);
-    M.fgx = static_cast<double*>(p[8]);
-    M.fgy = static_cast<double*>(p[9]);
-    M.ecols = static_cast<double*>(p[10]);
+    M.qw[1] = nullptr;  // add_accumulators
+    M.gxp = static_cast<double*>(p[3]);
+    M.gyp = static_cast<double*>(p[4]);
+    M.gxv = static_cast<double*>(p[5]);
+    M.gyv = static_cast<double*>(p[6]);
+    M.fgx = static_cast<double*>(p[7]);
+    M.fgy = static_cast<double*>(p[8]);
+    M.ecols = static_cast<double*>(p[9]);
     M.dt = dt[m];
     e->choice[m] = default_choice(n[m], nr[m]);
   }
@@ -314,8 +352,6 @@ int solar_ens_create(solar_ens** out, int nmembers, const int* n, const int* nr,
   int rc;
   if ((rc = ens_alloc(e, &d, nmembers * sizeof(EnsMember), &e->allocs))) return bail(rc);
   e->dmem = static_cast<EnsMember*>(d);
-  if (hipMemcpy(e->dmem, e->mem.data(), nmembers * sizeof(EnsMember), hipMemcpyHostToDevice) != hipSuccess)
-    return bail(solar::set_error(SOLAR_ERR_HIP, "solar_ens_create: member table upload failed"));
   std::map<int, std::vector<int>> by_n;
   for (int m = 0; m < nmembers; ++m) by_n[n[m]].push_back(m);
   for (auto& kv : by_n) {
@@ -341,6 +377,9 @@ int solar_ens_create(solar_ens** out, int nmembers, const int* n, const int* nr,
     e->gg.push_back(G);
   }
   if ((rc = build_lists(e))) return bail(rc);
+  add_accumulators(e);
+  if (hipMemcpy(e->dmem, e->mem.data(), nmembers * sizeof(EnsMember), hipMemcpyHostToDevice) != hipSuccess)
+    return bail(solar::set_error(SOLAR_ERR_HIP, "solar_ens_create: member table upload failed"));
   if ((rc = clear_state(e))) return bail(rc);
   *out = e;
   solar::clear_error();
@@ -396,7 +435,8 @@ int solar_ens_autotune(solar_ens* e, int reps) {
         if ((rc = make_launch(e, sh[0], sh[1], items, &L))) return rc;
         float ms = 0.f;
         if ((rc = time_launch(e, reps, [&]() {
-               return solar::launch_stage_ens(e->dmem, L.items, L.nitems, L.grid, L.ti, L.tj, 1, 0, 0, e->stream);
+               return solar::launch_stage_ens(e->dmem, L.items, L.nitems, L.grid, L.ti, L.tj, 1, 0, 0, e->stored_q,
+                                             e->stream);
              }, &ms)))
           return rc;
         if (ms < best_s) {

@@ -1772,7 +1772,7 @@ hipError_t launch_place(const double* src, void* dst, bool f32, size_t nf, int d
 
 template <int TI, int TJ>
 static hipError_t launch_stage_ens_t(const EnsMember* M, const int4* items, int nitems, int grid, int stage, int cur,
-                                     int wcur, hipStream_t st) {
+                                     int wcur, bool stored_q, hipStream_t st) {
   StageArgs<double> a{};
   a.alpha = kAlphaRk4[stage];
   a.beta = kBetaRk4[stage];
@@ -1783,7 +1783,11 @@ static hipError_t launch_stage_ens_t(const EnsMember* M, const int4* items, int 
   a.cur = cur;
   a.wcur = wcur;
   const dim3 g(grid), block(TI, TJ);
-  if (stage == 0)
+  if (!stored_q && stage == 0)
+    hipLaunchKernelGGL((k_stage<TI, TJ, 0, double, 1>), g, block, 0, st, a);
+  else if (!stored_q && stage < 4)
+    hipLaunchKernelGGL((k_stage<TI, TJ, 1, double, 1>), g, block, 0, st, a);
+  else if (stage == 0)
     hipLaunchKernelGGL((k_stage<TI, TJ, 0, double, 1, false, kStoreNoQ>), g, block, 0, st, a);
   else if (stage == 2)
     hipLaunchKernelGGL((k_stage<TI, TJ, 1, double, 1, false, kStoreNoQ>), g, block, 0, st, a);
@@ -1795,13 +1799,13 @@ static hipError_t launch_stage_ens_t(const EnsMember* M, const int4* items, int 
 }
 
 hipError_t launch_stage_ens(const EnsMember* M, const int* items, int nitems, int grid, int ti, int tj, int stage,
-                            int cur, int wcur, hipStream_t st) {
+                            int cur, int wcur, bool stored_q, hipStream_t st) {
   const int4* it = reinterpret_cast<const int4*>(items);
   if (nitems <= 0) return hipSuccess;
   if (stage < 0 || stage > 4) return hipErrorInvalidValue;
-  if (ti == 64 && tj == 8) return launch_stage_ens_t<64, 8>(M, it, nitems, grid, stage, cur, wcur, st);
-  if (ti == 32 && tj == 8) return launch_stage_ens_t<32, 8>(M, it, nitems, grid, stage, cur, wcur, st);
-  if (ti == 16 && tj == 16) return launch_stage_ens_t<16, 16>(M, it, nitems, grid, stage, cur, wcur, st);
+  if (ti == 64 && tj == 8) return launch_stage_ens_t<64, 8>(M, it, nitems, grid, stage, cur, wcur, stored_q, st);
+  if (ti == 32 && tj == 8) return launch_stage_ens_t<32, 8>(M, it, nitems, grid, stage, cur, wcur, stored_q, st);
+  if (ti == 16 && tj == 16) return launch_stage_ens_t<16, 16>(M, it, nitems, grid, stage, cur, wcur, stored_q, st);
   return hipErrorInvalidValue;
 }
 

@@ -31,7 +31,8 @@ struct DevTables {
 };
 
 // One member of a batched ensemble (FP64): its tables, state ping-pong
-// buffers, the two 2N accumulators of the stored-q schedule, ghost strips, edge-column copies (written by
+// buffers, the two 2N accumulators of the stored-q schedule (the second null
+// where q is stored after every stage), ghost strips, edge-column copies (written by
 // every stage, read by the next gather, edge_cols_elems(n, nr) values) and
 // time step.
 struct EnsMember {
@@ -103,12 +104,12 @@ hipError_t launch_filter(const DevTables& T, const void* qin, void* qout, bool f
 // Ensemble launches.  items: 4 ints per work item, (member, bi | bj << 16,
 // P (stage) or 5P+F (filter) | k0 << 8, k1); grid blocks walk the list with a
 // grid-sized stride.  Stage ti x tj in {64x8, 32x8, 16x16}, filter in
-// {32x16, 16x16, 32x8}.  The state goes from M.q[cur] to M.q[1-cur].  The
-// stages run the stored-q schedule (kStoreNoQ for stages 0 and 2, kStageRecon
-// for 1 and 3): qw is read from M.qw[wcur], and a rebuilding stage writes its
-// own to M.qw[1-wcur].
+// {32x16, 16x16, 32x8}.  The state goes from M.q[cur] to M.q[1-cur].  With
+// stored_q the stages run that schedule (kStoreNoQ for stages 0 and 2,
+// kStageRecon for 1 and 3): qw is read from M.qw[wcur], and a rebuilding stage
+// writes its own to M.qw[1-wcur].
 hipError_t launch_stage_ens(const EnsMember* M, const int* items, int nitems, int grid, int ti, int tj, int stage,
-                            int cur, int wcur, hipStream_t st);
+                            int cur, int wcur, bool stored_q, hipStream_t st);
 hipError_t launch_filter_ens(const EnsMember* M, const int* items, int nitems, int grid, int ti, int tj, int cur,
                              hipStream_t st);
 // A gather over a group of members: table[x] = first block of the group's
