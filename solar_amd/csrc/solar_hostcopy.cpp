@@ -25,13 +25,14 @@ constexpr int kThreads = 4;
 constexpr size_t kPiece = size_t(4) << 20;
 constexpr size_t kSettle = size_t(64) << 10;
 constexpr size_t kLeast = size_t(32) << 20;  // below, starting the threads costs more than it gives
-// Making the staging costs up to 4.2 ms (pinning 32 MiB; less where the runtime
-// has such memory left over), and it saves 0.012 ms a MB to the device and 0.07
-// from it.  So the copies of an object that has none yet are counted, each by
-// what the staging would have saved, and the one that brings them to this many
-// bytes to the device makes it.  First copies of a process, made at once and
-// now: 35 MB to the device 4.5 -> 1.8 ms, 126 MB 6.6 -> 5.0, as the runtime's.
-constexpr size_t kMake = size_t(384) << 20, kDownWeight = 6;
+// A new staging costs about 3.4 ms, for the page faults of its first use (less
+// where the runtime has such memory left over from another handle), and saves
+// 0.012 ms a MB to the device and 0.07 from it.  So the first copy of an object
+// makes it only where that copy pays for it; a second one shows a program that
+// goes on copying.  First copies of a process, made at once and now: 35 MB to
+// the device 4.5 -> 1.8 ms, 126 MB 6.6 -> 5.0, 35 MB from it 11.7 -> 4.3, as the
+// runtime's own.
+constexpr size_t kPaysUp = size_t(320) << 20, kPaysDown = size_t(56) << 20;
 
 // Makes `device` current for the calling thread while it lives: events belong
 // to the device that is current when they are made, and the caller's comes back.
@@ -153,8 +154,9 @@ hipError_t HostCopy::run(void* host, void* dev, size_t bytes, bool down, int dev
     return plain();
   }
   if (!s_) {
-    owed_ += down ? kDownWeight * bytes : bytes;
-    if (owed_ < kMake) return plain();
+    const bool first = !copied_;
+    copied_ = true;
+    if (first && bytes < (down ? kPaysDown : kPaysUp)) return plain();
     Staging* s = new (std::nothrow) Staging();
     if (!s || s->make() != hipSuccess) {
       delete s;

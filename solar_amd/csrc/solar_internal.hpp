@@ -45,7 +45,7 @@ class HostCopy {
  private:
   struct Staging;
   Staging* s_ = nullptr;
-  size_t owed_ = 0;  // bytes of plain copies that the staging would have sped up, weighted
+  bool copied_ = false;  // there was a large copy
   std::mutex mu_;  // held by the copy that uses them
   hipError_t run(void* host, void* dev, size_t bytes, bool down, int device, hipStream_t st);
   hipError_t part(int t, char* host, char* dev, size_t bytes, bool down, int device, hipStream_t st);
