@@ -2,8 +2,9 @@
 //
 // An array that the runtime knows (pinned, managed, a device's) is copied by it
 // alone: staged, 35 MB of pinned memory took 1.0 ms instead of 0.63, 1 GB 21.5
-// instead of 17.5.  A caller's array is mostly pageable and often fresh: the runtime's own copy of
-// 830 MB into new arrays runs at 9 GB/s, one thread faulting their pages in.
+// instead of 17.5.  A caller's array is mostly pageable and often fresh: the
+// runtime's own copy of 830 MB into new arrays runs at 9 GB/s, one thread
+// faulting their pages in.
 // Here a few threads each take a contiguous part of the array through two
 // pinned pieces of their own: while one piece is on the link, the other is
 // copied to or from the array.  Measured on 830 MB of ensemble states: into

@@ -425,8 +425,9 @@ struct StageArgs {
 constexpr int kStageRhs = 4;  // evaluates the RHS alone (rhs_mode holds its flags), KIND 0
 constexpr int kStageAux = 8;  // c2f or divout is given
 // The streams that no other block reads (q and qw stores; rho' and qw loads)
-// are non-temporal; kStagePlain: they are not (launch_stage_t).  Partial tiles
-// load plainly either way: they share 128-byte lines with their neighbours.
+// are non-temporal; kStagePlain: they are not (launch_stage_t; single grids, and
+// with a c^2 field or kept divergences only the stored-q variants).  Partial
+// tiles load plainly either way: they share 128-byte lines with their neighbours.
 constexpr int kStagePlain = 16;
 // The stage computes its tiles' ghost cells itself (gather_tile): no gather
 // launch before it.  Short chunks of planes only (launch_stage_t).
@@ -444,11 +445,13 @@ constexpr bool kStageRcp = sizeof(S) == 4;
 // Occupancy floor of the stage kernel in waves per SIMD.  Every variant takes
 // 96 to 167 registers and none spills at three; floors of two and four
 // measured within 1% of three in every case but one (four, where the divergences
-// are kept, makes the rebuilding stage spill: gradient 218 -> 229 ms).
+// are kept, makes the rebuilding stage spill: gradient 218 -> 229 ms).  The
+// partial tiles' own-ghost stages run at four (below).
 constexpr int kStageWaves = 3;
-// Four where a plain stage computes its ghost cells: left alone it takes 130
-// registers, and of blocks of five waves only one fits a CU (6x40^2x30: 19 us
-// a stage against 13).
+// Four where a partial tile's stage computes its ghost cells (the rebuilding one
+// aside): left alone it takes 130 registers, and of blocks of five waves only one
+// fits a CU (6x40^2x30: 19 us a stage against 13, which a spill of 12 to 16 bytes
+// a lane is in).
 constexpr int kGatherWaves = 4;
 
 // One RK stage (or one RHS evaluation, kStageRhs), one pass over HBM.  A
@@ -481,11 +484,13 @@ constexpr int kGatherWaves = 4;
 //   load through an in-panel point, read cells of the LDS tiles and write
 //   nothing.
 //
-// What bounds it.  At 6x256^2x384 a march of as many streams, with no
-// arithmetic, in the same tiles reaches 4.8 to 5.0 TB/s on this card (one shot
-// over the same streams: 5.5); the five FP64 stages move their 640 bytes a
-// point at 4.8.  On small grids it is the instructions issued per point and
-// plane.  So
+// What bounds it.  Memory on large grids: at 6x256^2x384 the five FP64 stages
+// move their 640 bytes a point at 4.96 TB/s (first 4.76, rebuilding 4.88, third
+// 5.24, last 5.05; 6x128^2x256 4.64, 4.62, 5.11, 5.03).  A march of 10, 15 or 20
+// streams with no arithmetic, plane by plane in the same tiles, moves 4.8 (4.9 at
+// 6x128^2x256) whatever their number, and one shot over the streams 5.5: the
+// march is no ceiling, and what keeps either from 5.5 is not known.  On small
+// grids it is the instructions issued per point and plane.  So
 //   - every access is a wave-uniform base plus a 32-bit lane offset;
 //   - a halo cell is loaded by one thread (y halos by the first waves, x
 //     halos by the next, so which of v_xi and v_eta a wave needs is uniform);
@@ -1462,7 +1467,9 @@ static hipError_t launch_stage_t(StageArgs<S> a, int stage, int xf, hipStream_t 
   if (tiles * nkch < 1536) nkch = small_grid_chunks(tiles, T.nr, 1.0, 3, 1.25);
   if (ls.stage_chunks > 0) nkch = ls.stage_chunks;
   // Non-temporal streams, but not where the step's buffers stay in the 256 MB
-  // last-level cache between launches (stream_past_cache), and in partial
+  // last-level cache between launches (stream_past_cache; the stages without a
+  // plain form stay non-temporal there: the last of a step that keeps
+  // divergences or has a c^2 field, every FP32-state one with a field), and in partial
   // tiles only where rows and tiles are of whole 64-byte segments: else a
   // neighbouring tile completes the segment in L2 (stage, 6x204^2x100: 1.03 ->
   // 0.95 ms; with whole segments, 6x200^2x150, plain stores are slower: 1.17 ->
