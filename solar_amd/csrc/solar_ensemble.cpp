@@ -65,6 +65,7 @@ struct solar_ens {
   int gchunks = 0;  // > 0: the chunks of every group (launch-shape sweeps)
   int persist = 0;   // > 0: grid cap of the work-list launches
   std::vector<void*> allocs;
+  std::vector<void*> second;  // the members' second accumulators
   std::vector<void*> list_allocs;  // work lists, rebuilt by the autotuner
   size_t bytes = 0;
   int device = 0;
@@ -92,10 +93,19 @@ void drop_graph(solar_ens* e) {
   e->graph = nullptr;
 }
 
+void free_second(solar_ens* e) {
+  for (size_t m = 0; m < e->second.size(); ++m) {
+    (void)hipFree(e->second[m]);
+    e->bytes -= static_cast<size_t>(e->n[m]) * e->n[m] * e->nr[m] * 30 * sizeof(double);
+  }
+  e->second.clear();
+}
+
 void release(solar_ens* e) {
   drop_graph(e);
   for (void* p : e->list_allocs) (void)hipFree(p);
   for (void* p : e->allocs) (void)hipFree(p);
+  free_second(e);
   if (e->stream) (void)hipStreamDestroy(e->stream);
   e->list_allocs.clear();
   e->allocs.clear();
@@ -224,36 +234,25 @@ int clear_state(solar_ens* e) {
   return SOLAR_OK;
 }
 
-// The members' second accumulators, one more state's worth each.  Taken where
-// they leave at least as much device memory free as they need, for what the
-// program allocates after them: an ensemble that nearly fills the card is made
-// without them, as is one under SOLAR_STEP_STORE_ALL.
-void add_accumulators(solar_ens* e) {
+// Whether the members get second accumulators, one more state's worth each:
+// where these leave at least as much device memory free as they need, for what
+// the program allocates after them.  An ensemble that nearly fills the card is
+// made without them, as is one under SOLAR_STEP_STORE_ALL.
+bool room_for_second(const solar_ens* e) {
   const char* all = std::getenv("SOLAR_STEP_STORE_ALL");
-  if (all && all[0] && std::strcmp(all, "0") != 0) return;
-  std::vector<size_t> size(e->nm);
-  size_t total = 0, freeb = 0, cap = 0;
-  for (int m = 0; m < e->nm; ++m)
-    total += size[m] = static_cast<size_t>(e->n[m]) * e->n[m] * e->nr[m] * 30 * sizeof(double);
-  if (hipMemGetInfo(&freeb, &cap) != hipSuccess || total > freeb / 2) {
-    (void)hipGetLastError();
-    return;
-  }
-  std::vector<void*> got;
+  if (all && all[0] && std::strcmp(all, "0") != 0) return false;
+  size_t state = 0, rest = 0, freeb = 0, cap = 0;
   for (int m = 0; m < e->nm; ++m) {
-    void* p = nullptr;
-    if (hipMalloc(&p, size[m]) != hipSuccess) break;
-    got.push_back(p);
+    if (e->n[m] < 1 || e->nr[m] < 1) return false;  // refused below
+    const size_t n = e->n[m], nr = e->nr[m];
+    state += n * n * nr * 30 * sizeof(double);
+    rest += (14 * 36 * n * nr + solar::edge_cols_elems(e->n[m], e->nr[m])) * sizeof(double);  // ghosts, edge columns
   }
-  if (got.size() < static_cast<size_t>(e->nm)) {  // in pieces the memory was not to be had
-    for (void* p : got) (void)hipFree(p);
+  if (hipMemGetInfo(&freeb, &cap) != hipSuccess) {
     (void)hipGetLastError();
-    return;
+    return false;
   }
-  for (int m = 0; m < e->nm; ++m) e->mem[m].qw[1] = static_cast<double*>(got[m]);
-  e->allocs.insert(e->allocs.end(), got.begin(), got.end());
-  e->bytes += total;
-  e->stored_q = true;
+  return 5 * state + rest <= freeb;
 }
 
 // Mean time (ms) of reps launches of `launch` on the ensemble's stream.
@@ -306,6 +305,7 @@ int solar_ens_create(solar_ens** out, int nmembers, const int* n, const int* nr,
     if (c >= 1 && c <= 64) e->gchunks = c;
   }
   if (hipStreamCreate(&e->stream) != hipSuccess) return bail(solar::set_error(SOLAR_ERR_HIP, "hipStreamCreate failed"));
+  e->stored_q = room_for_second(e);
   size_t roff = 0;
   for (int m = 0; m < nmembers; ++m) {
     if (!(dt[m] > 0.0))
@@ -327,31 +327,45 @@ int solar_ens_create(solar_ens** out, int nmembers, const int* n, const int* nr,
     if (rc) return bail(rc);
     const size_t nq = static_cast<size_t>(n[m]) * n[m] * nr[m] * 30;
     const size_t ng = static_cast<size_t>(12) * nr[m] * n[m] * 3;
-    void* p[10];
-    const size_t sz[10] = {nq, nq, nq, ng, ng, ng, ng, 5 * ng, 5 * ng, solar::edge_cols_elems(n[m], nr[m])};
-    for (int a = 0; a < 10; ++a) {
-      if ((rc = ens_alloc(e, &p[a], sz[a] * sizeof(double), &e->allocs))) return bail(rc);
+    void* p[11];
+    const size_t sz[11] = {nq, nq, nq, nq, ng, ng, ng, ng, 5 * ng, 5 * ng, solar::edge_cols_elems(n[m], nr[m])};
+    for (int a = 0; a < 11; ++a) {
+      const bool second = a == 3;
+      p[a] = nullptr;
+      if (second && !e->stored_q) continue;
+      rc = ens_alloc(e, &p[a], sz[a] * sizeof(double), second ? &e->second : &e->allocs);
+      if (rc && e->stored_q) {  // in pieces the memory is not to be had: without the second accumulators
+        (void)hipGetLastError();
+        free_second(e);
+        e->stored_q = false;
+        rc = second ? SOLAR_OK : ens_alloc(e, &p[a], sz[a] * sizeof(double), &e->allocs);
+        if (second) continue;
+      }
+      if (rc) return bail(rc);
       if (hipMemset(p[a], 0, sz[a] * sizeof(double)) != hipSuccess)
         return bail(solar::set_error(SOLAR_ERR_HIP, "solar_ens_create: hipMemset failed"));
     }
     M.q[0] = static_cast<double*>(p[0]);
     M.q[1] = static_cast<double*>(p[1]);
     M.qw[0] = static_cast<double*>(p[2]);
-    M.qw[1] = nullptr;  // add_accumulators
-    M.gxp = static_cast<double*>(p[3]);
-    M.gyp = static_cast<double*>(p[4]);
-    M.gxv = static_cast<double*>(p[5]);
-    M.gyv = static_cast<double*>(p[6]);
-    M.fgx = static_cast<double*>(p[7]);
-    M.fgy = static_cast<double*>(p[8]);
-    M.ecols = static_cast<double*>(p[9]);
+    M.qw[1] = nullptr;  // set when all members have theirs
+    M.gxp = static_cast<double*>(p[4]);
+    M.gyp = static_cast<double*>(p[5]);
+    M.gxv = static_cast<double*>(p[6]);
+    M.gyv = static_cast<double*>(p[7]);
+    M.fgx = static_cast<double*>(p[8]);
+    M.fgy = static_cast<double*>(p[9]);
+    M.ecols = static_cast<double*>(p[10]);
     M.dt = dt[m];
     e->choice[m] = default_choice(n[m], nr[m]);
   }
+  for (size_t m = 0; m < e->second.size(); ++m) e->mem[m].qw[1] = static_cast<double*>(e->second[m]);
   void* d = nullptr;
   int rc;
   if ((rc = ens_alloc(e, &d, nmembers * sizeof(EnsMember), &e->allocs))) return bail(rc);
   e->dmem = static_cast<EnsMember*>(d);
+  if (hipMemcpy(e->dmem, e->mem.data(), nmembers * sizeof(EnsMember), hipMemcpyHostToDevice) != hipSuccess)
+    return bail(solar::set_error(SOLAR_ERR_HIP, "solar_ens_create: member table upload failed"));
   std::map<int, std::vector<int>> by_n;
   for (int m = 0; m < nmembers; ++m) by_n[n[m]].push_back(m);
   for (auto& kv : by_n) {
@@ -377,9 +391,6 @@ int solar_ens_create(solar_ens** out, int nmembers, const int* n, const int* nr,
     e->gg.push_back(G);
   }
   if ((rc = build_lists(e))) return bail(rc);
-  add_accumulators(e);
-  if (hipMemcpy(e->dmem, e->mem.data(), nmembers * sizeof(EnsMember), hipMemcpyHostToDevice) != hipSuccess)
-    return bail(solar::set_error(SOLAR_ERR_HIP, "solar_ens_create: member table upload failed"));
   if ((rc = clear_state(e))) return bail(rc);
   *out = e;
   solar::clear_error();

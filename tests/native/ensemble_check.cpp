@@ -10,6 +10,7 @@
 #include <string>
 #include <vector>
 
+static size_t reported = 0;  // free memory the runtime names, if not what there is
 static std::string steps;  // per stage launch: stage, q buffer, qw buffer, stored-q or all
 
 extern "C" {
@@ -21,7 +22,7 @@ hipError_t hipMemset(void* d, int v, size_t n) { std::memset(d, v, n); return hi
 hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { std::memset(d, v, n); return hipSuccess; }
 hipError_t hipMemGetInfo(size_t* f, size_t* t) {
   *t = stub::device_limit;
-  *f = stub::device_limit - stub::device_used;
+  *f = reported ? reported : stub::device_limit - stub::device_used;
   return hipSuccess;
 }
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
@@ -53,7 +54,8 @@ hipError_t launch_gather_ens(const EnsMember*, const int*, int, int, int, bool, 
 }
 }  // namespace solar
 
-// Arguments: the device memory in states of the ensemble, as a decimal number.
+// Arguments: the device memory in states of the ensemble, as a decimal number,
+// and (optional) how much of it the runtime says is free.
 // Prints the stages of a step, then ", " and the states' worth it allocated.
 int main(int argc, char** argv) {
   const int nm = 2, n[nm] = {48, 64}, nr[nm] = {40, 30}, sponge[nm] = {3, 3};
@@ -68,7 +70,8 @@ int main(int argc, char** argv) {
       g0.push_back(0.0);
     }
   }
-  if (argc != 2) return 2;
+  if (argc < 2) return 2;
+  if (argc > 2) reported = static_cast<size_t>(std::atof(argv[2]) * static_cast<double>(state));
   stub::device_limit = static_cast<size_t>(std::atof(argv[1]) * static_cast<double>(state));
   const double a_sponge[nm] = {0.1, 0.1}, dt[nm] = {1e-3, 1e-3};
   solar_ens* e = nullptr;

@@ -26,11 +26,11 @@ def program(tmp_path_factory):
     return out
 
 
-def _run(program, states, **env):
+def _run(program, *states, **env):
     env = dict({k: v for k, v in os.environ.items() if k != "SOLAR_STEP_STORE_ALL"}, **env)
-    r = subprocess.run([program, str(states)], capture_output=True, text=True, timeout=60, env=env)
+    r = subprocess.run([program, *map(str, states)], capture_output=True, text=True, timeout=60, env=env)
     assert r.returncode == 0, r.stdout + r.stderr
-    order, held = r.stdout.strip().split(",")
+    order, held = r.stdout.strip().splitlines()[-1].split(",")
     return order.split(), int(held)
 
 
@@ -45,6 +45,14 @@ def test_schedule_by_the_memory_there_is(program, states, order, held):
 
 def test_the_switch_declines_the_second_accumulator(program):
     got, have = _run(program, 40, SOLAR_STEP_STORE_ALL="1")
+    assert list(dict.fromkeys(got)) == STORE_ALL.split() and have == 3
+
+
+# memory that is free, but not in pieces: the second member's accumulator fails (3.5, 3.8), its
+# ghosts do (4.3); the first member's state is a bit less than half of the two
+@pytest.mark.parametrize("states", [3.5, 3.8, 4.3])
+def test_accumulators_that_fail_on_the_way_are_given_back(program, states):
+    got, have = _run(program, states, 40)
     assert list(dict.fromkeys(got)) == STORE_ALL.split() and have == 3
 
 
